@@ -64,6 +64,9 @@
  *   qpam_resid_norm     the decode's residual adds and pre-norms, V11Block.forward
  *                       (v11/model.py:1039-1049) with ComplexNorm
  *                       (v11/complex_ops.py:188-189)
+ *   qpam_planes         the split-real unpacking around the scan and the delta
+ *                       write (x[..., 0], x[..., 1] and torch.stack of
+ *                       v11/flash_pam.py:56-152, v11/model.py:378-417, 491-576)
  *   qpam_cgu_mix        the CGU's activation and gate between its projections,
  *                       ComplexGatedUnit.forward (v11/complex_ops.py:216-220;
  *                       activations :102-143)
@@ -668,6 +671,32 @@ typedef struct {
 } qpam_cgu_mix_args;
 
 int qpam_cgu_mix(const qpam_cgu_mix_args *a, void *stream);
+
+/* ------------------------------------------------ split-real <-> planes --
+ * (ABI 15)  One launch moves up to QPAM_PLANES_MAX tensors between the
+ * split-real layout [n0][n1][n2_il][d][2] (il: element strides l0, l1, l2,
+ * the last two axes contiguous) and a pair of planes [n0][n1][n2][dp] (strides
+ * p0, p1, p2), converting between fp32 and bf16 (rounded to nearest even).
+ * merge 0: il -> planes, columns d..dp-1 and rows n2_il..n2-1 of the planes
+ * zero (dp a multiple of 4, plane rows 16-byte aligned, 8 in bf16); merge 1:
+ * planes -> il, the padding dropped.  Any alignment of il. */
+#define QPAM_PLANES_MAX 4
+typedef struct {
+    void *il;
+    int64_t l0, l1, l2;
+    void *re, *im;
+    int64_t p0, p1, p2;
+    int32_t n0, n1, n2, n2_il, d, dp;
+    int32_t il_dtype, pl_dtype;
+} qpam_planes_item;
+
+typedef struct {
+    int32_t count;
+    int32_t merge;
+    qpam_planes_item item[QPAM_PLANES_MAX];
+} qpam_planes_args;
+
+int qpam_planes(const qpam_planes_args *a, void *stream);
 
 /* -------------------------------------------------------------------- CE --
  * Tied complex LM-head cross-entropy over hidden rows H [N, D] and weights

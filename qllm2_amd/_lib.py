@@ -12,7 +12,7 @@ import os
 import torch  # noqa: F401  (must be loaded before the HIP library)
 
 LIB_NAME = "libqpam.so"
-ABI_VERSION = 14
+ABI_VERSION = 15
 _HERE = os.path.dirname(os.path.abspath(__file__))
 
 QPAM_F32 = 0
@@ -226,6 +226,22 @@ class CguMixArgs(ctypes.Structure):
         ("ldo", c_i64),
     ]
 
+
+QPAM_PLANES_MAX = 4
+
+
+class PlanesItem(ctypes.Structure):
+    _fields_ = [
+        ("il", c_ptr), ("l0", c_i64), ("l1", c_i64), ("l2", c_i64), ("re", c_ptr), ("im", c_ptr),
+        ("p0", c_i64), ("p1", c_i64), ("p2", c_i64), ("n0", c_i32), ("n1", c_i32), ("n2", c_i32), ("n2_il", c_i32),
+        ("d", c_i32), ("dp", c_i32), ("il_dtype", c_i32), ("pl_dtype", c_i32),
+    ]
+
+
+class PlanesArgs(ctypes.Structure):
+    _fields_ = [("count", c_i32), ("merge", c_i32), ("item", PlanesItem * QPAM_PLANES_MAX)]
+
+
 SIGNATURES = {
     "qpam_version": (ctypes.c_int, []),
     "qpam_last_error": (ctypes.c_char_p, []),
@@ -265,6 +281,7 @@ SIGNATURES = {
     "qpam_cweight_pack": (ctypes.c_int, [ctypes.POINTER(CWeightArgs), c_ptr]),
     "qpam_cweight_unpack": (ctypes.c_int, [ctypes.POINTER(CWeightArgs), c_ptr]),
     "qpam_cabs_bwd_acc": (ctypes.c_int, [c_i32, c_i64, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr]),
+    "qpam_planes": (ctypes.c_int, [ctypes.POINTER(PlanesArgs), c_ptr]),
     "qpam_slice_sum": (ctypes.c_int, [c_i32, c_i32, c_i32, c_i64, c_i64, c_ptr, c_ptr, c_ptr]),
 }
 

@@ -22,7 +22,7 @@ from typing import List, Optional
 import torch
 from torch import Tensor
 
-from . import _lib
+from . import _lib, planes
 from .pam_scan import _cview, _mview
 
 CHUNK_EPS = 1e-6
@@ -75,6 +75,12 @@ def delta_fwd_op(q_re: Tensor, q_im: Tensor, k_re: Tensor, k_im: Tensor, v_re: T
                  gamma: Tensor, beta: Tensor, s0_re: Optional[Tensor], s0_im: Optional[Tensor], q_scale: float,
                  gamma_eps: float, chunk: int, exact_write: bool, keep_workspace: bool) -> List[Tensor]:
     """Returns [y_re, y_im ([B,H,T,d] fp32), s_re, s_im ([B,H,d,d]), workspace]."""
+    return _delta_fwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, beta, s0_re, s0_im, q_scale, gamma_eps, chunk,
+                      exact_write, keep_workspace)
+
+
+def _delta_fwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, beta, s0_re, s0_im, q_scale, gamma_eps, chunk, exact_write,
+               keep_workspace):
     a, keep = _fill(q_re, q_im, k_re, k_im, v_re, v_im, gamma, beta, s0_re, s0_im, q_scale, gamma_eps, chunk,
                     exact_write)
     B, H, T, d = q_re.shape
@@ -136,6 +142,12 @@ def delta_bwd_op(q_re: Tensor, q_im: Tensor, k_re: Tensor, k_im: Tensor, v_re: T
                  ds_re: Optional[Tensor], ds_im: Optional[Tensor]) -> List[Tensor]:
     """Returns [dq_re, dq_im, dk_re, dk_im, dv_re, dv_im, dgamma, dbeta, ds0_re, ds0_im]
     (ds0 empty without s0)."""
+    return _delta_bwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, beta, s0_re, s0_im, q_scale, gamma_eps, chunk,
+                      exact_write, ws, dy_re, dy_im, ds_re, ds_im)
+
+
+def _delta_bwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, beta, s0_re, s0_im, q_scale, gamma_eps, chunk, exact_write,
+               ws, dy_re, dy_im, ds_re, ds_im):
     # the kernels write dgamma and dbeta with gamma's strides: contiguous planes,
     # matching the gradients allocated below
     gamma, beta = gamma.contiguous(), beta.contiguous()
@@ -247,15 +259,92 @@ def delta_planar(q_re, q_im, k_re, k_im, v_re, v_im, gamma, beta, *, q_scale, ga
     return out[0], out[1], out[2], out[3]
 
 
+# ---------------------------------------------------------------- split-real front end
+
+@torch.library.custom_op("qpam::delta_il_fwd", mutates_args=())
+def delta_il_fwd_op(q: Tensor, k: Tensor, v: Tensor, gamma: Tensor, beta: Tensor, q_scale: float, chunk: int,
+                    keep_workspace: bool) -> List[Tensor]:
+    """The delta write on split-real q, k, v [B,H,T,d,2] (d <= 64, fp32 or bf16),
+    unpacked into padded fp32 planes by one launch, y and the state packed by
+    another.  Returns [y, s in q's dtype, planes [3,2,B,H,T,64], workspace]."""
+    pl = planes.split_rows((q, k, v), torch.float32)
+    y_re, y_im, s_re, s_im, ws = _delta_fwd(pl[0, 0], pl[0, 1], pl[1, 0], pl[1, 1], pl[2, 0], pl[2, 1], gamma, beta,
+                                            None, None, q_scale, CHUNK_EPS, chunk, False, keep_workspace)
+    y, s = planes.merge([(y_re, y_im)], [(s_re, s_im)], q.shape[3], q.dtype)
+    return [y, s, pl, ws]
+
+
+@delta_il_fwd_op.register_fake
+def _(q, k, v, gamma, beta, q_scale, chunk, keep_workspace):
+    B, H, T, d = q.shape[:4]
+    f32 = torch.float32
+    return [q.new_empty(B, H, T, d, 2), q.new_empty(B, H, d, d, 2), q.new_empty(3, 2, B, H, T, planes.KD, dtype=f32),
+            q.new_empty(_ws_bytes(B, H, T, chunk=chunk) // 4 if keep_workspace else 0, dtype=f32)]
+
+
+@torch.library.custom_op("qpam::delta_il_bwd", mutates_args=())
+def delta_il_bwd_op(pl: Tensor, gamma: Tensor, beta: Tensor, q_scale: float, chunk: int, ws: Tensor,
+                    dy: Optional[Tensor], ds: Optional[Tensor], d: int, bf16: bool) -> List[Tensor]:
+    """[dq, dk, dv [B,H,T,d,2] (bf16 or fp32), dgamma, dbeta]."""
+    if dy is not None:
+        dyp = planes.split_rows((dy,), torch.float32)[0]
+    else:
+        dyp = torch.zeros(pl.shape[1:], device=pl.device, dtype=torch.float32)
+    dsp = planes.split_states(ds) if ds is not None else (None, None)
+    g = _delta_bwd(pl[0, 0], pl[0, 1], pl[1, 0], pl[1, 1], pl[2, 0], pl[2, 1], gamma, beta, None, None, q_scale,
+                   CHUNK_EPS, chunk, False, ws, dyp[0], dyp[1], dsp[0], dsp[1])
+    return planes.merge([(g[0], g[1]), (g[2], g[3]), (g[4], g[5])], [], d,
+                        torch.bfloat16 if bf16 else torch.float32) + [g[6], g[7]]
+
+
+@delta_il_bwd_op.register_fake
+def _(pl, gamma, beta, q_scale, chunk, ws, dy, ds, d, bf16):
+    _, _, B, H, T, _ = pl.shape
+    dt = torch.bfloat16 if bf16 else torch.float32
+    return [pl.new_empty(B, H, T, d, 2, dtype=dt) for _ in range(3)] + [gamma.new_empty(B, H, T) for _ in range(2)]
+
+
+def _il_setup(ctx, inputs, output):
+    q, k, v, gamma, beta, q_scale, chunk, keep_ws = inputs
+    ctx.save_for_backward(output[2], gamma, beta, output[3])
+    ctx.q_scale, ctx.chunk, ctx.keep, ctx.d, ctx.bf16 = q_scale, chunk, keep_ws, q.shape[3], q.dtype == torch.bfloat16
+    ctx.set_materialize_grads(False)
+
+
+def _il_backward(ctx, grads):
+    pl, gamma, beta, ws = ctx.saved_tensors
+    if not ctx.keep:
+        raise RuntimeError("qpam delta: the forward ran without its backward workspace (keep_workspace=False)")
+    g = delta_il_bwd_op(pl, gamma, beta, ctx.q_scale, ctx.chunk, ws, grads[0], grads[1], ctx.d, ctx.bf16)
+    return g[0], g[1], g[2], g[3], g[4], None, None, None
+
+
+delta_il_fwd_op.register_autograd(_il_backward, setup_context=_il_setup)
+
+
+def _il_covers(q, k, v, gamma, beta, state):
+    """Calls the split-real op takes: equal [B,H,T,d,2] shapes (d <= 64) in one
+    dtype of the kernels, no start state; others go through delta_planar."""
+    return (q.dim() == 5 and q.shape[-1] == 2 and 1 <= q.shape[-2] <= planes.KD and k.shape == q.shape
+            and v.shape == q.shape and planes.covers(q, k, v) and gamma.is_cuda and beta.is_cuda
+            and gamma.shape == q.shape[:3] and beta.shape == gamma.shape and q.numel() > 0 and state is None
+            and planes.fits(q, 1))
+
+
 def forward_delta(queries, keys, protected_values, decay_gamma, write_beta, head_dim, state=None, chunk=64):
     """V11PAMLayer._forward_delta (v11/model.py:491-576) on split-real
     [B,H,T,d,2] tensors (queries unscaled), decay_gamma / write_beta [B,H,T],
     chunks of `chunk` steps (the layer's delta_chunk, v11/model.py:494).
     Returns (output [B,H,T,d,2], memory_state [B,H,d,d,2]) in the input dtype."""
     dtype = queries.dtype
-    planes = [x[..., i] for x in (queries, keys, protected_values) for i in (0, 1)]
+    if _il_covers(queries, keys, protected_values, decay_gamma, write_beta, state):
+        gamma, beta = decay_gamma.float(), write_beta.float()
+        keep = torch.is_grad_enabled() and any(t.requires_grad for t in (queries, keys, protected_values, gamma, beta))
+        out = delta_il_fwd_op(queries, keys, protected_values, gamma, beta, head_dim ** -0.5, int(chunk), keep)
+        return out[0], out[1]
+    planes_ = [x[..., i] for x in (queries, keys, protected_values) for i in (0, 1)]
     s0 = (state[..., 0], state[..., 1]) if state is not None else None
-    y_re, y_im, s_re, s_im = delta_planar(*planes, decay_gamma, write_beta, q_scale=head_dim ** -0.5,
+    y_re, y_im, s_re, s_im = delta_planar(*planes_, decay_gamma, write_beta, q_scale=head_dim ** -0.5,
                                           gamma_eps=CHUNK_EPS, s0=s0, chunk=chunk)
     return torch.stack([y_re, y_im], -1).to(dtype), torch.stack([s_re, s_im], -1).to(dtype)
 
@@ -267,8 +356,8 @@ def recur_step_delta(memory_state, decay_gamma, value_t, key_t, query_t, write_b
     the input state is not modified.  The step's write has weight 1 (the
     exact recurrence) and gamma is used as given (no 1e-6 shift)."""
     dtype = memory_state.dtype
-    planes = [x[..., i].unsqueeze(2) for x in (query_t, key_t, value_t) for i in (0, 1)]
-    y_re, y_im, s_re, s_im = delta_planar(*planes, decay_gamma.unsqueeze(-1), write_beta_t.unsqueeze(-1),
+    step = [x[..., i].unsqueeze(2) for x in (query_t, key_t, value_t) for i in (0, 1)]
+    y_re, y_im, s_re, s_im = delta_planar(*step, decay_gamma.unsqueeze(-1), write_beta_t.unsqueeze(-1),
                                           q_scale=1.0, gamma_eps=0.0, exact_write=True,
                                           s0=(memory_state[..., 0], memory_state[..., 1]))
     return torch.stack([y_re[:, :, 0], y_im[:, :, 0]], -1).to(dtype), torch.stack([s_re, s_im], -1).to(dtype)

@@ -21,7 +21,7 @@ from typing import List, Optional, Tuple
 import torch
 from torch import Tensor
 
-from . import _lib
+from . import _lib, planes
 
 KERNEL_CHUNKS = (16, 32, 64)
 SEG = 4  # 64-step chunks per segment of the bf16 kernels (workspace layout)
@@ -140,6 +140,10 @@ def scan_fwd_op(q_re: Tensor, q_im: Tensor, k_re: Tensor, k_im: Tensor, v_re: Te
     y_re slot (re and im planes of a token side by side, the [N, 2 H d] input
     of one output-projection GEMM) and an empty y_im; 3: layout 2 in bf16 (bf16
     inputs, chunk 64: the kernel rounds y once from its fp32 result)."""
+    return _scan_fwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, s0_im, q_scale, chunk, y_layout)
+
+
+def _scan_fwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, s0_im, q_scale, chunk, y_layout):
     _validate(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, s0_im, chunk)
     M, B, H, T = gamma.shape
     d = q_re.shape[-1]
@@ -211,6 +215,12 @@ def scan_bwd_op(q_re: Tensor, q_im: Tensor, k_re: Tensor, k_im: Tensor, v_re: Te
                 ds_re: Optional[Tensor], ds_im: Optional[Tensor], y_layout: int) -> List[Tensor]:
     """Returns [dq_re, dq_im, dk_re, dk_im, dv_re, dv_im, dgamma, drot_re, drot_im, ds0_re, ds0_im]
     (drot/ds0 are empty tensors when rot/s0 were not given); dy in y's layout."""
+    return _scan_bwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, s0_im, q_scale, chunk, ws,
+                     dy_re, dy_im, ds_re, ds_im, y_layout)
+
+
+def _scan_bwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, s0_im, q_scale, chunk, ws, dy_re,
+              dy_im, ds_re, ds_im, y_layout):
     M, B, H, T = gamma.shape
     d = q_re.shape[-1]
     dev = q_re.device
@@ -451,6 +461,82 @@ def _scan_blocks(q_re, q_im, k_re, k_im, v_re, v_im, gamma, q_scale, chunk, rot,
     return y_re, y_im, s_re, s_im
 
 
+# ---------------------------------------------------------------- split-real front end
+
+@torch.library.custom_op("qpam::scan_il_fwd", mutates_args=())
+def scan_il_fwd_op(q: Tensor, k: Tensor, v: Tensor, gamma: Tensor, rot_re: Optional[Tensor],
+                   rot_im: Optional[Tensor], q_scale: float, chunk: int) -> List[Tensor]:
+    """The scan on split-real q, k, v [B,H,T,d,2] (d <= 64, fp32 or bf16): one
+    launch unpacks them into padded planes, one packs y and the state.  Returns
+    [y [B,H,T,d,2], s [M,B,H,d,d,2] in q's dtype, planes [3,2,B,H,T,64],
+    workspace]; the planes are what the backward reads."""
+    d = q.shape[3]
+    pl = planes.split_rows((q, k, v), q.dtype)
+    y_re, y_im, s_re, s_im, ws = _scan_fwd(pl[0, 0], pl[0, 1], pl[1, 0], pl[1, 1], pl[2, 0], pl[2, 1], gamma, rot_re,
+                                           rot_im, None, None, q_scale, chunk, 0)
+    y, s = planes.merge([(y_re, y_im)], [(s_re, s_im)], d, q.dtype)
+    return [y, s, pl, ws]
+
+
+@scan_il_fwd_op.register_fake
+def _(q, k, v, gamma, rot_re, rot_im, q_scale, chunk):
+    M, B, H, T = gamma.shape
+    d = q.shape[3]
+    nbytes = fwd_workspace_bytes(M, B, H, T, chunk, q.dtype == torch.bfloat16)
+    return [q.new_empty(B, H, T, d, 2), q.new_empty(M, B, H, d, d, 2), q.new_empty(3, 2, B, H, T, planes.KD),
+            q.new_empty((nbytes + 3) // 4, dtype=torch.float32)]
+
+
+@torch.library.custom_op("qpam::scan_il_bwd", mutates_args=())
+def scan_il_bwd_op(pl: Tensor, gamma: Tensor, rot_re: Optional[Tensor], rot_im: Optional[Tensor], q_scale: float,
+                   chunk: int, ws: Tensor, dy: Optional[Tensor], ds: Optional[Tensor], d: int) -> List[Tensor]:
+    """[dq, dk, dv [B,H,T,d,2] in the planes' dtype, dgamma, drot_re, drot_im]."""
+    if dy is not None:
+        dyp = planes.split_rows((dy,), torch.float32)[0]
+    else:
+        dyp = torch.zeros(pl.shape[1:], device=pl.device, dtype=torch.float32)
+    dsp = planes.split_states(ds) if ds is not None else (None, None)
+    g = _scan_bwd(pl[0, 0], pl[0, 1], pl[1, 0], pl[1, 1], pl[2, 0], pl[2, 1], gamma, rot_re, rot_im, None, None,
+                  q_scale, chunk, ws, dyp[0], dyp[1], dsp[0], dsp[1], 0)
+    return planes.merge([(g[0], g[1]), (g[2], g[3]), (g[4], g[5])], [], d, pl.dtype) + [g[6], g[7], g[8]]
+
+
+@scan_il_bwd_op.register_fake
+def _(pl, gamma, rot_re, rot_im, q_scale, chunk, ws, dy, ds, d):
+    _, _, B, H, T, _ = pl.shape
+    dr = [torch.empty_like(gamma) if rot_re is not None else gamma.new_empty(0) for _ in range(2)]
+    return [pl.new_empty(B, H, T, d, 2) for _ in range(3)] + [torch.empty_like(gamma)] + dr
+
+
+def _il_setup(ctx, inputs, output):
+    q, k, v, gamma, rot_re, rot_im, q_scale, chunk = inputs
+    ctx.save_for_backward(output[2], gamma, rot_re, rot_im, output[3])
+    ctx.q_scale, ctx.chunk, ctx.d = q_scale, chunk, q.shape[3]
+    ctx.set_materialize_grads(False)
+
+
+def _il_backward(ctx, grads):
+    pl, gamma, rot_re, rot_im, ws = ctx.saved_tensors
+    g = scan_il_bwd_op(pl, gamma, rot_re, rot_im, ctx.q_scale, ctx.chunk, ws, grads[0], grads[1], ctx.d)
+    drot = (g[4], g[5]) if rot_re is not None else (None, None)
+    return g[0], g[1], g[2], g[3], drot[0], drot[1], None, None
+
+
+scan_il_fwd_op.register_autograd(_il_backward, setup_context=_il_setup)
+
+
+def _il_covers(q, k, v, gamma, rot, s0):
+    """Calls the split-real op takes: equal [B,H,T,d,2] shapes (d <= 64) in one
+    dtype of the kernels, up to MAX_STATES states, no start state.  Others go
+    through separate planes (pam_scan_planar), which splits head dims and states
+    over several launches and raises for what no kernel takes."""
+    return (q.dim() == 5 and q.shape[-1] == 2 and 1 <= q.shape[-2] <= planes.KD and k.shape == q.shape
+            and v.shape == q.shape and planes.covers(q, k, v) and gamma.is_cuda and gamma.dim() == 4
+            and gamma.shape[1:] == q.shape[:3] and 1 <= gamma.shape[0] <= MAX_STATES and q.numel() > 0 and s0 is None
+            and planes.fits(q, gamma.shape[0])
+            and (rot is None or (rot[0].shape == gamma.shape and rot[1].shape == gamma.shape)))
+
+
 def _planes(z):
     return z[..., 0], z[..., 1]
 
@@ -461,6 +547,11 @@ def pam_scan_interleaved(queries, keys, values, gamma_all, head_dim, chunk_size,
     gamma_all [M,B,H,T]; rot optional (re, im) planes [M,B,H,T]; s0 optional
     [M,B,H,d,d,2].  Returns (Y [B,H,T,d,2], S [M,B,H,d,d,2]) in the input dtype."""
     dtype = queries.dtype
+    if _il_covers(queries, keys, values, gamma_all, rot, s0):
+        rot_re, rot_im = (rot[0].float(), rot[1].float()) if rot is not None else (None, None)
+        out = scan_il_fwd_op(queries, keys, values, gamma_all.float(), rot_re, rot_im,
+                             head_dim ** -0.5 if scale_queries else 1.0, chunk_for(chunk_size, queries.shape[2]))
+        return out[0], out[1]
     work = torch.bfloat16 if dtype == torch.bfloat16 else torch.float32
     qr, qi = (x.to(work) for x in _planes(queries))
     kr, ki = (x.to(work) for x in _planes(keys))
