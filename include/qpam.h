@@ -67,6 +67,8 @@
  *   qpam_planes         the split-real unpacking around the scan and the delta
  *                       write (x[..., 0], x[..., 1] and torch.stack of
  *                       v11/flash_pam.py:56-152, v11/model.py:378-417, 491-576)
+ *   qpam_pc_fwd/_bwd    v11/model.py:421-489 V11PAMLayer._forward_chunked_perchannel
+ *                       and its autograd backward
  *   qpam_cgu_mix        the CGU's activation and gate between its projections,
  *                       ComplexGatedUnit.forward (v11/complex_ops.py:216-220;
  *                       activations :102-143)
@@ -576,6 +578,39 @@ typedef struct {
 } qpam_pc_scan_args;
 
 int qpam_pc_scan(const qpam_pc_scan_args *a, void *stream);
+
+/* (ABI 15) The whole per-channel chunked form for head dims up to 64, forward
+ * and backward, V11PAMLayer._forward_chunked_perchannel (v11/model.py:421-489)
+ * from a zero state: q, k [B,H,T,d,2] in dtype, v in v_dtype (element strides
+ * sb, sh, st, all even; complex elements aligned), gamma [B,H,T,d] in g_dtype
+ * (channels contiguous); n = ceil(T / chunk) chunks, N = B H chains.
+ * qpam_pc_fwd writes y [B,H,T,d,2] (dtype, contiguous), s_fin [N][d][d][2],
+ * atot [N][n][d] (each chunk's column decays) and x [N][n][d][d][2] (the state
+ * entering each chunk), fp32.  qpam_pc_bwd takes that x as s_in and atot, dy
+ * (y's layout) and dfin (s_fin's, optional), uses x as its workspace (the state
+ * gradients, same size) and writes dq, dk (dtype), dv (v_dtype) [B,H,T,d,2] and
+ * dgamma (g_dtype) [B,H,T,d], contiguous. */
+typedef struct {
+    int32_t dtype, v_dtype, g_dtype, chunk;
+    int64_t B, H, T, d;
+    float q_scale;
+    int32_t reserved0;
+    const void *q; int64_t q_sb, q_sh, q_st;
+    const void *k; int64_t k_sb, k_sh, k_st;
+    const void *v; int64_t v_sb, v_sh, v_st;
+    const void *gamma; int64_t g_sb, g_sh, g_st;
+    void *y;
+    float *x;
+    float *atot;
+    float *s_fin;
+    const float *s_in;
+    const void *dy;
+    const float *dfin;
+    void *dq, *dk, *dv, *dgamma;
+} qpam_pc_args;
+
+int qpam_pc_fwd(const qpam_pc_args *a, void *stream);
+int qpam_pc_bwd(const qpam_pc_args *a, void *stream);
 
 /* ------------------------------------------------ complex elementwise -----
  * Split-real complex tensors [rows, dim, 2] (interleaved re/im, contiguous),

@@ -199,6 +199,19 @@ class PcScanArgs(ctypes.Structure):
     ]
 
 
+class PcArgs(ctypes.Structure):
+    _fields_ = [
+        ("dtype", c_i32), ("v_dtype", c_i32), ("g_dtype", c_i32), ("chunk", c_i32),
+        ("B", c_i64), ("H", c_i64), ("T", c_i64), ("d", c_i64), ("q_scale", c_f32), ("reserved0", c_i32),
+        ("q", c_ptr), ("q_sb", c_i64), ("q_sh", c_i64), ("q_st", c_i64),
+        ("k", c_ptr), ("k_sb", c_i64), ("k_sh", c_i64), ("k_st", c_i64),
+        ("v", c_ptr), ("v_sb", c_i64), ("v_sh", c_i64), ("v_st", c_i64),
+        ("gamma", c_ptr), ("g_sb", c_i64), ("g_sh", c_i64), ("g_st", c_i64),
+        ("y", c_ptr), ("x", c_ptr), ("atot", c_ptr), ("s_fin", c_ptr), ("s_in", c_ptr), ("dy", c_ptr), ("dfin", c_ptr),
+        ("dq", c_ptr), ("dk", c_ptr), ("dv", c_ptr), ("dgamma", c_ptr),
+    ]
+
+
 class CWeightArgs(ctypes.Structure):
     _fields_ = [
         ("dtype", c_i32), ("layout", c_i32), ("R", c_i64), ("C", c_i64), ("wr", c_ptr), ("wi", c_ptr),
@@ -278,6 +291,8 @@ SIGNATURES = {
     "qpam_pc_fold_fwd": (ctypes.c_int, [ctypes.POINTER(PcFoldArgs), c_ptr]),
     "qpam_pc_fold_bwd": (ctypes.c_int, [ctypes.POINTER(PcFoldArgs), c_ptr]),
     "qpam_pc_scan": (ctypes.c_int, [ctypes.POINTER(PcScanArgs), c_ptr]),
+    "qpam_pc_fwd": (ctypes.c_int, [ctypes.POINTER(PcArgs), c_ptr]),
+    "qpam_pc_bwd": (ctypes.c_int, [ctypes.POINTER(PcArgs), c_ptr]),
     "qpam_cweight_pack": (ctypes.c_int, [ctypes.POINTER(CWeightArgs), c_ptr]),
     "qpam_cweight_unpack": (ctypes.c_int, [ctypes.POINTER(CWeightArgs), c_ptr]),
     "qpam_cabs_bwd_acc": (ctypes.c_int, [c_i32, c_i64, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr]),

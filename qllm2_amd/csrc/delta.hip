@@ -21,7 +21,7 @@
 // for dq, dk, dgamma, dbeta.  The forward leaves what they need in its
 // workspace: the state entering every chunk, U, and the chunk's products in the
 // orders the backward reads them.
-#include "common.h"
+#include "gauss.h"
 
 namespace qpam {
 namespace {
@@ -103,10 +103,6 @@ constexpr int BW_G = 0, BW_W = 2 * D * D, BW_PQ = 4 * D * D, BW_PK = BW_PQ + NBL
 
 __device__ __forceinline__ int blk(int b, int c) { return b * (b + 1) / 2 + c; }  // c <= b
 
-__device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
 // Complex 16 x 16 blocks in the prep kernel's LDS: rows of LP floats (one pad
 // float: the MFMA A-operand reads step the 16 lanes of a group over rows, which a
 // pitch of 16 would put on one bank in four), re plane then im plane (LPL apart).
@@ -133,23 +129,6 @@ __device__ __forceinline__ void blk_export(float *dst, const float *src, int tid
         dst[e] = src[pl * LPL + row * LP + 4 * ks + gg];
     }
 }
-
-// Gauss accumulation of a complex product over k: t1 += ar br, t2 += ai bi,
-// t3 += (ar + ai)(br + bi); then re = t1 - t2, im = t3 - t1 - t2.  Three real
-// MFMAs per complex product instead of four.
-struct Gauss {
-    floatx4 t1, t2, t3;
-};
-__device__ __forceinline__ void gz(Gauss &x) {
-    x.t1 = x.t2 = x.t3 = floatx4{0.f, 0.f, 0.f, 0.f};
-}
-__device__ __forceinline__ void gstep(Gauss &x, float ar, float ai, float br, float bi) {
-    x.t1 = mfma4(ar, br, x.t1);
-    x.t2 = mfma4(ai, bi, x.t2);
-    x.t3 = mfma4(ar + ai, br + bi, x.t3);
-}
-__device__ __forceinline__ floatx4 gre(const Gauss &x) { return x.t1 - x.t2; }
-__device__ __forceinline__ floatx4 gim(const Gauss &x) { return x.t3 - x.t1 - x.t2; }
 
 // C = A B for complex 16 x 16 LDS blocks (Gauss)
 __device__ __forceinline__ void blk_mul_g(Gauss &x, const float *A, const float *B, int l16, int g) {

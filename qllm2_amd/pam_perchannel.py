@@ -4,22 +4,24 @@
 Per chunk of `chunk` steps the reference folds the decay into the operands
 (L = max(cumsum(log max(gamma, 1e-6)), -30) per key channel): queries carry
 e^{L} q_scale, keys e^{-L}, the state-write keys e^{L_last - L}, and the state
-decays column j by e^{L_last[j]}.  Here:
+decays column j by e^{L_last[j]}.  Head dims up to 64 run whole on the HIP
+library (qpam_pc_fwd / qpam_pc_bwd): the operands are folded on their way into
+LDS, the chunk products run on fp32 MFMA, and only the chunk states pass through
+HBM.  Larger head dims (two or more 64-wide tiles per operand) run as
 
-  * the fold runs in one HIP kernel over all chunks at once (qpam_pc_fold_fwd;
+  * the fold in one HIP kernel over all chunks at once (qpam_pc_fold_fwd;
     its backward, qpam_pc_fold_bwd, forms dq, dk and dgamma through both
     clamps);
   * the chunk-parallel products -- the masked score Q K^H, its read of V, the
-    chunk's state increment V^T conj(W) and the carried read Q S^T -- are
+    chunk's state increment V^T conj(W) and the carried read Q S^T -- as
     batched complex GEMMs over every (b, h, chunk) at once (the library GEMM,
     fp32 complex);
-  * the state entering each chunk comes from the per-column decayed scan over
-    the chunks (qpam_pc_scan; backward: the same kernel in reverse).
+  * the state entering each chunk from the per-column decayed scan over the
+    chunks (qpam_pc_scan; backward: the same kernel in reverse).
 
-Autograd runs through the GEMMs and the two custom functions, so the layer's
-training forward has gradients for q, k, v and gamma.  The whole computation
-is fp32 (the reference computes in the input dtype); outputs are cast back to
-the input dtype.
+Both have gradients for q, k, v and gamma.  The whole computation is fp32 (the
+reference computes in the input dtype); outputs are cast back to the input
+dtype.
 """
 
 import ctypes
@@ -148,6 +150,68 @@ class _Scan(torch.autograd.Function):
         return dx, da
 
 
+KERNEL_D = 64  # head dims up to this run on the chunk kernels
+
+
+def _aligned(x):
+    """x [..., d, 2] whose complex elements start on their own alignment."""
+    x = _pairs(x)
+    ok = all(s % 2 == 0 for s in x.stride()[:3]) and x.data_ptr() % (2 * x.element_size()) == 0
+    return x if ok else x.clone(memory_format=torch.contiguous_format)
+
+
+class _Chunked(torch.autograd.Function):
+    """(q, k, v [B,H,T,d,2], gamma [B,H,T,d], d <= 64) -> y [B,H,T,d,2] in q's
+    dtype and the final state [B,H,d,d,2] fp32."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, gamma, chunk, q_scale):
+        q, k, v = _aligned(q), _aligned(k), _aligned(v)
+        gamma = gamma if gamma.stride(-1) == 1 else gamma.contiguous()
+        B, H, T, d = q.shape[:4]
+        n = -(-T // chunk)
+        f32 = dict(device=q.device, dtype=torch.float32)
+        y = torch.empty(B, H, T, d, 2, device=q.device, dtype=q.dtype)
+        x, atot = torch.empty(B * H, n, d, d, 2, **f32), torch.empty(B * H, n, d, **f32)
+        s_fin = torch.empty(B, H, d, d, 2, **f32)
+        a = _Chunked._args(q, k, v, gamma, chunk, q_scale, x, atot)
+        a.y, a.s_fin = y.data_ptr(), s_fin.data_ptr()
+        with torch.cuda.device(q.device):
+            _lib.check(_lib.lib().qpam_pc_fwd(ctypes.byref(a), _lib.stream_ptr(q.device)), "qpam_pc_fwd")
+        ctx.save_for_backward(q, k, v, gamma, x, atot)
+        ctx.chunk, ctx.q_scale = chunk, q_scale
+        ctx.set_materialize_grads(False)
+        return y, s_fin
+
+    @staticmethod
+    def _args(q, k, v, gamma, chunk, q_scale, x, atot):
+        a = _lib.PcArgs()
+        a.dtype, a.v_dtype, a.g_dtype, a.chunk = _dt(q), _dt(v), _dt(gamma), chunk
+        a.B, a.H, a.T, a.d = q.shape[:4]
+        a.q_scale = q_scale
+        a.q, a.k, a.v, a.gamma = q.data_ptr(), k.data_ptr(), v.data_ptr(), gamma.data_ptr()
+        a.q_sb, a.q_sh, a.q_st = q.stride()[:3]
+        a.k_sb, a.k_sh, a.k_st = k.stride()[:3]
+        a.v_sb, a.v_sh, a.v_st = v.stride()[:3]
+        a.g_sb, a.g_sh, a.g_st = gamma.stride()[:3]
+        a.x, a.atot = x.data_ptr(), atot.data_ptr()
+        return a
+
+    @staticmethod
+    def backward(ctx, dy, dfin):
+        q, k, v, gamma, s_in, atot = ctx.saved_tensors
+        dy = dy.contiguous() if dy is not None else torch.zeros(q.shape, device=q.device, dtype=q.dtype)
+        dfin = dfin.contiguous() if dfin is not None else None
+        dq, dk, dv, dgamma = (torch.empty(t.shape, device=t.device, dtype=t.dtype) for t in (q, k, v, gamma))
+        ws = torch.empty_like(s_in)
+        a = _Chunked._args(q, k, v, gamma, ctx.chunk, ctx.q_scale, ws, atot)
+        a.s_in, a.dy, a.dfin = s_in.data_ptr(), dy.data_ptr(), _ptr(dfin)
+        a.dq, a.dk, a.dv, a.dgamma = dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dgamma.data_ptr()
+        with torch.cuda.device(q.device):
+            _lib.check(_lib.lib().qpam_pc_bwd(ctypes.byref(a), _lib.stream_ptr(q.device)), "qpam_pc_bwd")
+        return dq, dk, dv, dgamma, None, None
+
+
 def perchannel_chunked(queries, keys, protected_values, decay_gamma, head_dim, chunk_size):
     """V11PAMLayer._forward_chunked_perchannel (v11/model.py:421-489):
     queries, keys, protected_values [B,H,T,d,2], decay_gamma [B,H,T,d] (CUDA,
@@ -159,6 +223,17 @@ def perchannel_chunked(queries, keys, protected_values, decay_gamma, head_dim, c
     C = int(chunk_size)
     if not 1 <= C <= 64:
         raise ValueError(f"qpam per-channel scan: chunk_size {C} outside 1..64")
+    if d <= KERNEL_D:
+        if queries.dim() != 5 or keys.shape != queries.shape or protected_values.shape != queries.shape \
+                or queries.shape[-1] != 2 or decay_gamma.shape != queries.shape[:4]:
+            raise ValueError(f"qpam per-channel scan: q, k, v [B,H,T,d,2] and gamma [B,H,T,d] expected, got "
+                             f"{tuple(queries.shape)}, {tuple(keys.shape)}, {tuple(protected_values.shape)}, "
+                             f"{tuple(decay_gamma.shape)}")
+        v = protected_values
+        y, s_fin = _Chunked.apply(queries, keys.to(queries.dtype),
+                                  v if v.dtype in (torch.float32, torch.bfloat16) else v.float(), decay_gamma, C,
+                                  head_dim ** -0.5)
+        return y, s_fin.to(queries.dtype)
     n = -(-T // C)
     qf, kf, wf, atot = _Fold.apply(queries, keys, decay_gamma, C, head_dim ** -0.5)
     Q, K, W = (torch.view_as_complex(t) for t in (qf, kf, wf))   # [N, n, C, d]

@@ -1,0 +1,66 @@
+"""The per-channel chunk kernels (head dims up to 64, qpam_pc_fwd / qpam_pc_bwd)
+against the general path (fold kernels and batched library products), which is
+itself checked against the oracle: same calls over head dims and chunk lengths at
+the edges of the 16-wide tiles, ragged last chunks, one step, mixed dtypes,
+strided / misaligned / expanded layouts, prefixes past the -30 clamp and missing
+output gradients.  Both sum the same fp32 products in other orders: a 64-term
+sum of both sits within 64 * 2^-24 = 4e-6 of the exact one relative to the sum of
+magnitudes, and the two chained products and e^{+-L} factors (2^-22 each) add
+about as much: 2e-5 of the tensor's largest value.  bf16 results differ by one
+rounding on each side at most: 2^-8."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _layout(x, how):
+    if how == "bthd":
+        return x.transpose(1, 2).contiguous().transpose(1, 2)
+    if how == "offset":          # complex elements start between their alignments
+        buf = x.new_zeros(x.numel() + 1)
+        buf[1:] = x.reshape(-1)
+        return buf[1:].view(x.shape)
+    return x[:1].expand(x.shape) if how == "expanded" else x.contiguous()
+
+
+@pytest.mark.parametrize("d,C,T,dtypes,how,given,strong", [
+    (64, 64, 130, "fff", "contiguous", "both", False), (64, 64, 64, "fff", "bthd", "y", False),
+    (33, 33, 70, "fff", "offset", "both", False), (32, 64, 129, "bbb", "contiguous", "both", False),
+    (31, 17, 50, "bff", "bthd", "s", False), (16, 16, 33, "fbf", "offset", "both", True),
+    (17, 64, 63, "ffb", "expanded", "both", False), (48, 48, 1, "fff", "contiguous", "both", False),
+    (1, 1, 5, "fff", "contiguous", "both", False), (2, 64, 65, "bfb", "contiguous", "y", True),
+    (64, 32, 100, "bbb", "offset", "both", True), (64, 15, 46, "fff", "bthd", "both", False),
+])
+def test_chunk_kernels_equal_general_path(gpu_lib, monkeypatch, d, C, T, dtypes, how, given, strong):
+    from qllm2_amd import pam_perchannel as P
+    print(f"case d={d} C={C} T={T} {dtypes} {how} {given} strong={strong}", flush=True)
+    B, H = 2, 3
+    dt = [{"f": torch.float32, "b": torch.bfloat16}[x] for x in dtypes]      # q and k, v, gamma
+    g = torch.Generator().manual_seed(T + d)
+    rn = lambda *s: torch.randn(*s, generator=g).cuda()  # noqa: E731
+    q, k, v = (_layout((rn(B, H, T, d, 2) * (2 * d) ** -0.5).to(t), how) for t in (dt[0], dt[0], dt[1]))
+    gamma = torch.sigmoid(rn(B, H, T, d) + (-1.0 if strong else 3.0)).to(dt[2])
+    leaves = [x.detach().requires_grad_(True) for x in (q, k, v, gamma)]
+    dy = rn(B, H, T, d, 2).to(dt[0]) if given != "s" else None
+    ds = rn(B, H, d, d, 2).to(dt[0]) if given != "y" else None
+    res = []
+    for limit in (64, 0):
+        monkeypatch.setattr(P, "KERNEL_D", limit)
+        y, s = P.perchannel_chunked(*leaves, d, C)
+        outs, gs = zip(*[(o, x) for o, x in ((y, dy), (s, ds)) if x is not None])
+        res.append([y, s, *torch.autograd.grad(outs, leaves, gs, allow_unused=True)])
+    for name, a, b in zip(("y", "s", "dq", "dk", "dv", "dgamma"), *res):
+        if b is None:            # the general path has no gradient here (dq from the state alone)
+            assert a is None or not a.any(), name
+            continue
+        assert a.dtype == b.dtype and a.shape == b.shape, name
+        tol = 2e-5 if a.dtype == torch.float32 and "b" not in dtypes else 2.0 ** -8
+        err, top = (a.float() - b.float()).abs().max().item(), b.float().abs().max().item()
+        if name == "dgamma" and res[1][2] is not None:
+            # dgamma sums q dq - k dk, which cancel (to exactly zero over one step): the error is
+            # relative to the terms, over the smallest gamma
+            terms = (q.float() * res[1][2].float()).abs().max() + (k.float() * res[1][3].float()).abs().max()
+            top = max(top, (terms / gamma.float().min()).item())
+        assert err <= tol * max(top, 1e-30), f"{name}: {err:.2e} of {top:.2e}"
