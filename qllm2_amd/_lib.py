@@ -337,9 +337,30 @@ def check(status, what):
         raise QpamError(f"{what} failed (status {status}): {msg}")
 
 
+class _Here:
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_HERE_CTX = _Here()
+
+
+def device(dev):
+    """Context for launches on `dev`: nothing to do when it is the current device
+    already (torch.cuda.device enters and leaves it through four runtime calls)."""
+    if dev.type == "cuda" and dev.index == torch._C._cuda_getDevice():
+        return _HERE_CTX
+    return torch.cuda.device(dev)
+
+
 def stream_ptr(device=None):
     """Raw hipStream_t of torch's current stream on `device`."""
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    if device is None or device.index is None:
+        return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(device.index))
 
 
 def ptr(t):

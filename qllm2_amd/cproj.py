@@ -81,7 +81,7 @@ def _pack(layout, wr, wi, tail=None, rows=None):
     w = torch.empty(rows, 2 * C, device=wr.device, dtype=wr.dtype)
     a = _args(layout, wr, wi, tail, rows - 2 * R - tail_rows, 2 * C)
     a.w = w.data_ptr()
-    with torch.cuda.device(wr.device):
+    with _lib.device(wr.device):
         _lib.check(_lib.lib().qpam_cweight_pack(ctypes.byref(a), _lib.stream_ptr(wr.device)), "qpam_cweight_pack")
     return w
 
@@ -96,7 +96,7 @@ def _unpack(layout, g, slices, wr, wi, tail, rows):
     a.g_wr, a.g_wi = g_wr.data_ptr(), g_wi.data_ptr()
     if tail is not None:
         a.g_tail = g_tail.data_ptr()
-    with torch.cuda.device(wr.device):
+    with _lib.device(wr.device):
         _lib.check(_lib.lib().qpam_cweight_unpack(ctypes.byref(a), _lib.stream_ptr(wr.device)), "qpam_cweight_unpack")
     return g_wr, g_wi, g_tail
 
@@ -105,7 +105,7 @@ def _cabs(x2):
     """|z| per complex feature of x2 [..., 2C] (qpam_cabs_fwd, cabs of
     v11/complex_ops.py:86-87) -> [..., C] in x2's dtype."""
     mag = torch.empty(x2.shape[:-1] + (x2.shape[-1] // 2,), device=x2.device, dtype=x2.dtype)
-    with torch.cuda.device(x2.device):
+    with _lib.device(x2.device):
         _lib.check(_lib.lib().qpam_cabs_fwd(_code(x2), mag.numel(), x2.data_ptr(), mag.data_ptr(),
                                             _lib.stream_ptr(x2.device)), "qpam_cabs_fwd")
     return mag
@@ -134,7 +134,7 @@ class _LinearIn(torch.autograd.Function):
             if mag is not None and g_mag is not None:
                 # the gradient through |x| added into the projections' in one pass
                 gm = g_mag.to(mag.dtype).contiguous()
-                with torch.cuda.device(x2.device):
+                with _lib.device(x2.device):
                     _lib.check(_lib.lib().qpam_cabs_bwd_acc(_code(x2), mag.numel(), x2.data_ptr(), mag.data_ptr(),
                                                             gm.data_ptr(), gx.data_ptr(),
                                                             _lib.stream_ptr(x2.device)), "qpam_cabs_bwd_acc")
@@ -238,7 +238,7 @@ class _GateLinear(torch.autograd.Function):
         s = _splits(n, out, inp)
         gws = torch.bmm(g2.view(s, n // s, out).transpose(1, 2), x2.view(s, n // s, inp))   # [S, out, in]
         gw = torch.empty(out, inp, device=w.device, dtype=w.dtype)
-        with torch.cuda.device(w.device):
+        with _lib.device(w.device):
             _lib.check(_lib.lib().qpam_slice_sum(_code(gws), _code(gw), s, out * inp, out * inp, gws.data_ptr(),
                                                  gw.data_ptr(), _lib.stream_ptr(w.device)), "qpam_slice_sum")
         gb = (_ones_row(n, g2) @ g2).view(out).to(ctx.b_dtype)

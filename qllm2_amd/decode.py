@@ -151,7 +151,7 @@ def decode_step(state, q, k, v, gamma, *, active=None, rot=None, q_scale=1.0, ou
             raise ValueError(f"pos must hold one position per slot ({n_slots}), got {pos.numel()}")
         a.rope, a.pos, a.rope_len = rope.data_ptr(), pos.data_ptr(), rope.shape[0]
     L = _lib.lib()
-    with torch.cuda.device(state.device):
+    with _lib.device(state.device):
         _lib.check(L.qpam_decode_step(a, _lib.stream_ptr(state.device)), "qpam_decode_step")
     return y
 
@@ -234,7 +234,7 @@ def decode_step_proj(state, proj, dt_bias, *, gate=None, protect_col=-1, phase_c
         if pos.numel() != n_slots:
             raise ValueError(f"pos must hold one position per slot ({n_slots}), got {pos.numel()}")
         a.rope, a.pos, a.rope_len = rope.data_ptr(), pos.data_ptr(), rope.shape[0]
-    with torch.cuda.device(state.device):
+    with _lib.device(state.device):
         _lib.check(_lib.lib().qpam_decode_step(a, _lib.stream_ptr(state.device)), "qpam_decode_step")
     return y
 
@@ -267,7 +267,7 @@ class _DecodeStep(torch.autograd.Function):
         a.state, a.gamma, a.q, a.k, a.v, a.dy = (t.data_ptr() for t in (state, gamma, q, k, v, dy))
         a.dstate_new = dnew.data_ptr() if dnew is not None else None
         a.dstate, a.dgamma, a.dq, a.dk, a.dv = (t.data_ptr() for t in (dstate, dgamma, dq, dk, dv))
-        with torch.cuda.device(state.device):
+        with _lib.device(state.device):
             _lib.check(_lib.lib().qpam_decode_step_bwd(a, _lib.stream_ptr(state.device)), "qpam_decode_step_bwd")
         return dstate, dgamma, dv, dk, dq
 

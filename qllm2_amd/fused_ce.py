@@ -22,6 +22,7 @@ import torch
 from torch import Tensor
 
 from . import _lib, _reference
+from ._ops import op
 
 __all__ = ["fused_linear_cross_entropy", "linear_ce_per_token", "linear_ce_stats"]
 
@@ -69,7 +70,7 @@ def _run_fwd(h, w, dtype, targets, mask, ignore_index, want_correct):
     nbytes = L.qpam_ce_fwd_workspace_size(a)
     ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
     a.workspace, a.workspace_bytes = ws.data_ptr(), nbytes
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(L.qpam_ce_fwd(a, _lib.stream_ptr(dev)), "qpam_ce_fwd")
     return lse, loss, correct, red
 
@@ -85,7 +86,7 @@ def _prep_targets(targets, mask, n):
     return targets, mask
 
 
-@torch.library.custom_op("qpam::ce_fwd", mutates_args=())
+@op("qpam::ce_fwd")
 def ce_fwd_op(hidden_rows: Tensor, weight_matrix: Tensor, targets: Tensor, mask: Optional[Tensor],
               ignore_index: int) -> List[Tensor]:
     """Returns [loss (0-d fp32, as the reference's fp32 chunk sums), lse [N] fp32, denom (0-d fp32)]."""
@@ -104,7 +105,7 @@ def _(hidden_rows, weight_matrix, targets, mask, ignore_index):
             hidden_rows.new_empty((), dtype=torch.float32)]
 
 
-@torch.library.custom_op("qpam::ce_bwd", mutates_args=())
+@op("qpam::ce_bwd")
 def ce_bwd_op(hidden_rows: Tensor, weight_matrix: Tensor, targets: Tensor, mask: Optional[Tensor],
               ignore_index: int, lse: Tensor, grad_scale: Tensor, chunk: int, dw_fp32: bool = False) -> List[Tensor]:
     """Returns [d hidden_rows, d weight_matrix] in the input dtypes (d
@@ -136,7 +137,7 @@ def ce_bwd_op(hidden_rows: Tensor, weight_matrix: Tensor, targets: Tensor, mask:
     nbytes = L.qpam_ce_bwd_workspace_size(a)
     ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
     a.workspace, a.workspace_bytes = ws.data_ptr(), nbytes
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(L.qpam_ce_bwd(a, _lib.stream_ptr(dev)), "qpam_ce_bwd")
     return [dh.to(hidden_rows.dtype), dw if fp32_dw else dw.to(weight_matrix.dtype)]
 

@@ -87,7 +87,7 @@ def resid_norm(x, scale, eps, y=None, y_scale=None, out_dtype=torch.float32):
         a.y, a.y_dtype, a.ldy, a.y_scale = y.data_ptr(), _code(y), y.stride(0), y_scale.data_ptr()
     a.norm_scale = scale.data_ptr()
     a.out, a.out_dtype, a.ldo = out.data_ptr(), _code(out), out.stride(0)
-    with torch.cuda.device(x.device):
+    with _lib.device(x.device):
         _lib.check(_lib.lib().qpam_resid_norm(ctypes.byref(a), _lib.stream_ptr(x.device)), "qpam_resid_norm")
     return out
 
@@ -114,7 +114,7 @@ def cgu_mix(gu, hid, bias, beta=None, phase_alpha=None, phase_beta=None, out_dty
     a.phase_alpha = phase_alpha.data_ptr() if phase_alpha is not None else None
     a.phase_beta = phase_beta.data_ptr() if phase_beta is not None else None
     a.out, a.out_dtype, a.ldo = out.data_ptr(), _code(out), out.stride(0)
-    with torch.cuda.device(gu.device):
+    with _lib.device(gu.device):
         _lib.check(_lib.lib().qpam_cgu_mix(ctypes.byref(a), _lib.stream_ptr(gu.device)), "qpam_cgu_mix")
     return out
 

@@ -12,7 +12,7 @@ fp32 MFMA, forward and backward, over the reference's chunks of delta_chunk
 steps (its clamped decay matrix and state-write weights included); the single
 step uses the recurrence's exact write weight.
 
-`delta_planar` is differentiable (torch.library custom op with a registered
+`delta_planar` is differentiable (a registered operator, _ops.py, with an
 autograd formula); `forward_delta` and `recur_step_delta` keep the reference
 methods' split-real signatures.
 """
@@ -23,6 +23,7 @@ import torch
 from torch import Tensor
 
 from . import _lib, planes
+from ._ops import op
 from .pam_scan import _cview, _mview
 
 CHUNK_EPS = 1e-6
@@ -70,7 +71,7 @@ def _fill(q_re, q_im, k_re, k_im, v_re, v_im, gamma, beta, s0_re, s0_im, q_scale
     return a, keep
 
 
-@torch.library.custom_op("qpam::delta_fwd", mutates_args=())
+@op("qpam::delta_fwd")
 def delta_fwd_op(q_re: Tensor, q_im: Tensor, k_re: Tensor, k_im: Tensor, v_re: Tensor, v_im: Tensor,
                  gamma: Tensor, beta: Tensor, s0_re: Optional[Tensor], s0_im: Optional[Tensor], q_scale: float,
                  gamma_eps: float, chunk: int, exact_write: bool, keep_workspace: bool) -> List[Tensor]:
@@ -103,7 +104,7 @@ def _delta_fwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, beta, s0_re, s0_im, q_
         # caching allocator keeps the block for the next call)
         scratch = torch.empty((L.qpam_delta_scratch_size(a) + 3) // 4, device=dev, dtype=torch.float32)
         a.scratch, a.scratch_bytes = scratch.data_ptr(), scratch.numel() * 4
-        with torch.cuda.device(dev):
+        with _lib.device(dev):
             _lib.check(L.qpam_delta_fwd(a, _lib.stream_ptr(dev)), "qpam_delta_fwd")
         del scratch
     else:
@@ -135,7 +136,7 @@ def _(q_re, q_im, k_re, k_im, v_re, v_im, gamma, beta, s0_re, s0_im, q_scale, ga
     return [y, torch.empty_like(y), s, torch.empty_like(s), ws]
 
 
-@torch.library.custom_op("qpam::delta_bwd", mutates_args=())
+@op("qpam::delta_bwd")
 def delta_bwd_op(q_re: Tensor, q_im: Tensor, k_re: Tensor, k_im: Tensor, v_re: Tensor, v_im: Tensor,
                  gamma: Tensor, beta: Tensor, s0_re: Optional[Tensor], s0_im: Optional[Tensor], q_scale: float,
                  gamma_eps: float, chunk: int, exact_write: bool, ws: Tensor, dy_re: Tensor, dy_im: Tensor,
@@ -177,7 +178,7 @@ def _delta_bwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, beta, s0_re, s0_im, q_
     nbytes = L.qpam_delta_bwd_workspace_size(g)
     ws2 = torch.empty((nbytes + 3) // 4 + 4, device=dev, dtype=torch.float32)
     g.workspace, g.workspace_bytes = ws2.data_ptr(), ws2.numel() * 4
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(L.qpam_delta_bwd(g, _lib.stream_ptr(dev)), "qpam_delta_bwd")
     del keep
     return outs + [dgamma, dbeta] + ds0
@@ -261,7 +262,7 @@ def delta_planar(q_re, q_im, k_re, k_im, v_re, v_im, gamma, beta, *, q_scale, ga
 
 # ---------------------------------------------------------------- split-real front end
 
-@torch.library.custom_op("qpam::delta_il_fwd", mutates_args=())
+@op("qpam::delta_il_fwd")
 def delta_il_fwd_op(q: Tensor, k: Tensor, v: Tensor, gamma: Tensor, beta: Tensor, q_scale: float, chunk: int,
                     keep_workspace: bool) -> List[Tensor]:
     """The delta write on split-real q, k, v [B,H,T,d,2] (d <= 64, fp32 or bf16),
@@ -282,7 +283,7 @@ def _(q, k, v, gamma, beta, q_scale, chunk, keep_workspace):
             q.new_empty(_ws_bytes(B, H, T, chunk=chunk) // 4 if keep_workspace else 0, dtype=f32)]
 
 
-@torch.library.custom_op("qpam::delta_il_bwd", mutates_args=())
+@op("qpam::delta_il_bwd")
 def delta_il_bwd_op(pl: Tensor, gamma: Tensor, beta: Tensor, q_scale: float, chunk: int, ws: Tensor,
                     dy: Optional[Tensor], ds: Optional[Tensor], d: int, bf16: bool) -> List[Tensor]:
     """[dq, dk, dv [B,H,T,d,2] (bf16 or fp32), dgamma, dbeta]."""

@@ -77,7 +77,7 @@ class _Fold(torch.autograd.Function):
         atot = torch.empty(B * H, n, d, device=dev, dtype=torch.float32)
         a = _Fold._args(q, k, gamma, chunk, q_scale)
         a.qf, a.kf, a.wf, a.atot = qf.data_ptr(), kf.data_ptr(), wf.data_ptr(), atot.data_ptr()
-        with torch.cuda.device(dev):
+        with _lib.device(dev):
             _lib.check(_lib.lib().qpam_pc_fold_fwd(ctypes.byref(a), _lib.stream_ptr(dev)), "qpam_pc_fold_fwd")
         ctx.save_for_backward(q, k, gamma)
         ctx.chunk, ctx.q_scale = chunk, q_scale
@@ -106,7 +106,7 @@ class _Fold(torch.autograd.Function):
         a = _Fold._args(q, k, gamma, ctx.chunk, ctx.q_scale)
         a.dqf, a.dkf, a.dwf, a.datot = (_ptr(g) for g in grads)
         a.dq, a.dk, a.dgamma = dq.data_ptr(), dk.data_ptr(), dgamma.data_ptr()
-        with torch.cuda.device(q.device):
+        with _lib.device(q.device):
             _lib.check(_lib.lib().qpam_pc_fold_bwd(ctypes.byref(a), _lib.stream_ptr(q.device)), "qpam_pc_fold_bwd")
         return dq, dk, dgamma, None, None
 
@@ -117,7 +117,7 @@ def _scan(x, a, out, init, fin, reverse):
     s.N, s.n, s.d = N, n, d
     s.x, s.a, s.out, s.init, s.fin = x.data_ptr(), a.data_ptr(), out.data_ptr(), _ptr(init), _ptr(fin)
     s.reverse = 1 if reverse else 0
-    with torch.cuda.device(x.device):
+    with _lib.device(x.device):
         _lib.check(_lib.lib().qpam_pc_scan(ctypes.byref(s), _lib.stream_ptr(x.device)), "qpam_pc_scan")
 
 
@@ -176,7 +176,7 @@ class _Chunked(torch.autograd.Function):
         s_fin = torch.empty(B, H, d, d, 2, **f32)
         a = _Chunked._args(q, k, v, gamma, chunk, q_scale, x, atot)
         a.y, a.s_fin = y.data_ptr(), s_fin.data_ptr()
-        with torch.cuda.device(q.device):
+        with _lib.device(q.device):
             _lib.check(_lib.lib().qpam_pc_fwd(ctypes.byref(a), _lib.stream_ptr(q.device)), "qpam_pc_fwd")
         ctx.save_for_backward(q, k, v, gamma, x, atot)
         ctx.chunk, ctx.q_scale = chunk, q_scale
@@ -207,7 +207,7 @@ class _Chunked(torch.autograd.Function):
         a = _Chunked._args(q, k, v, gamma, ctx.chunk, ctx.q_scale, ws, atot)
         a.s_in, a.dy, a.dfin = s_in.data_ptr(), dy.data_ptr(), _ptr(dfin)
         a.dq, a.dk, a.dv, a.dgamma = dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dgamma.data_ptr()
-        with torch.cuda.device(q.device):
+        with _lib.device(q.device):
             _lib.check(_lib.lib().qpam_pc_bwd(ctypes.byref(a), _lib.stream_ptr(q.device)), "qpam_pc_bwd")
         return dq, dk, dv, dgamma, None, None
 

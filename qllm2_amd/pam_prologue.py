@@ -15,7 +15,7 @@ logits dt, and the rest (up to a multiple of 8 columns) padding.  Its
 gradient is produced whole by the backward kernel, so autograd hands it to
 the GEMM's backward without assembling slices.
 
-`pam_prologue` is differentiable (torch.library custom op with a registered
+`pam_prologue` is differentiable (a registered operator, _ops.py, with an
 autograd formula); the gradients of dt_bias and the state offsets are sums of
 the kernel's per-element dpre over the broadcast axes.  The backward writes
 the logits' gradients in the logits' own [B,T,H(,M)] layouts.
@@ -27,6 +27,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
+from ._ops import op
 
 HEAD_DIM = 64                       # the layer's production head dim (the fused decode prologue's)
 HEAD_DIMS = (16, 32, 64, 128)       # head dims of the prologue kernels
@@ -135,7 +136,7 @@ def _fill(proj, protect, phase, routing, dt_bias, dt_bias2, state_offset, rope, 
     return a, keep
 
 
-@torch.library.custom_op("qpam::prologue_fwd", mutates_args=())
+@op("qpam::prologue_fwd")
 def prologue_fwd_op(proj: Tensor, protect: Optional[Tensor], phase: Optional[Tensor], routing: Optional[Tensor],
                     dt_bias: Tensor, dt_bias2: Optional[Tensor], state_offset: Optional[Tensor],
                     rope: Optional[Tensor], H: int, M: int, D: int, rope_offset: int, qk_norm: bool,
@@ -157,7 +158,7 @@ def prologue_fwd_op(proj: Tensor, protect: Optional[Tensor], phase: Optional[Ten
         a.rot_re, a.rot_im = rot[0].data_ptr(), rot[1].data_ptr()
     else:
         rot = [gamma.new_empty(0), gamma.new_empty(0)]
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(_lib.lib().qpam_prologue_fwd(a, _lib.stream_ptr(dev)), "qpam_prologue_fwd")
     del keep
     return outs + [gamma] + rot
@@ -185,7 +186,7 @@ def _gate_covered(gate, protect_col, phase_col, H, M):
     return end == gate.shape[2]
 
 
-@torch.library.custom_op("qpam::prologue_bwd", mutates_args=())
+@op("qpam::prologue_bwd")
 def prologue_bwd_op(proj: Tensor, protect: Optional[Tensor], phase: Optional[Tensor], routing: Optional[Tensor],
                     dt_bias: Tensor, dt_bias2: Optional[Tensor], state_offset: Optional[Tensor],
                     rope: Optional[Tensor], H: int, M: int, D: int, rope_offset: int, qk_norm: bool,
@@ -246,7 +247,7 @@ def prologue_bwd_op(proj: Tensor, protect: Optional[Tensor], phase: Optional[Ten
             if routing is not None:
                 drouting = torch.empty_like(dphase)
                 g.drouting = drouting.data_ptr()
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(_lib.lib().qpam_prologue_bwd(g, _lib.stream_ptr(dev)), "qpam_prologue_bwd")
     del keep, gs
     return [dproj, dprotect, dphase, drouting, dgate, dbias, doffset]
@@ -352,7 +353,7 @@ def prologue_decode(proj, dt_bias, *, n_heads, n_states=1, state_offset=None, pr
     if phase is not None:
         rot = (torch.empty_like(gamma), torch.empty_like(gamma))
         a.rot_re, a.rot_im = rot[0].data_ptr(), rot[1].data_ptr()
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(_lib.lib().qpam_prologue_fwd(a, _lib.stream_ptr(dev)), "qpam_prologue_fwd")
     del keep
     return (outs[0], outs[1]), (outs[2], outs[3]), (outs[4], outs[5]), gamma, rot
@@ -376,21 +377,21 @@ def mag_linear(z, weight, bias=None, out_dtype=torch.float32):
     w = weight.float().contiguous()
     b = bias.float().contiguous() if bias is not None else None
     out = torch.empty(n, G, device=z.device, dtype=out_dtype)
-    with torch.cuda.device(z.device):
+    with _lib.device(z.device):
         _lib.check(_lib.lib().qpam_mag_linear(_dt_code(z), _dt_code(out), n, dim, G, z.data_ptr(), w.data_ptr(),
                                               b.data_ptr() if b is not None else None, out.data_ptr(), G,
                                               _lib.stream_ptr(z.device)), "qpam_mag_linear")
     return out
 
 
-@torch.library.custom_op("qpam::cabs", mutates_args=())
+@op("qpam::cabs")
 def cabs_op(z: Tensor) -> Tensor:
     """|z| = sqrt(re^2 + im^2 + 1e-8) of a complex [..., 2] tensor (fp32 or bf16)."""
     if not z.is_cuda:
         raise ValueError("qpam cabs: tensors must be on the GPU (no CPU path in this library)")
     zc = z.contiguous()
     mag = torch.empty(z.shape[:-1], device=z.device, dtype=z.dtype)
-    with torch.cuda.device(z.device):
+    with _lib.device(z.device):
         _lib.check(_lib.lib().qpam_cabs_fwd(_dt_code(z), mag.numel(), zc.data_ptr(), mag.data_ptr(),
                                             _lib.stream_ptr(z.device)), "qpam_cabs_fwd")
     return mag
@@ -401,11 +402,11 @@ def _(z):
     return z.new_empty(z.shape[:-1])
 
 
-@torch.library.custom_op("qpam::cabs_bwd", mutates_args=())
+@op("qpam::cabs_bwd")
 def cabs_bwd_op(z: Tensor, mag: Tensor, gmag: Tensor) -> Tensor:
     zc, gc = z.contiguous(), gmag.contiguous()
     gz = torch.empty_like(zc)
-    with torch.cuda.device(z.device):
+    with _lib.device(z.device):
         _lib.check(_lib.lib().qpam_cabs_bwd(_dt_code(z), mag.numel(), zc.data_ptr(), mag.data_ptr(), gc.data_ptr(),
                                             gz.data_ptr(), _lib.stream_ptr(z.device)), "qpam_cabs_bwd")
     return gz

@@ -7,8 +7,8 @@ Planar API: every complex tensor is a pair of real planes.  q, k, v are
 Outputs Y (fp32 planes [B, H, T, d]) and the final state S (fp32 planes
 [M, B, H, d, d]).  Math: v11/model.py:378-417 (M = 1) and 657-781 (M > 1).
 
-The ops are registered with torch.library (custom_op + register_fake +
-register_autograd) so autograd and torch.compile see them as single nodes.
+The ops are registered with torch.library (_ops.py: register_fake and
+register_autograd), so autograd and torch.compile see them as single nodes.
 
 Chunking: the kernels run chunks of 16, 32 or 64 steps.  With gamma + 1e-6 < 1
 the chunked result does not depend on the chunk length (every term is a
@@ -22,6 +22,7 @@ import torch
 from torch import Tensor
 
 from . import _lib, planes
+from ._ops import op
 
 KERNEL_CHUNKS = (16, 32, 64)
 SEG = 4  # 64-step chunks per segment of the bf16 kernels (workspace layout)
@@ -53,43 +54,35 @@ def _dtype_code(t):
 
 
 def _aligned_plane(t):
+    if t.is_contiguous() and t.data_ptr() % 16 == 0:  # rows of 64 elements
+        return t
     vec = 4 if t.dtype == torch.float32 else 8
     ok = t.stride(-1) == 1 and all(s % vec == 0 for s in t.stride()[:-1]) and t.data_ptr() % 16 == 0
     return t if ok else t.contiguous()
 
 
 def _cview(re, im):
-    if re.stride() != im.stride():
+    st = re.stride()
+    if st != im.stride():
         im = im.contiguous() if re.is_contiguous() else im
         re = re.contiguous()
         im = im.contiguous()
-    v = _lib.CView()
-    v.re, v.im = re.data_ptr(), im.data_ptr()
-    v.s0, v.s1, v.s2 = re.stride(0), re.stride(1), re.stride(2)
-    return v, re, im
+        st = re.stride()
+    return _lib.CView(re.data_ptr(), im.data_ptr(), *st[:3]), re, im
 
 
 def _mview(re, im):
-    v = _lib.MView()
-    v.re, v.im = re.data_ptr(), im.data_ptr()
-    v.s0, v.s1, v.s2 = re.stride(0), re.stride(1), re.stride(2)
-    return v
+    return _lib.MView(re.data_ptr(), im.data_ptr(), *re.stride()[:3])
 
 
 def _fill_args(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, s0_im, q_scale, chunk):
     M, B, H, T = gamma.shape
-    d = q_re.shape[-1]
-    a = _lib.ScanArgs()
-    a.B, a.H, a.T, a.d, a.C, a.M = B, H, T, d, chunk, M
-    a.dtype = _dtype_code(q_re)
-    a.q_scale = float(q_scale)
-    keep = []
-    for name, (re, im) in (("q", (q_re, q_im)), ("k", (k_re, k_im)), ("v", (v_re, v_im))):
-        view, re, im = _cview(_aligned_plane(re), _aligned_plane(im))
-        keep += [re, im]
-        setattr(a, name, view)
-    a.gamma = gamma.data_ptr()
-    a.sg_m, a.sg_b, a.sg_h, a.sg_t = gamma.stride()
+    q, qr, qi = _cview(_aligned_plane(q_re), _aligned_plane(q_im))
+    k, kr, ki = _cview(_aligned_plane(k_re), _aligned_plane(k_im))
+    v, vr, vi = _cview(_aligned_plane(v_re), _aligned_plane(v_im))
+    keep = [qr, qi, kr, ki, vr, vi]
+    a = _lib.ScanArgs(B, H, T, q_re.shape[-1], chunk, M, _dtype_code(q_re), q_scale, 0, 0, q, k, v, gamma.data_ptr(),
+                      *gamma.stride())
     if rot_re is not None:
         if rot_re.stride() != rot_im.stride():
             rot_re, rot_im = rot_re.contiguous(), rot_im.contiguous()
@@ -109,10 +102,11 @@ def _validate(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, 
     if gamma.dim() != 4:
         raise ValueError("gamma must be [M, B, H, T]")
     M, B, H, T = gamma.shape
+    want, dtype = (B, H, T), q_re.dtype
     for t in (q_re, q_im, k_re, k_im, v_re, v_im):
-        if t.dim() != 4 or tuple(t.shape[:3]) != (B, H, T):
+        if t.dim() != 4 or t.shape[:3] != want:
             raise ValueError(f"q/k/v planes must be [B={B}, H={H}, T={T}, d], got {tuple(t.shape)}")
-        if t.dtype != q_re.dtype:
+        if t.dtype != dtype:
             raise ValueError("q, k, v must share one dtype")
         if not t.is_cuda:
             raise ValueError("qpam scan: tensors must be on the GPU (no CPU path in this library)")
@@ -123,14 +117,14 @@ def _validate(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, 
     if M > 4:
         raise NotImplementedError("the HIP scan supports up to 4 states")
     for t in (rot_re, rot_im):
-        if t is not None and (tuple(t.shape) != (M, B, H, T) or t.dtype != torch.float32):
+        if t is not None and (t.shape != gamma.shape or t.dtype != torch.float32):
             raise ValueError("rot planes must be fp32 [M, B, H, T]")
     for t in (s0_re, s0_im):
-        if t is not None and (tuple(t.shape) != (M, B, H, 64, 64) or t.dtype != torch.float32):
+        if t is not None and (t.shape != (M, B, H, 64, 64) or t.dtype != torch.float32):
             raise ValueError("s0 planes must be fp32 [M, B, H, 64, 64]")
 
 
-@torch.library.custom_op("qpam::scan_fwd", mutates_args=())
+@op("qpam::scan_fwd")
 def scan_fwd_op(q_re: Tensor, q_im: Tensor, k_re: Tensor, k_im: Tensor, v_re: Tensor, v_im: Tensor,
                 gamma: Tensor, rot_re: Optional[Tensor], rot_im: Optional[Tensor], s0_re: Optional[Tensor],
                 s0_im: Optional[Tensor], q_scale: float, chunk: int, y_layout: int) -> List[Tensor]:
@@ -169,7 +163,7 @@ def _scan_fwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, 
     if prof is not None:
         a.prof_ev[0], a.prof_ev[1] = prof.ev[0], prof.ev[1]
         _PROFILE["fwd"] = None
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(L.qpam_scan_fwd(a, _lib.stream_ptr(dev)), "qpam_scan_fwd")
     del keep
     return [y_re, y_im, s_re, s_im, ws]
@@ -208,7 +202,7 @@ def _(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, s0_im, q
     return [y, torch.empty_like(y), s, torch.empty_like(s), ws]
 
 
-@torch.library.custom_op("qpam::scan_bwd", mutates_args=())
+@op("qpam::scan_bwd")
 def scan_bwd_op(q_re: Tensor, q_im: Tensor, k_re: Tensor, k_im: Tensor, v_re: Tensor, v_im: Tensor,
                 gamma: Tensor, rot_re: Optional[Tensor], rot_im: Optional[Tensor], s0_re: Optional[Tensor],
                 s0_im: Optional[Tensor], q_scale: float, chunk: int, ws: Tensor, dy_re: Tensor, dy_im: Tensor,
@@ -267,7 +261,7 @@ def _scan_bwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, 
     nbytes = L.qpam_scan_bwd_workspace_size(bw)
     ws2 = torch.empty((nbytes + 3) // 4 + 1, device=dev, dtype=torch.float32)
     bw.workspace, bw.workspace_bytes = ws2.data_ptr(), ws2.numel() * 4
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(L.qpam_scan_bwd(bw, _lib.stream_ptr(dev)), "qpam_scan_bwd")
     del keep
     return outs + [dgamma, drot_re, drot_im, ds0_re, ds0_im]
@@ -463,7 +457,7 @@ def _scan_blocks(q_re, q_im, k_re, k_im, v_re, v_im, gamma, q_scale, chunk, rot,
 
 # ---------------------------------------------------------------- split-real front end
 
-@torch.library.custom_op("qpam::scan_il_fwd", mutates_args=())
+@op("qpam::scan_il_fwd")
 def scan_il_fwd_op(q: Tensor, k: Tensor, v: Tensor, gamma: Tensor, rot_re: Optional[Tensor],
                    rot_im: Optional[Tensor], q_scale: float, chunk: int) -> List[Tensor]:
     """The scan on split-real q, k, v [B,H,T,d,2] (d <= 64, fp32 or bf16): one
@@ -487,7 +481,7 @@ def _(q, k, v, gamma, rot_re, rot_im, q_scale, chunk):
             q.new_empty((nbytes + 3) // 4, dtype=torch.float32)]
 
 
-@torch.library.custom_op("qpam::scan_il_bwd", mutates_args=())
+@op("qpam::scan_il_bwd")
 def scan_il_bwd_op(pl: Tensor, gamma: Tensor, rot_re: Optional[Tensor], rot_im: Optional[Tensor], q_scale: float,
                    chunk: int, ws: Tensor, dy: Optional[Tensor], ds: Optional[Tensor], d: int) -> List[Tensor]:
     """[dq, dk, dv [B,H,T,d,2] in the planes' dtype, dgamma, drot_re, drot_im]."""

@@ -32,15 +32,11 @@ def _pairs(x):
 
 
 def _launch(items, merge, device):
-    a = _lib.PlanesArgs()
-    a.count, a.merge = len(items), merge
-    for it, (il, re, im, n0, n1, n2, n2_il, d, dp, ls, ps) in zip(a.item, items):
-        it.il, it.re, it.im = il.data_ptr(), re.data_ptr(), im.data_ptr()
-        it.l0, it.l1, it.l2 = ls
-        it.p0, it.p1, it.p2 = ps
-        it.n0, it.n1, it.n2, it.n2_il, it.d, it.dp = n0, n1, n2, n2_il, d, dp
-        it.il_dtype, it.pl_dtype = _CODE[il.dtype], _CODE[re.dtype]
-    with torch.cuda.device(device):
+    a = _lib.PlanesArgs(len(items), merge)
+    for i, (il, re, im, n0, n1, n2, n2_il, d, dp, ls, ps) in enumerate(items):
+        a.item[i] = _lib.PlanesItem(il.data_ptr(), *ls, re.data_ptr(), im.data_ptr(), *ps, n0, n1, n2, n2_il, d, dp,
+                                    _CODE[il.dtype], _CODE[re.dtype])
+    with _lib.device(device):
         _lib.check(_lib.lib().qpam_planes(a, _lib.stream_ptr(device)), "qpam_planes")
 
 

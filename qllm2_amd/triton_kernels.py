@@ -29,6 +29,7 @@ import torch.nn.functional as F
 from torch import Tensor
 
 from . import _lib, _reference
+from ._ops import op
 
 __all__ = ["fused_decay_matrix", "fused_complex_norm", "fused_mod_swish", "fused_mod_relu", "fused_cgu_gate",
            "set_triton_enabled", "triton_enabled", "HAS_TRITON", "HAS_HIP"]
@@ -85,13 +86,13 @@ def _pt_decay_matrix(decay_gamma: Tensor, seq_len: int) -> Tensor:
 
 # ---------------------------------------------------------------- decay matrix (HIP forward)
 
-@torch.library.custom_op("qpam::decay_matrix", mutates_args=())
+@op("qpam::decay_matrix")
 def decay_matrix_op(decay_gamma: Tensor, seq_len: int) -> Tensor:
     g = decay_gamma.to(torch.float32).contiguous()
     n = g.shape[0]
     out = torch.empty(n, seq_len, seq_len, device=g.device, dtype=torch.float32)
     L = _lib.lib()
-    with torch.cuda.device(g.device):
+    with _lib.device(g.device):
         _lib.check(L.qpam_decay_matrix(n, seq_len, g.data_ptr(), g.stride(0), out.data_ptr(),
                                        _lib.stream_ptr(g.device)), "qpam_decay_matrix")
     return out
@@ -157,13 +158,13 @@ def _none_if_empty(t):
     return t if t.numel() else None
 
 
-@torch.library.custom_op("qpam::cplx_fwd", mutates_args=())
+@op("qpam::cplx_fwd")
 def cplx_fwd_op(op: int, z: Tensor, up: Optional[Tensor], p0: Optional[Tensor], p1: Optional[Tensor],
                 eps: float) -> Tensor:
     out = torch.empty_like(z)
     a = _cplx_args(op, z, up, p0, p1, eps)
     a.out = _lib.ptr(out)
-    with torch.cuda.device(z.device):
+    with _lib.device(z.device):
         _lib.check(_lib.lib().qpam_cplx_fwd(ctypes.byref(a), _lib.stream_ptr(z.device)), "qpam_cplx_fwd")
     return out
 
@@ -173,7 +174,7 @@ def _(op, z, up, p0, p1, eps):
     return torch.empty_like(z)
 
 
-@torch.library.custom_op("qpam::cplx_bwd", mutates_args=())
+@op("qpam::cplx_bwd")
 def cplx_bwd_op(op: int, z: Tensor, up: Optional[Tensor], p0: Optional[Tensor], p1: Optional[Tensor], eps: float,
                 gout: Tensor) -> List[Tensor]:
     """[d z, d up, d p0, d p1]; the entries an op has no input for are empty."""
@@ -190,7 +191,7 @@ def cplx_bwd_op(op: int, z: Tensor, up: Optional[Tensor], p0: Optional[Tensor], 
     ws = torch.empty(max(1, (L.qpam_cplx_workspace_size(ctypes.byref(a)) + 3) // 4), device=z.device,
                      dtype=torch.float32)
     a.workspace, a.workspace_bytes = _lib.ptr(ws), ws.numel() * 4
-    with torch.cuda.device(z.device):
+    with _lib.device(z.device):
         _lib.check(L.qpam_cplx_bwd(ctypes.byref(a), _lib.stream_ptr(z.device)), "qpam_cplx_bwd")
     return [gz, gup, gp0, gp1]
 
