@@ -74,6 +74,22 @@ __device__ __forceinline__ void tile_load(F32Tile<ROWS> &t, const float *base, i
     }
 }
 
+// The same tile through a wave-uniform row pointer and one 32-bit lane offset (its
+// loads share one address register).  Rows past the chunk re-read its last step:
+// for consumers that weight those rows by zero or drop their results.
+template <int ROWS>
+__device__ __forceinline__ void tile_load_u(F32Tile<ROWS> &t, const float *base, int64_t st, int valid, int tid) {
+    if (valid == ROWS && st >= 0 && st < (1 << 26)) {
+        const unsigned off = (unsigned)(tid >> 4) * (unsigned)st + 4u * (tid & 15);
+#pragma unroll
+        for (int i = 0; i < ROWS / 16; ++i) t.v[i] = *reinterpret_cast<const float4 *>(base + 16 * i * st + off);
+    } else {
+#pragma unroll
+        for (int i = 0; i < ROWS / 16; ++i)
+            t.v[i] = *reinterpret_cast<const float4 *>(base + min((tid >> 4) + 16 * i, valid - 1) * st + 4 * (tid & 15));
+    }
+}
+
 template <int ROWS>
 __device__ __forceinline__ void tile_store(float *lds, const F32Tile<ROWS> &t, float scale) {
 #pragma unroll
