@@ -27,4 +27,26 @@ __device__ __forceinline__ void gstep(Gauss &x, float ar, float ai, float br, fl
 __device__ __forceinline__ floatx4 gre(const Gauss &x) { return x.t1 - x.t2; }
 __device__ __forceinline__ floatx4 gim(const Gauss &x) { return x.t3 - x.t1 - x.t2; }
 
+// Interleaved complex LDS tiles: 64 rows of pitch CP.  One 8-byte read gives both
+// parts of an operand down a column, two 16-byte reads four consecutive ones along
+// a row; CP = 68 puts the four lane groups' rows 4 g + r of a column read on
+// distinct banks.
+constexpr int CP = 64 + 4;     // row pitch, complex elements
+constexpr int TILE = 64 * CP;  // complex elements of a tile
+
+// operand reads of a tile: four consecutive elements of a row from column k (16-byte
+// aligned), or one element down a column
+struct Four {
+    float re[4], im[4];
+};
+__device__ __forceinline__ Four row4(const float2 *t, int row, int k) {
+    const float4 a = *reinterpret_cast<const float4 *>(t + row * CP + k);
+    const float4 b = *reinterpret_cast<const float4 *>(t + row * CP + k + 2);
+    return Four{{a.x, a.z, b.x, b.z}, {a.y, a.w, b.y, b.w}};
+}
+__device__ __forceinline__ void put4(float2 *t, int row, int k, const floatx4 &re, const floatx4 &im) {
+    *reinterpret_cast<float4 *>(t + row * CP + k) = make_float4(re[0], im[0], re[1], im[1]);
+    *reinterpret_cast<float4 *>(t + row * CP + k + 2) = make_float4(re[2], im[2], re[3], im[3]);
+}
+
 }  // namespace qpam

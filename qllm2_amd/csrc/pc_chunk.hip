@@ -15,19 +15,13 @@
 // kernels are bound by each block's load, product and store phases following one
 // another at one to three blocks per CU, not by the matrix cores.
 //
-// LDS tiles are interleaved complex, 64 rows of pitch CP: one 8-byte read gives
-// both parts of an operand down a column, two 16-byte reads four consecutive
-// ones along a row; CP = 68 puts the four lane groups' rows 4 g + r of a column
-// read on distinct banks.  Tiles are staged by lane = column, so a wave's access
-// to a row is one 512-byte run.
+// Tiles are staged by lane = column, so a wave's access to a row is one 512-byte run.
 #include "gauss.h"
 
 namespace qpam {
 namespace {
 
 constexpr int CH = 64;                   // rows of a kernel chunk (steps past the chunk's are zero)
-constexpr int CP = CH + 4;               // LDS row pitch, complex elements
-constexpr int TILE = CH * CP;            // complex elements of a tile
 constexpr float GAMMA_FLOOR = 1e-6f;     // gamma.clamp_min(1e-6), v11/model.py:436
 constexpr float CUM_FLOOR = -30.f;       // cumsum.clamp(min=-30), v11/model.py:438
 
@@ -142,21 +136,6 @@ __device__ __forceinline__ float prefix(const Pos<ROWS> &p, const float (&gam)[R
     if (p.grp == CH / ROWS - 1) sLast[p.j] = fmaxf(cs[ROWS - 1], CUM_FLOOR);
     __syncthreads();
     return sLast[p.j];
-}
-
-// operand reads of a tile: four consecutive elements of a row from column k (16-byte
-// aligned), or one element down a column
-struct Four {
-    float re[4], im[4];
-};
-__device__ __forceinline__ Four row4(const float2 *t, int row, int k) {
-    const float4 a = *reinterpret_cast<const float4 *>(t + row * CP + k);
-    const float4 b = *reinterpret_cast<const float4 *>(t + row * CP + k + 2);
-    return Four{{a.x, a.z, b.x, b.z}, {a.y, a.w, b.y, b.w}};
-}
-__device__ __forceinline__ void put4(float2 *t, int row, int k, const floatx4 &re, const floatx4 &im) {
-    *reinterpret_cast<float4 *>(t + row * CP + k) = make_float4(re[0], im[0], re[1], im[1]);
-    *reinterpret_cast<float4 *>(t + row * CP + k + 2) = make_float4(re[2], im[2], re[3], im[3]);
 }
 
 // ------------------------------------------------------------- pc_state --

@@ -20,11 +20,13 @@
 //      gradient of D and cum -> partial dL/dL_t in the workspace;
 //   4. key_side (chunk-parallel, wave = key tile): dK, dV, the decay_last and
 //      total gradients, and the final d gamma of the chunk.
+// fp32 inputs with 64-step chunks run 3 and 4 as one kernel (chunk_grad_f32).
 // bf16 inputs with 64-step chunks: grad_pass_bf16 (the sequential dS chain,
 // writing a bf16 snapshot of dS after every chunk), then chunk_grad_bf16 (the
 // query and key sides of a chunk in one block).
 #include <type_traits>
 
+#include "gauss.h"
 #include "scan_common.h"
 
 namespace qpam {
@@ -843,6 +845,373 @@ __global__ void __launch_bounds__(THREADS) key_side_kernel(BwdParams p) {
             if (lane < valid) {
                 const int64_t go = m * a.sg_m + b * a.sg_b + h * a.sg_h + (int64_t)(c0 + lane) * a.sg_t;
                 p.dgamma[go] = x / (a.gamma[go] + LOG_EPS);
+            }
+        }
+    }
+}
+
+// ------------------------------------------------ fp32, 64-step chunks --
+// The query and key sides of a chunk in one block of 8 waves, Q~, K, V and dY in
+// LDS (148 KB: one block per CU).  Waves 0-3 take query tile w, waves 4-7 key tile
+// w (a SIMD holds one of each, so its causal work does not depend on w); all
+// results accumulate transposed, a lane holding one step and four consecutive
+// columns.  Per state m, S_m and G'_m then take V's and dY's tiles (the lanes keep
+// their own rows of both).  The decay gradient's row sums over s stay in the lane,
+// its column sums over t are DPP row sums into one LDS slice per wave, added in
+// wave order, so the result is reproducible.  Three real MFMAs per complex product
+// (gauss.h), but four separate real sums for the two products the decay gradient is made
+// of (+2 us): over lengths 50-930 and 1-4 states the gradients' error against 64 bits is
+// 0.92 of the two kernels', the worst output of every case no larger.  Bound by the matrix
+// cores (60 us at full rate for 768 chunks) and the causal steps' decay arithmetic between
+// them.  Against the query and key sides as kernels of four waves, each staging all four
+// tiles and using four-product MFMAs: B=4, H=12, T=1000, M=1: 115 + 129 -> 133 us.
+constexpr int CGF_THREADS = 512;
+template <int M>
+constexpr size_t cgf_smem() { return 4 * TILE * sizeof(float2) + (11 * M * 64 + 8 * M) * sizeof(float); }
+
+template <int M>
+__global__ void __launch_bounds__(CGF_THREADS, 2) chunk_grad_f32_kernel(BwdParams p) {
+    extern __shared__ __align__(16) float2 ctile[];
+    float2 *sQ = ctile, *sK = sQ + TILE, *sV = sK + TILE, *sY = sV + TILE;
+    float *sL = reinterpret_cast<float *>(sY + TILE), *sRr = sL + M * 64, *sRi = sRr + M * 64;
+    float *sRow = sRi + M * 64;                     // query side: row sums and the carried read's part
+    float *sDRr = sRow + M * 64, *sDRi = sDRr + M * 64;
+    float *sCol = sDRi + M * 64;                    // [wave][m][64] column sums
+    float *sGp = sCol + 4 * M * 64;                 // [m][64] decay_last terms per key
+    float *sRed = sGp + M * 64;                     // [m][wave] Re<G', S>
+
+    const qpam_scan_args &a = p.a;
+    const int c = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+    const int c0 = c * 64, valid = min(64, a.T - c0), last = (valid - 1) >> 4;
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), w = wv & 3;
+    const int lane = tid & 63, l16 = lane & 15, g = lane >> 4, own = 16 * w + l16;
+    const bool carry = (c > 0) || (a.s0_re != nullptr), qside = wv < 4, active = w <= last;
+
+    // planar rows -> interleaved tiles; thread: rows tid / 16 and + 32, columns 4 (tid % 16) ..
+    const int sr = tid >> 4, sc = 4 * (tid & 15);
+    struct Piece {
+        float4 re[2], im[2];
+    };
+    const auto load = [&](Piece &x, const float *re, const float *im, int64_t st, int rows) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int64_t o = min(sr + 32 * i, rows - 1) * st + sc;
+            x.re[i] = *reinterpret_cast<const float4 *>(re + o);
+            x.im[i] = *reinterpret_cast<const float4 *>(im + o);
+        }
+    };
+    const auto put = [&](float2 *t, const Piece &x, float f, int rows) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int r = sr + 32 * i;
+            const bool ok = r < rows;
+            const float4 u = x.re[i], v = x.im[i];
+            put4(t, r, sc, floatx4{ok ? u.x * f : 0.f, ok ? u.y * f : 0.f, ok ? u.z * f : 0.f, ok ? u.w * f : 0.f},
+                 floatx4{ok ? v.x * f : 0.f, ok ? v.y * f : 0.f, ok ? v.z * f : 0.f, ok ? v.w * f : 0.f});
+        }
+    };
+    const auto view = [&](Piece &x, const qpam_cview &v) {
+        const int64_t o = b * v.s0 + h * v.s1 + (int64_t)c0 * v.s2;
+        load(x, static_cast<const float *>(v.re) + o, static_cast<const float *>(v.im) + o, v.s2, valid);
+    };
+    float gam = 1.f;  // wave m < M: gamma of step `lane` in state m
+    {
+        Piece xq, xk, xv, xy;
+        view(xq, a.q);
+        view(xk, a.k);
+        view(xv, a.v);
+        view(xy, p.dy);
+        if (wv < M) {
+            const float *gp = a.gamma + wv * a.sg_m + b * a.sg_b + h * a.sg_h + (int64_t)c0 * a.sg_t;
+            gam = gp[(int64_t)min(lane, valid - 1) * a.sg_t];
+            float rr = 1.f, ri = 0.f;
+            if (a.rot_re && lane < valid) {
+                const int64_t ro = wv * a.sr_m + b * a.sr_b + h * a.sr_h + (int64_t)(c0 + lane) * a.sr_t;
+                rr = a.rot_re[ro];
+                ri = a.rot_im[ro];
+            }
+            sL[wv * 64 + lane] = log_prefix(gam, valid, lane);
+            sRr[wv * 64 + lane] = rr;
+            sRi[wv * 64 + lane] = ri;
+        }
+        for (int e = tid; e < 8 * M * 64; e += CGF_THREADS) sRow[e] = 0.f;  // sRow, sDRr, sDRi, sCol, sGp
+        put(sQ, xq, a.q_scale, valid);
+        put(sK, xk, 1.f, valid);
+        put(sV, xv, 1.f, valid);
+        put(sY, xy, 1.f, valid);
+    }
+    __syncthreads();
+
+    Four row[4];                                   // query: the dY row of step `own`; key: its V row
+    floatx4 xr[4], xi[4], yr[4], yi[4];            // query: dQ (x); key: dV (x) and dK (y)
+    Gauss acc[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) gz(acc[k]), xr[k] = xi[k] = yr[k] = yi[k] = zero4();
+    if (active) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) row[k] = row4(qside ? sY : sV, own, 16 * k + 4 * g);
+        if (qside) {
+            const int t = own;
+            float rowp[M], grr[M], gri[M];
+#pragma unroll
+            for (int m = 0; m < M; ++m) rowp[m] = grr[m] = gri[m] = 0.f;
+#pragma unroll 1
+            for (int st = 0; st <= w; ++st) {
+                // W[t][s] and dA[t][s], s = 16 st + 4 g + r: the decay gradient is made of
+                // their products' differences, so four real sums here, each on its own
+                floatx4 x[4], y[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) x[k] = y[k] = zero4();
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const Four kk = row4(sK, 16 * st + l16, 16 * k + 4 * g), q = row4(sQ, own, 16 * k + 4 * g);
+                    const Four v = row4(sV, 16 * st + l16, 16 * k + 4 * g);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        x[0] = mfma4(kk.re[r], q.re[r], x[0]);
+                        x[1] = mfma4(kk.im[r], q.im[r], x[1]);
+                        x[2] = mfma4(kk.re[r], q.im[r], x[2]);
+                        x[3] = mfma4(kk.im[r], q.re[r], x[3]);
+                        y[0] = mfma4(v.re[r], row[k].re[r], y[0]);
+                        y[1] = mfma4(v.im[r], row[k].im[r], y[1]);
+                        y[2] = mfma4(v.re[r], row[k].im[r], y[2]);
+                        y[3] = mfma4(v.im[r], row[k].re[r], y[3]);
+                    }
+                }
+                const floatx4 Wr = x[0] + x[1], Wi = x[2] - x[3], Ar = y[0] + y[1], Ai = y[2] - y[3];
+                floatx4 gwr = zero4(), gwi = zero4();
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int s = 16 * st + 4 * g + r;
+                    float col[M];
+                    float dtr = 0.f, dti = 0.f;
+                    const float gdr = Ar[r] * Wr[r] + Ai[r] * Wi[r], gdi = Ai[r] * Wr[r] - Ar[r] * Wi[r];  // dA conj(W)
+#pragma unroll
+                    for (int m = 0; m < M; ++m) {
+                        const float lx = sL[m * 64 + t] - sL[m * 64 + s];
+                        const float Dm = s <= t ? __expf(fminf(lx, 0.f)) : 0.f;
+                        const float rr = sRr[m * 64 + t], ri = sRi[m * 64 + t];
+                        dtr += rr * Dm;
+                        dti += ri * Dm;
+                        // D's clamp passes no gradient; on the diagonal +g and -g cancel
+                        const float gp = (s < t && lx <= 0.f) ? (gdr * rr + gdi * ri) * Dm : 0.f;
+                        rowp[m] += gp;
+                        col[m] = gp;
+                        grr[m] += gdr * Dm;
+                        gri[m] += gdi * Dm;
+                    }
+                    if (s <= t) {
+                        gwr[r] = Ar[r] * dtr + Ai[r] * dti;  // dA conj(D~)
+                        gwi[r] = Ai[r] * dtr - Ar[r] * dti;
+                    }
+#pragma unroll
+                    for (int m = 0; m < M; ++m) {
+                        const float x16 = row16_sum(col[m]);
+                        if (l16 == 0) sCol[(w * M + m) * 64 + s] = x16;
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r)  // dQ^T[j][t] += K[s][j] gW[t][s]
+#pragma unroll
+                    for (int jt = 0; jt < 4; ++jt) {
+                        const float2 e = sK[(16 * st + 4 * g + r) * CP + 16 * jt + l16];
+                        gstep(acc[jt], e.x, e.y, gwr[r], gwi[r]);
+                    }
+            }
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                float u = rowp[m], v = grr[m], z = gri[m];
+                u += __shfl_xor(u, 16), v += __shfl_xor(v, 16), z += __shfl_xor(z, 16);
+                u += __shfl_xor(u, 32), v += __shfl_xor(v, 32), z += __shfl_xor(z, 32);
+                if (g == 0) sRow[m * 64 + t] = u, sDRr[m * 64 + t] = v, sDRi[m * 64 + t] = z;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) xr[k] = gre(acc[k]), xi[k] = gim(acc[k]);
+        } else {
+            // X[t][s] = A[t] . conj(B[s]) times D~ (or its conjugate), t = 16 tt + 4 g + r, lane s = own,
+            // then acc^T[.][s] += C[t][.] conj(X[t][s])
+            const auto side = [&](const float2 *A, const float2 *B, const float2 *Cx, float conj) {
+#pragma unroll 1
+                for (int tt = w; tt <= last; ++tt) {
+                    Gauss x;
+                    gz(x);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const Four u = row4(A, 16 * tt + l16, 16 * k + 4 * g), v = row4(B, own, 16 * k + 4 * g);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) gstep(x, u.re[r], u.im[r], v.re[r], -v.im[r]);
+                    }
+                    const floatx4 ur = gre(x), ui = gim(x);
+                    floatx4 pr, pi;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int t = 16 * tt + 4 * g + r;
+                        float dtr = 0.f, dti = 0.f;
+#pragma unroll
+                        for (int m = 0; m < M; ++m) {
+                            const float Dm = own <= t ? __expf(fminf(sL[m * 64 + t] - sL[m * 64 + own], 0.f)) : 0.f;
+                            dtr += sRr[m * 64 + t] * Dm;
+                            dti += sRi[m * 64 + t] * Dm;
+                        }
+                        dti *= conj;
+                        pr[r] = own <= t ? ur[r] * dtr - ui[r] * dti : 0.f;
+                        pi[r] = own <= t ? ur[r] * dti + ui[r] * dtr : 0.f;
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+#pragma unroll
+                        for (int it = 0; it < 4; ++it) {
+                            const float2 e = Cx[(16 * tt + 4 * g + r) * CP + 16 * it + l16];
+                            gstep(acc[it], e.x, e.y, pr[r], -pi[r]);
+                        }
+                }
+            };
+            side(sQ, sK, sY, 1.f);  // A = W D~, dV = A^H dY
+#pragma unroll
+            for (int k = 0; k < 4; ++k) xr[k] = gre(acc[k]), xi[k] = gim(acc[k]), gz(acc[k]);
+            side(sY, sV, sQ, -1.f);  // gW = dA conj(D~), dK = gW^H Q~
+#pragma unroll
+            for (int k = 0; k < 4; ++k) yr[k] = gre(acc[k]), yi[k] = gim(acc[k]);
+        }
+    }
+
+#pragma unroll 1
+    for (int m = 0; m < M; ++m) {
+        Piece xg, xs;
+        const float *gsrc = gstate(p, m, b, h, c), *ssrc = fstate(p, m, b, h, c);
+        load(xg, gsrc, gsrc + D * D, D, 64);
+        if (carry) load(xs, ssrc, ssrc + D * D, D, 64);
+        __syncthreads();  // the tiles' readers are done
+        put(sY, xg, 1.f, 64);
+        if (carry) {
+            put(sV, xs, 1.f, 64);
+            float part = 0.f;  // g_total = sum Re(conj(G') S)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                part += xg.re[i].x * xs.re[i].x + xg.im[i].x * xs.im[i].x + xg.re[i].y * xs.re[i].y + xg.im[i].y * xs.im[i].y;
+                part += xg.re[i].z * xs.re[i].z + xg.im[i].z * xs.im[i].z + xg.re[i].w * xs.re[i].w + xg.im[i].w * xs.im[i].w;
+            }
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) part += __shfl_xor(part, off);
+            if (lane == 0) sRed[m * 8 + wv] = part;
+        }
+        __syncthreads();
+        if (!active) continue;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) gz(acc[k]);
+        // acc^T[j][own] = sum_i conj(A[i][j]) row[i]
+        const auto columns = [&](const float2 *A) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int jt = 0; jt < 4; ++jt) {
+                        const float2 e = A[(16 * k + 4 * g + r) * CP + 16 * jt + l16];
+                        gstep(acc[jt], e.x, -e.y, row[k].re[r], row[k].im[r]);
+                    }
+        };
+        if (qside) {
+            if (!carry) continue;
+            columns(sV);  // X = dY conj(S); dQ~ += conj(rho) X; g_rho[t] = sum_j conj(q~) X
+            const float cum = __expf(sL[m * 64 + own]), rr = sRr[m * 64 + own], ri = sRi[m * 64 + own];
+            const float rhr = rr * cum, rhi = ri * cum;
+            float pr = 0.f, pi = 0.f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const floatx4 ur = gre(acc[k]), ui = gim(acc[k]);
+                const Four q = row4(sQ, own, 16 * k + 4 * g);
+                xr[k] += rhr * ur + rhi * ui;
+                xi[k] += rhr * ui - rhi * ur;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    pr += q.re[r] * ur[r] + q.im[r] * ui[r];
+                    pi += q.re[r] * ui[r] - q.im[r] * ur[r];
+                }
+            }
+            pr += __shfl_xor(pr, 16), pi += __shfl_xor(pi, 16);
+            pr += __shfl_xor(pr, 32), pi += __shfl_xor(pi, 32);
+            if (g == 0) {  // step `own` is this wave's
+                sDRr[m * 64 + own] += pr * cum;
+                sDRi[m * 64 + own] += pi * cum;
+                sRow[m * 64 + own] += (pr * rr + pi * ri) * cum;  // Re(g_rho conj(r)) cum
+            }
+        } else {
+            const float lx = sL[m * 64 + valid - 1] - sL[m * 64 + own];
+            const float dl = own < valid ? __expf(fminf(lx, 0.f)) : 0.f;
+            columns(sY);  // dK += dl V conj(G')
+#pragma unroll
+            for (int k = 0; k < 4; ++k) yr[k] += dl * gre(acc[k]), yi[k] += dl * gim(acc[k]), gz(acc[k]);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {  // Z = K G'^T; dV += dl Z; gdl = Re<V, Z>
+                const Four kk = row4(sK, own, 16 * k + 4 * g);
+#pragma unroll
+                for (int it = 0; it < 4; ++it) {
+                    const Four gg = row4(sY, 16 * it + l16, 16 * k + 4 * g);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) gstep(acc[it], gg.re[r], gg.im[r], kk.re[r], kk.im[r]);
+                }
+            }
+            float gdl = 0.f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const floatx4 zr = gre(acc[k]), zi = gim(acc[k]);
+                xr[k] += dl * zr;
+                xi[k] += dl * zi;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) gdl += row[k].re[r] * zr[r] + row[k].im[r] * zi[r];
+            }
+            gdl += __shfl_xor(gdl, 16);
+            gdl += __shfl_xor(gdl, 32);
+            if (g == 0) sGp[m * 64 + own] = (own < valid - 1 && lx <= 0.f) ? gdl * dl : 0.f;
+        }
+    }
+    const auto store = [&](const qpam_mview &v, const floatx4 (&re)[4], const floatx4 (&im)[4], float f) {
+        const int64_t o = b * v.s0 + h * v.s1 + (int64_t)(c0 + own) * v.s2 + 4 * g;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            *reinterpret_cast<floatx4 *>(v.re + o + 16 * k) = re[k] * f;
+            *reinterpret_cast<floatx4 *>(v.im + o + 16 * k) = im[k] * f;
+        }
+    };
+    if (own < valid) {
+        if (qside) {
+            store(p.dq, xr, xi, a.q_scale);
+        } else {
+            store(p.dv, xr, xi, 1.f);
+            store(p.dk, yr, yi, 1.f);
+        }
+    }
+    __syncthreads();
+    // d gamma of state m (wave m): dL/dL_t, its reverse cumsum inside the chunk, 1 / (gamma + 1e-6)
+    if (wv < M) {
+        const int m = wv;
+        const float *col = sCol + m * 64 + lane;
+        float x = sRow[m * 64 + lane] - (((col[0] + col[M * 64]) + col[2 * M * 64]) + col[3 * M * 64]);
+        const float gp = sGp[m * 64 + lane];
+        x -= gp;
+        float sum = gp;
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off);
+        if (carry) {
+            float tot = 0.f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) tot += sRed[m * 8 + k];
+            sum += tot * __expf(sL[m * 64 + valid - 1]);
+        }
+        if (lane == valid - 1) x += sum;
+        x = lane < valid ? x : 0.f;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const float y = __shfl_down(x, off);
+            if (lane + off < 64) x += y;
+        }
+        if (lane < valid) {
+            p.dgamma[m * a.sg_m + b * a.sg_b + h * a.sg_h + (int64_t)(c0 + lane) * a.sg_t] = x / (gam + LOG_EPS);
+            if (p.drot_re) {
+                const int64_t ro = m * a.sr_m + b * a.sr_b + h * a.sr_h + (int64_t)(c0 + lane) * a.sr_t;
+                p.drot_re[ro] = sDRr[m * 64 + lane];
+                p.drot_im[ro] = sDRi[m * 64 + lane];
             }
         }
     }
@@ -1793,10 +2162,44 @@ size_t qside_smem() { return (size_t)(6 * C * P + 2 * D * P + 10 * MAX_M * 64) *
 template <int C>
 size_t kside_smem() { return (size_t)(4 * C * P + 4 * D * P + 5 * MAX_M * 64 + 4 + 64) * sizeof(float); }
 
+template <int M>
+int launch_chunk_grad_f32(const BwdParams &p, hipStream_t stream) {
+    const void *k = (const void *)chunk_grad_f32_kernel<M>;
+    QPAM_CHECK_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)cgf_smem<M>()));
+    hipLaunchKernelGGL(chunk_grad_f32_kernel<M>, dim3(p.n_chunks, p.a.H, p.a.B), dim3(CGF_THREADS), cgf_smem<M>(), stream,
+                       p);
+    return launch_status("chunk_grad_f32_kernel");
+}
+
+// chunk_grad_f32 stores gradient rows in 16-byte runs; other output layouts keep
+// the query and key sides as kernels of their own
+bool rows16(const qpam_mview &v) {
+    return (((uintptr_t)v.re | (uintptr_t)v.im) % 16) == 0 && v.s0 % 4 == 0 && v.s1 % 4 == 0 && v.s2 % 4 == 0;
+}
+
 template <typename Tin, int C>
 int launch_bwd(const BwdParams &p, hipStream_t stream) {
     const qpam_scan_args &a = p.a;
     dim3 grid(p.n_chunks, a.H, a.B);
+    if constexpr (std::is_same<Tin, float>::value && C == 64) {
+        if (rows16(p.dq) && rows16(p.dk) && rows16(p.dv)) {
+            const size_t s1 = gcs_smem<C>();
+            QPAM_CHECK_HIP(hipFuncSetAttribute((const void *)grad_chunk_state_kernel<Tin, C>,
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)s1));
+            hipLaunchKernelGGL((grad_chunk_state_kernel<Tin, C>), grid, dim3(THREADS), s1, stream, p);
+            int r = launch_status("grad_chunk_state_kernel");
+            if (r) return r;
+            hipLaunchKernelGGL(grad_state_scan_kernel, dim3(a.M * a.B * a.H * SCAN_BLOCKS), dim3(THREADS), 0, stream, p);
+            r = launch_status("grad_state_scan_kernel");
+            if (r) return r;
+            switch (a.M) {
+                case 1: return launch_chunk_grad_f32<1>(p, stream);
+                case 2: return launch_chunk_grad_f32<2>(p, stream);
+                case 3: return launch_chunk_grad_f32<3>(p, stream);
+                default: return launch_chunk_grad_f32<4>(p, stream);
+            }
+        }
+    }
     const size_t s1 = gcs_smem<C>(), s3 = qside_smem<C>(), s4 = kside_smem<C>();
     QPAM_CHECK_HIP(hipFuncSetAttribute((const void *)grad_chunk_state_kernel<Tin, C>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)s1));

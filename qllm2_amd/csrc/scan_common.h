@@ -131,6 +131,17 @@ __device__ __forceinline__ float chunk_log_prefix(const float *g, int64_t gs, in
     return x;
 }
 
+// The same prefix from a lane's own gamma (lanes past the chunk's steps pass any value).
+__device__ __forceinline__ float log_prefix(float gamma, int valid, int lane) {
+    float x = (lane < valid) ? logf(gamma + LOG_EPS) : 0.f;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        float y = __shfl_up(x, off);
+        if (lane >= off) x += y;
+    }
+    return x;
+}
+
 // Sequential state scans: float4 per thread and blocks per (m, b, h) state.
 constexpr int SCAN_EPT = 2;
 constexpr int SCAN_BLOCKS = (2 * 64 * 64 / 4) / (THREADS * SCAN_EPT);

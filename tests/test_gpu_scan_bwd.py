@@ -369,3 +369,42 @@ def test_scan_backward_deterministic(gpu_lib, dtype, M, T, C):
     for name, a, b in zip(NAMES, runs[0], runs[1]):
         if a is not None:
             assert torch.equal(a, b), f"{name}: differs between two runs"
+
+
+@pytest.mark.parametrize("M,T,with_rot,with_s0", [
+    (1, 1, False, False), (1, 1, False, True),      # one step, without and with a state to carry
+    (2, 15, True, False), (3, 17, True, True),      # around a tile of 16 steps
+    (4, 63, True, True), (1, 64, False, False), (4, 65, True, False),  # around a chunk
+    (2, 16 * 7, True, True), (1, 64 * 3 + 33, False, True),
+])
+def test_fused_chunk_grad_equals_query_and_key_kernels(gpu_lib, monkeypatch, M, T, with_rot, with_s0):
+    """fp32 with 64-step chunks: gradient planes with 16-byte rows take one fused
+    kernel, others the query-side and key-side kernels.  The same pass over planes
+    with rows of 65 elements gives the same gradients within rounding: a gradient
+    chains three sums of at most 128 terms, each kernel within 3 * 128 * 2^-24 of
+    the exact value in norm."""
+    from qllm2_amd import pam_scan
+    B, H, d = 2, 3, 64
+    case = _case(M, B, H, T, d, 7000 + 10 * M + T, with_rot, with_s0, torch.float32)
+    fused = _gpu_grads(*case, d, 64, torch.float32, with_rot)
+    mview, run = pam_scan._mview, pam_scan._scan_bwd
+    pads = []
+
+    def padded_mview(re, im):
+        pads.append([torch.empty(*x.shape[:-1], d + 1, device=x.device)[..., :d] for x in (re, im)])
+        return mview(*pads[-1])
+
+    def padded_bwd(*args):
+        with monkeypatch.context() as mp:
+            mp.setattr(pam_scan, "_mview", padded_mview)
+            out = run(*args)
+        for i, x in enumerate(x for pair in pads for x in pair):
+            out[i].copy_(x)
+        return out
+
+    monkeypatch.setattr(pam_scan, "_scan_bwd", padded_bwd)
+    general = _gpu_grads(*case, d, 64, torch.float32, with_rot)
+    assert pads
+    for name, a, b in zip(NAMES, fused, general):
+        if a is not None:
+            assert float((a - b).norm()) <= 2 * 3 * 128 * 2.0 ** -24 * float(b.norm()), name
