@@ -14,11 +14,11 @@
 // v_i, gamma, beta), so the chunk pass splits a chain's 64 value rows over four
 // blocks.
 //
-// Backward: the same chunked form differentiated, on fp32 MFMA in three
+// Backward: the same chunked form differentiated, on fp32 MFMA in two
 // launches (described at the kernels): a reverse pass along the chunks for the
 // gradient of the state (rows of it are independent again: four blocks per
-// chain), then two chunk-parallel kernels for the score-matrix gradients and
-// for dq, dk, dgamma, dbeta.  The forward leaves what they need in its
+// chain), then a chunk-parallel kernel for the score-matrix gradients and from
+// them dq, dk, dgamma, dbeta.  The forward leaves what they need in its
 // workspace: the state entering every chunk, U, and the chunk's products in the
 // orders the backward reads them.
 #include "gauss.h"
@@ -92,14 +92,8 @@ constexpr int WS_S = 0, WS_U = 2 * D * D, WS_TH = 4 * D * D, WS_AH = WS_TH + NBL
               WS_AA = WS_AH + NBLK * BLK, WS_GA = WS_AA + NBLK * BLK, WS_L = WS_GA + NBLK * BLK,
               WS_REC = WS_L + CH;
 // The backward's workspace, one record per (b, h, chunk): G (the gradient of the
-// state after the chunk) [plane][i][j], dW [plane][t][i], dP = D.dAhat and
-// dGk = beta D.dM in two layouts each (x_Q: transposed accumulator order, lane
-// (l16, g), r <-> t = 16 bt + l16, s = 16 bs + 4 g + r; x_K: accumulator order),
-// and two per-step vectors: the score part of the log-decay gradient and the
-// beta gradient through M.
-constexpr int BW_G = 0, BW_W = 2 * D * D, BW_PQ = 4 * D * D, BW_PK = BW_PQ + NBLK * BLK,
-              BW_GQ = BW_PK + NBLK * BLK, BW_GK = BW_GQ + NBLK * BLK, BW_V = BW_GK + NBLK * BLK,
-              BW_REC = BW_V + 2 * CH;
+// state after the chunk) [plane][i][j] and dW [plane][t][i].
+constexpr int BW_G = 0, BW_W = 2 * D * D, BW_REC = 4 * D * D;
 
 __device__ __forceinline__ int blk(int b, int c) { return b * (b + 1) / 2 + c; }  // c <= b
 
@@ -622,13 +616,6 @@ __device__ __forceinline__ void ops_fetch_up(OpRegs &x, const float *base, int w
     }
 }
 
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), vmcnt / expcnt unconstrained
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ __forceinline__ float wave_sum(float x) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) x += __shfl_xor(x, off);
@@ -850,429 +837,308 @@ __global__ void __launch_bounds__(256, 2) delta_bwd_chain_kernel(qpam_delta_bwd_
     }
 }
 
-// delta_bwd_score_kernel: the score-matrix gradients of one chunk (a block per
-// (b, h, chunk), 4 waves).  U is staged in LDS; wave w forms dAhat on query tile
-// w and dM on query tile 3 - w (five 16 x 16 blocks either way), its dY and dW
-// rows straight from global memory as MFMA operands (k = i in the order
-// 16 q + 4 g + r: 16-byte loads), U rows as 16-byte LDS reads.  dP and dGk leave
-// in both layouts (a 16 x 16 LDS transpose per block and wave); E's row sums and
-// the beta part complete in the wave, its column sums per block through LDS,
-// added in a fixed order.
-__global__ void __launch_bounds__(256) delta_bwd_score_kernel(qpam_delta_bwd_args bw, qpam_delta_args a,
-                                                              int n_chunks) {
-    __shared__ __align__(16) float sUr[CH * KP], sUi[CH * KP];  // U [s][i]
-    __shared__ float sX[4][2][16 * 17];                         // each wave's transpose of one block
-    __shared__ float sRow[2][CH], sCol[2][4][CH], sDb[CH], sL[CH], sBt[CH];
-    const int chain = blockIdx.x / n_chunks, c = blockIdx.x % n_chunks;
-    const int b = chain / a.H, h = chain % a.H;
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
-    const int t0 = c * chunk_len(a), valid = min(chunk_len(a), a.T - t0);
-    const float *rec = static_cast<const float *>(a.workspace) + ((int64_t)chain * n_chunks + c) * WS_REC;
-    float *brec = static_cast<float *>(bw.workspace) + ((int64_t)chain * n_chunks + c) * BW_REC;
-    // this lane's MFMA A rows: dY of step 16 w + l16, dW of step 16 (3 - w) + l16;
-    // element (q, r) is column 16 q + 4 g + r
-    floatx4 opr[2][4], opi[2][4];
-    {
-        const int t = 16 * w + l16;
-        const float f = t < valid ? 1.f : 0.f;
-        const int64_t o = b * bw.dy.s0 + h * bw.dy.s1 + (int64_t)(t0 + min(t, valid - 1)) * bw.dy.s2 + 4 * g;
-        const float *dw = brec + BW_W + (16 * (3 - w) + l16) * D + 4 * g;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            opr[0][q] = *reinterpret_cast<const floatx4 *>(static_cast<const float *>(bw.dy.re) + o + 16 * q) * f;
-            opi[0][q] = *reinterpret_cast<const floatx4 *>(static_cast<const float *>(bw.dy.im) + o + 16 * q) * f;
-            opr[1][q] = *reinterpret_cast<const floatx4 *>(dw + 16 * q);
-            opi[1][q] = *reinterpret_cast<const floatx4 *>(dw + D * D + 16 * q);
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {  // U -> LDS, 16-byte pieces
-        const int e = tid + 256 * k, pl = e >> 10, row = (e >> 4) & 63, c4 = 4 * (e & 15);
-        const floatx4 v = *reinterpret_cast<const floatx4 *>(rec + WS_U + pl * D * D + row * D + c4);
-        *reinterpret_cast<floatx4 *>((pl ? sUi : sUr) + row * KP + c4) = v;
-    }
-    if (w == 0) {
-        sL[lane] = rec[WS_L + lane];
-        const float bt = a.beta[b * a.sg_b + h * a.sg_h + (int64_t)(t0 + min(lane, valid - 1)) * a.sg_t];
-        sBt[lane] = lane < valid ? bt : 0.f;
-    }
-    __syncthreads();
-
-    float rowacc[2][4], db2[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) rowacc[0][r] = rowacc[1][r] = db2[r] = 0.f;
-    float *X = sX[w][0], *Xi = sX[w][1];
-#pragma unroll
-    for (int kind = 0; kind < 2; ++kind) {
-        const int tt = kind ? 3 - w : w;  // query tile of this product
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-            if (st > tt) continue;
-            const int s = 16 * st + l16;
-            // acc[t = 16 tt + 4 g + r][s] = sum_i A[t][i] conj(U[s][i])
-            Gauss x;
-            gz(x);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const floatx4 ur4 = *reinterpret_cast<const floatx4 *>(sUr + s * KP + 16 * q + 4 * g);
-                const floatx4 ui4 = *reinterpret_cast<const floatx4 *>(sUi + s * KP + 16 * q + 4 * g);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) gstep(x, opr[kind][q][r], opi[kind][q][r], ur4[r], -ui4[r]);
-            }
-            const floatx4 dr = gre(x), di = gim(x);
-            const float *src = rec + (kind ? WS_GA : WS_AA) + blk(tt, st) * BLK + lane * 4;
-            const floatx4 xr4 = *reinterpret_cast<const floatx4 *>(src);       // Ahat or D.Gk
-            const floatx4 xi4 = *reinterpret_cast<const floatx4 *>(src + 256);
-            const float Ls = sL[s];
-            floatx4 pr, pi;
-            float cs = 0.f;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int t = 16 * tt + 4 * g + r;
-                const bool keep = kind ? (s < t) : (s <= t);
-                const float lx = sL[t] - Ls;
-                const float Dv = keep ? __expf(fminf(lx, 0.f)) : 0.f;
-                const float through = lx <= 0.f ? 1.f : 0.f;  // D's clamp: no gradient to L past it
-                float e;
-                if (kind == 0) {  // dP = D dAhat; E = Re(conj(Ahat) dAhat)
-                    pr[r] = Dv * dr[r];
-                    pi[r] = Dv * di[r];
-                    e = through * (xr4[r] * dr[r] + xi4[r] * di[r]);
-                } else {  // dM = -acc; dGk = beta D dM; E = beta Re(conj(D.Gk) dM)
-                    const float bt = sBt[t];
-                    const float e2 = -(xr4[r] * dr[r] + xi4[r] * di[r]);
-                    pr[r] = -bt * Dv * dr[r];
-                    pi[r] = -bt * Dv * di[r];
-                    e = through * bt * e2;
-                    db2[r] += e2;
-                }
-                rowacc[kind][r] += e;
-                cs += e;
-            }
-            cs += __shfl_xor(cs, 16);
-            cs += __shfl_xor(cs, 32);
-            if (g == 0) sCol[kind][tt][s] = cs;
-            // x_K layout: the accumulator order
-            float *dk_ = brec + (kind ? BW_GK : BW_PK) + blk(tt, st) * BLK + lane * 4;
-            *reinterpret_cast<floatx4 *>(dk_) = pr;
-            *reinterpret_cast<floatx4 *>(dk_ + 256) = pi;
-            // x_Q layout: lane (l16 = t, g), r <-> s = 4 g + r, through the wave's LDS block
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                X[(4 * g + r) * 17 + l16] = pr[r];
-                Xi[(4 * g + r) * 17 + l16] = pi[r];
-            }
-            wave_lds_sync();
-            floatx4 qr4, qi4;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                qr4[r] = X[l16 * 17 + 4 * g + r];
-                qi4[r] = Xi[l16 * 17 + 4 * g + r];
-            }
-            float *dq_ = brec + (kind ? BW_GQ : BW_PQ) + blk(tt, st) * BLK + lane * 4;
-            *reinterpret_cast<floatx4 *>(dq_) = qr4;
-            *reinterpret_cast<floatx4 *>(dq_ + 256) = qi4;
-            wave_lds_sync();
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const float v0 = row16_sum(rowacc[0][r]), v1 = row16_sum(rowacc[1][r]), vb = row16_sum(db2[r]);
-        if (l16 == 0) {
-            sRow[0][16 * w + 4 * g + r] = v0;
-            sRow[1][16 * (3 - w) + 4 * g + r] = v1;
-            sDb[16 * (3 - w) + 4 * g + r] = vb;
-        }
-    }
-    __syncthreads();
-    if (tid < CH) {
-        const int t = tid;
-        float col = 0.f;
-#pragma unroll
-        for (int kind = 0; kind < 2; ++kind)
-            for (int tt = t >> 4; tt < 4; ++tt) col += sCol[kind][tt][t];
-        brec[BW_V + t] = sRow[0][t] + sRow[1][t] - col;
-        brec[BW_V + CH + t] = sDb[t];
-    }
-}
-
 // delta_bwd_grad_kernel: dq, dk, dgamma and dbeta of one chunk (a block per
-// (b, h, chunk), 8 waves).  K, q~, S and G are staged in LDS (pitch KP: the
-// MFMA reads of rows 4 g + r, 16 consecutive columns, hit distinct banks); waves
-// 0-3 take query tile w: dq~ = dP K + alpha dY conj(S) and the t-side part of dk,
-// dGk K - alpha beta dW conj(S); waves 4-7 key tile w: dP^H q~ + dGk^H K +
-// dl U conj(G).  Outputs accumulate transposed (a lane holds one step and four
-// consecutive columns, so rows leave as 16-byte pieces), with the lane's own
-// operands (dP, dGk blocks in the matching layout, dY, dW, U rows) straight from
-// global memory.  The key side stores its part of dk and the query side adds
-// its own after a barrier; the per-step sums (dalpha, dbeta, ddl) and Re<S, G>
-// meet in LDS, and wave 4 forms dL, its reverse cumsum and dgamma.
-constexpr int G2_TILE = 2 * CH * KP;
-constexpr size_t G2_SMEM = (size_t)(4 * G2_TILE + 7 * CH + 8) * sizeof(float);
+// (b, h, chunk), 8 waves), with the score-matrix gradients kept in LDS.  Four
+// interleaved tiles (142 KB, one block per CU) hold in turn
+//   U, K, -> dP, dGk   scores: waves 0-3 form dP = D.dAhat of query tile w, waves 4-7
+//                      dGk = beta D.dM of tile 3 - w (five 16 x 16 blocks a SIMD); E's
+//                      row sums complete in the wave, its column sums go through LDS
+//   q~, K, dP, dGk     waves 0-3, query tile w: dP K; waves 4-7, key tile w: dP^H q~ +
+//                      dGk^H K and dGk K
+//   q~, K, S, G        waves 0-3: alpha dY conj(S); waves 4-7: dl U conj(G) - alpha beta
+//                      dW conj(S)
+// (each next tile waits in registers), so a step's dq and dk belong to one wave each.
+// Outputs accumulate transposed (a lane holds one step and four consecutive columns, so
+// rows leave as 16-byte pieces); the lane's own dY, dW and U rows come straight from
+// global memory.  All reductions run in a fixed order.  3072 chunks (B=8, H=12, T=2048)
+// move 1.2 GB (230 us at the rate of a large copy) and need 210 us of the matrix cores,
+// which one block per CU overlaps little; a score kernel of its own, handing dP and dGk on
+// in two layouts each, moved 2.3 GB: 132 + 441 -> 533 us, the call 1883 -> 1822 us and
+// 80 KB less workspace per chunk.
+constexpr size_t G2_SMEM = 4 * TILE * sizeof(float2) + (17 * CH + 8) * sizeof(float);
 
-__global__ void __launch_bounds__(512) delta_bwd_grad_kernel(qpam_delta_bwd_args bw, qpam_delta_args a,
-                                                             int n_chunks) {
-    extern __shared__ __align__(16) float sm[];
-    float *sK = sm, *sQ = sK + G2_TILE, *sS = sQ + G2_TILE, *sG = sS + G2_TILE;  // [plane][row][KP]
-    float *sL = sG + G2_TILE, *sBt = sL + CH, *sLp = sBt + CH, *sDb2 = sLp + CH;
-    float *sDa = sDb2 + CH, *sDb = sDa + CH, *sDdl = sDb + CH, *sRed = sDdl + CH;
+__global__ void __launch_bounds__(512, 2) delta_bwd_grad_kernel(qpam_delta_bwd_args bw, qpam_delta_args a,
+                                                                int n_chunks) {
+    extern __shared__ __align__(16) float2 tiles[];
+    float2 *sK = tiles, *sQ = sK + TILE, *sS = sQ + TILE, *sG = sS + TILE;
+    float2 *sU = sQ, *sP = sS, *sH = sG;  // U until q~ comes; dP and dGk until S and G come
+    float *sL = reinterpret_cast<float *>(sG + TILE), *sBt = sL + CH, *sRow = sBt + CH, *sCol = sRow + 2 * CH;
+    float *sDb2 = sCol + 8 * CH, *sDa = sDb2 + CH, *sDb = sDa + CH, *sDdl = sDb + CH, *sDk = sDdl + CH;
+    float *sRed = sDk + CH;
     const int chain = blockIdx.x / n_chunks, c = blockIdx.x % n_chunks;
     const int b = chain / a.H, h = chain % a.H;
-    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
-    const int w = wv & 3;
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), w = wv & 3;
+    const int lane = tid & 63, l16 = lane & 15, g = lane >> 4, own = 16 * w + l16;
     const bool qside = wv < 4;
     const int t0 = c * chunk_len(a), valid = min(chunk_len(a), a.T - t0);
     const float *rec = static_cast<const float *>(a.workspace) + ((int64_t)chain * n_chunks + c) * WS_REC;
     const float *brec = static_cast<const float *>(bw.workspace) + ((int64_t)chain * n_chunks + c) * BW_REC;
-    constexpr int PL = CH * KP;  // offset of the im plane in a staged tile
-    // stage K, q~ (rows past the end zero), S and G: 16 16-byte pieces per thread
+
+    // planar rows -> tiles; thread: rows tid / 16 and + 32, columns 4 (tid % 16) ..
+    const int sr = tid >> 4, sc = 4 * (tid & 15);
+    struct Piece {
+        floatx4 re[2], im[2];
+    };
+    const auto load = [&](Piece &x, const float *re, const float *im, int64_t st, int rows) {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        const int e = tid + 512 * k, m = e >> 11, pl = (e >> 10) & 1, row = (e >> 4) & 63, c4 = 4 * (e & 15);
-        floatx4 v;
-        if (m < 2) {
-            const qpam_cview &x = m ? a.q : a.k;
-            const float *base = static_cast<const float *>(pl ? x.im : x.re);
-            const float f = row < valid ? (m ? a.q_scale : 1.f) : 0.f;
-            v = *reinterpret_cast<const floatx4 *>(base + b * x.s0 + h * x.s1 +
-                                                   (int64_t)(t0 + min(row, valid - 1)) * x.s2 + c4) * f;
-        } else {
-            const float *src = (m == 2 ? rec + WS_S : brec + BW_G) + pl * D * D;
-            v = *reinterpret_cast<const floatx4 *>(src + row * D + c4);
+        for (int i = 0; i < 2; ++i) {
+            const int64_t o = min(sr + 32 * i, rows - 1) * st + sc;
+            x.re[i] = *reinterpret_cast<const floatx4 *>(re + o);
+            x.im[i] = *reinterpret_cast<const floatx4 *>(im + o);
         }
-        *reinterpret_cast<floatx4 *>(sm + m * G2_TILE + pl * PL + row * KP + c4) = v;
-    }
-    if (wv == 0) {
-        sL[lane] = rec[WS_L + lane];
-        const float bt = a.beta[b * a.sg_b + h * a.sg_h + (int64_t)(t0 + min(lane, valid - 1)) * a.sg_t];
-        sBt[lane] = lane < valid ? bt : 0.f;
-        sLp[lane] = brec[BW_V + lane];
-        sDb2[lane] = brec[BW_V + CH + lane];
+    };
+    const auto view = [&](Piece &x, const qpam_cview &v) {
+        const int64_t o = b * v.s0 + h * v.s1 + (int64_t)t0 * v.s2;
+        load(x, static_cast<const float *>(v.re) + o, static_cast<const float *>(v.im) + o, v.s2, valid);
+    };
+    const auto put = [&](float2 *t, const Piece &x, float scale, int rows) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const float f = sr + 32 * i < rows ? scale : 0.f;
+            put4(t, sr + 32 * i, sc, x.re[i] * f, x.im[i] * f);
+        }
+    };
+    Piece xq, xs, xg;
+    Four row[4];  // query: dY of step `own`; key: dW of step 16 (3 - w) + l16, then of `own`
+    const auto rows_of = [&](Four (&x)[4], const float *src, int step) {  // rows of a [plane][step][64] record
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const floatx4 re = *reinterpret_cast<const floatx4 *>(src + step * D + 16 * k + 4 * g);
+            const floatx4 im = *reinterpret_cast<const floatx4 *>(src + D * D + step * D + 16 * k + 4 * g);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[k].re[r] = re[r], x[k].im[r] = im[r];
+        }
+    };
+    {
+        Piece xu, xk;
+        load(xu, rec + WS_U, rec + WS_U + D * D, D, CH);
+        if (qside) {
+            const float f = own < valid ? 1.f : 0.f;
+            const int64_t o = b * bw.dy.s0 + h * bw.dy.s1 + (int64_t)(t0 + min(own, valid - 1)) * bw.dy.s2 + 4 * g;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const floatx4 re = *reinterpret_cast<const floatx4 *>(static_cast<const float *>(bw.dy.re) + o + 16 * k);
+                const floatx4 im = *reinterpret_cast<const floatx4 *>(static_cast<const float *>(bw.dy.im) + o + 16 * k);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) row[k].re[r] = re[r] * f, row[k].im[r] = im[r] * f;
+            }
+        } else {
+            rows_of(row, brec + BW_W, 16 * (3 - w) + l16);
+        }
+        view(xk, a.k);
+        view(xq, a.q);
+        if (wv == 0) {
+            sL[lane] = rec[WS_L + lane];
+            const float bt = a.beta[b * a.sg_b + h * a.sg_h + (int64_t)(t0 + min(lane, valid - 1)) * a.sg_t];
+            sBt[lane] = lane < valid ? bt : 0.f;
+        }
+        put(sU, xu, 1.f, CH);
+        put(sK, xk, 1.f, valid);
     }
     __syncthreads();
-    {  // Re<S, G>: this thread's 8 elements, summed per wave
+    load(xs, rec + WS_S, rec + WS_S + D * D, D, CH);
+    load(xg, brec + BW_G, brec + BW_G + D * D, D, CH);
+
+    {  // ---- scores of tile tt: acc[t = 16 tt + 4 g + r][s = 16 st + l16] = sum_i A[t][i] conj(U[s][i])
+        const int tt = qside ? w : 3 - w;
+        float2 *dst = qside ? sP : sH;
+        const float *src = rec + (qside ? WS_AA : WS_GA);  // Ahat or D.Gk
+        float rowacc[4], db2[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) rowacc[r] = db2[r] = 0.f;
+#pragma unroll 1
+        for (int st = 0; st <= tt; ++st) {
+            const int s = 16 * st + l16;
+            const floatx4 xr4 = *reinterpret_cast<const floatx4 *>(src + blk(tt, st) * BLK + lane * 4);
+            const floatx4 xi4 = *reinterpret_cast<const floatx4 *>(src + blk(tt, st) * BLK + lane * 4 + 256);
+            Gauss x;
+            gz(x);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const Four u = row4(sU, s, 16 * k + 4 * g);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) gstep(x, row[k].re[r], row[k].im[r], u.re[r], -u.im[r]);
+            }
+            const floatx4 dr = gre(x), di = gim(x);
+            const float Ls = sL[s];
+            float cs = 0.f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int t = 16 * tt + 4 * g + r;
+                const bool keep = qside ? (s <= t) : (s < t);
+                const float lx = sL[t] - Ls;
+                const float Dv = keep ? __expf(fminf(lx, 0.f)) : 0.f;
+                const float through = lx <= 0.f ? 1.f : 0.f;  // D's clamp: no gradient to L past it
+                const float re = xr4[r] * dr[r] + xi4[r] * di[r];
+                float f, e;
+                if (qside) {  // dP = D dAhat; E = Re(conj(Ahat) dAhat)
+                    f = Dv;
+                    e = through * re;
+                } else {  // dM = -acc; dGk = beta D dM; E = beta Re(conj(D.Gk) dM)
+                    const float bt = sBt[t];
+                    f = -bt * Dv;
+                    e = through * bt * -re;
+                    db2[r] -= re;
+                }
+                dst[t * CP + s] = make_float2(f * dr[r], f * di[r]);
+                rowacc[r] += e;
+                cs += e;
+            }
+            cs += __shfl_xor(cs, 16);
+            cs += __shfl_xor(cs, 32);
+            if (g == 0) sCol[((qside ? 0 : 4) + tt) * CH + s] = cs;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float v = row16_sum(rowacc[r]), vb = row16_sum(db2[r]);
+            if (l16 == 0) {
+                sRow[(qside ? 0 : CH) + 16 * tt + 4 * g + r] = v;
+                if (!qside) sDb2[16 * tt + 4 * g + r] = vb;
+            }
+        }
+    }
+    __syncthreads();  // U is read, dP and dGk are there
+    put(sQ, xq, a.q_scale, valid);
+    {  // Re<S, G>: this thread's elements, summed per wave
         float part = 0.f;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int e = tid + 512 * k, row = e >> 6, col = e & 63;
-            part += sS[row * KP + col] * sG[row * KP + col] + sS[PL + row * KP + col] * sG[PL + row * KP + col];
-        }
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part += xs.re[i][r] * xg.re[i][r] + xs.im[i][r] * xg.im[i][r];
         part = wave_sum(part);
         if (lane == 0) sRed[wv] = part;
     }
+    __syncthreads();
 
-    floatx4 xkr[4], xki[4];  // the query side's part of dk, [column tile]
+    Gauss acc[4];
+    floatx4 xr[4], xi[4];  // query: dq~ of step `own`; key: dk
+    floatx4 vr[4], vi[4];  // key: the v row of step `own`
+    // acc^T[j][own] += sum_s K[s][j] m[own][s], s-tiles up to the lane's own
+    const auto times_k = [&](const float2 *m) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) gz(acc[k]);
+#pragma unroll 1
+        for (int st = 0; st <= w; ++st) {
+            const Four u = row4(m, own, 16 * st + 4 * g);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int jt = 0; jt < 4; ++jt) {
+                    const float2 e = sK[(16 * st + 4 * g + r) * CP + 16 * jt + l16];
+                    gstep(acc[jt], e.x, e.y, u.re[r], u.im[r]);
+                }
+        }
+    };
+    times_k(qside ? sP : sH);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) xr[k] = gre(acc[k]), xi[k] = gim(acc[k]);
+    if (!qside) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) gz(acc[k]);
+#pragma unroll 1
+        for (int tt = w; tt < 4; ++tt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int t = 16 * tt + 4 * g + r;
+                const float2 p = sP[t * CP + own], m = sH[t * CP + own];
+#pragma unroll
+                for (int jt = 0; jt < 4; ++jt) {
+                    const float2 q = sQ[t * CP + 16 * jt + l16], k = sK[t * CP + 16 * jt + l16];
+                    gstep(acc[jt], q.x, q.y, p.x, -p.y);
+                    gstep(acc[jt], k.x, k.y, m.x, -m.y);
+                }
+            }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) xr[k] += gre(acc[k]), xi[k] += gim(acc[k]);
+        rows_of(row, brec + BW_W, own);
+        const int64_t o = b * a.v.s0 + h * a.v.s1 + (int64_t)(t0 + min(own, valid - 1)) * a.v.s2 + 4 * g;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            vr[k] = *reinterpret_cast<const floatx4 *>(static_cast<const float *>(a.v.re) + o + 16 * k);
+            vi[k] = *reinterpret_cast<const floatx4 *>(static_cast<const float *>(a.v.im) + o + 16 * k);
+        }
+    }
+    __syncthreads();  // dP and dGk are read
+    put(sS, xs, 1.f, CH);
+    put(sG, xg, 1.f, CH);
+    __syncthreads();
+
+    // acc^T[j][own] = sum_i conj(A[i][j]) x[i]
+    const auto columns = [&](const float2 *A, const Four (&x)[4]) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) gz(acc[k]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int jt = 0; jt < 4; ++jt) {
+                    const float2 e = A[(16 * k + 4 * g + r) * CP + 16 * jt + l16];
+                    gstep(acc[jt], e.x, -e.y, x[k].re[r], x[k].im[r]);
+                }
+    };
+    // xr + i xi += f acc; returns Re sum_j conj(m[own][j]) acc[j]
+    const auto fold = [&](const float2 *m, float f) {
+        float dot = 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const floatx4 ur = gre(acc[k]), ui = gim(acc[k]);
+            const Four q = row4(m, own, 16 * k + 4 * g);
+            xr[k] += f * ur;
+            xi[k] += f * ui;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) dot += q.re[r] * ur[r] + q.im[r] * ui[r];
+        }
+        dot += __shfl_xor(dot, 16);
+        dot += __shfl_xor(dot, 32);
+        return dot;
+    };
+    const auto store = [&](const qpam_mview &v, float f) {
+        const int64_t o = b * v.s0 + h * v.s1 + (int64_t)(t0 + own) * v.s2 + 4 * g;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            *reinterpret_cast<floatx4 *>(v.re + o + 16 * k) = xr[k] * f;
+            *reinterpret_cast<floatx4 *>(v.im + o + 16 * k) = xi[k] * f;
+        }
+    };
+    const float al = __expf(sL[own]), bt = sBt[own];
     if (qside) {
-        const int t = 16 * w + l16;  // this lane's step
-        const float al = __expf(sL[t]), bt = sBt[t];
-        const float *opbase;
-        floatx4 orr[4], oi[4], pr[4], pi[4];
-        {  // dY rows (zero past the end) and the dP blocks (w, st <= w) in x_Q layout
-            const float f = t < valid ? 1.f : 0.f;
-            const int64_t o = b * bw.dy.s0 + h * bw.dy.s1 + (int64_t)(t0 + min(t, valid - 1)) * bw.dy.s2 + 4 * g;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                orr[q] = *reinterpret_cast<const floatx4 *>(static_cast<const float *>(bw.dy.re) + o + 16 * q) * f;
-                oi[q] = *reinterpret_cast<const floatx4 *>(static_cast<const float *>(bw.dy.im) + o + 16 * q) * f;
-            }
-#pragma unroll
-            for (int st = 0; st < 4; ++st) {
-                if (st > w) continue;
-                opbase = brec + BW_PQ + blk(w, st) * BLK + lane * 4;
-                pr[st] = *reinterpret_cast<const floatx4 *>(opbase);
-                pi[st] = *reinterpret_cast<const floatx4 *>(opbase + 256);
-            }
-        }
-        float dal = 0.f;
-        float *dqr = bw.dq.re + b * bw.dq.s0 + h * bw.dq.s1 + (int64_t)(t0 + t) * bw.dq.s2;
-        float *dqi = bw.dq.im + b * bw.dq.s0 + h * bw.dq.s1 + (int64_t)(t0 + t) * bw.dq.s2;
-#pragma unroll 1  // (unrolled, the compiler keeps every column tile's operands live and spills)
-        for (int jt = 0; jt < 4; ++jt) {
-            const int j = 16 * jt + l16;
-            // sum_s K[s][j] dP[t][s]  (k = s = 16 st + 4 g + r)
-            Gauss x;
-            gz(x);
-#pragma unroll
-            for (int st = 0; st < 4; ++st) {
-                if (st > w) continue;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int s = 16 * st + 4 * g + r;
-                    gstep(x, sK[s * KP + j], sK[PL + s * KP + j], pr[st][r], pi[st][r]);
-                }
-            }
-            // YS^T[j][t] = sum_i conj(S[i][j]) dY[t][i]  (k = i = 16 q + 4 g + r)
-            Gauss y;
-            gz(y);
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int i = 16 * q + 4 * g + r;
-                    gstep(y, sS[i * KP + j], -sS[PL + i * KP + j], orr[q][r], oi[q][r]);
-                }
-            const floatx4 ysr = gre(y), ysi = gim(y);
-            const floatx4 qr4 = *reinterpret_cast<const floatx4 *>(sQ + t * KP + 16 * jt + 4 * g);
-            const floatx4 qi4 = *reinterpret_cast<const floatx4 *>(sQ + PL + t * KP + 16 * jt + 4 * g);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) dal += qr4[r] * ysr[r] + qi4[r] * ysi[r];
-            if (t < valid) {
-                *reinterpret_cast<floatx4 *>(dqr + 16 * jt + 4 * g) = (gre(x) + al * ysr) * a.q_scale;
-                *reinterpret_cast<floatx4 *>(dqi + 16 * jt + 4 * g) = (gim(x) + al * ysi) * a.q_scale;
-            }
-        }
-        {  // dW rows and the dGk blocks (w, st <= w) in x_Q layout
-            const float *dw = brec + BW_W + t * D + 4 * g;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                orr[q] = *reinterpret_cast<const floatx4 *>(dw + 16 * q);
-                oi[q] = *reinterpret_cast<const floatx4 *>(dw + D * D + 16 * q);
-            }
-#pragma unroll
-            for (int st = 0; st < 4; ++st) {
-                if (st > w) continue;
-                opbase = brec + BW_GQ + blk(w, st) * BLK + lane * 4;
-                pr[st] = *reinterpret_cast<const floatx4 *>(opbase);
-                pi[st] = *reinterpret_cast<const floatx4 *>(opbase + 256);
-            }
-        }
-        float dk2 = 0.f;
-#pragma unroll
-        for (int jt = 0; jt < 4; ++jt) {
-            const int j = 16 * jt + l16;
-            Gauss x;  // sum_s K[s][j] dGk[t][s]
-            gz(x);
-#pragma unroll
-            for (int st = 0; st < 4; ++st) {
-                if (st > w) continue;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int s = 16 * st + 4 * g + r;
-                    gstep(x, sK[s * KP + j], sK[PL + s * KP + j], pr[st][r], pi[st][r]);
-                }
-            }
-            Gauss y;  // WS^T[j][t] = sum_i conj(S[i][j]) dW[t][i]
-            gz(y);
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int i = 16 * q + 4 * g + r;
-                    gstep(y, sS[i * KP + j], -sS[PL + i * KP + j], orr[q][r], oi[q][r]);
-                }
-            const floatx4 wsr = gre(y), wsi = gim(y);
-            const floatx4 kr4 = *reinterpret_cast<const floatx4 *>(sK + t * KP + 16 * jt + 4 * g);
-            const floatx4 ki4 = *reinterpret_cast<const floatx4 *>(sK + PL + t * KP + 16 * jt + 4 * g);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) dk2 += kr4[r] * wsr[r] + ki4[r] * wsi[r];
-            xkr[jt] = gre(x) - (al * bt) * wsr;
-            xki[jt] = gim(x) - (al * bt) * wsi;
-        }
+        columns(sS, row);
+        const float dal = fold(sQ, al);
+        if (g == 0) sDa[own] = dal;
+        if (own < valid) store(bw.dq, a.q_scale);
+    } else {
         float dba = 0.f;  // Re sum_i conj(v[t][i]) dW[t][i]
-        {
-            const int64_t o = b * a.v.s0 + h * a.v.s1 + (int64_t)(t0 + min(t, valid - 1)) * a.v.s2 + 4 * g;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const floatx4 vr4 = *reinterpret_cast<const floatx4 *>(static_cast<const float *>(a.v.re) + o + 16 * q);
-                const floatx4 vi4 = *reinterpret_cast<const floatx4 *>(static_cast<const float *>(a.v.im) + o + 16 * q);
+        for (int k = 0; k < 4; ++k)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) dba += vr4[r] * orr[q][r] + vi4[r] * oi[q][r];
-            }
-        }
-        dal += __shfl_xor(dal, 16);
-        dal += __shfl_xor(dal, 32);
-        dk2 += __shfl_xor(dk2, 16);
-        dk2 += __shfl_xor(dk2, 32);
+            for (int r = 0; r < 4; ++r) dba += vr[k][r] * row[k].re[r] + vi[k][r] * row[k].im[r];
         dba += __shfl_xor(dba, 16);
         dba += __shfl_xor(dba, 32);
+        Four u[4];
+        rows_of(u, rec + WS_U, own);
+        columns(sS, row);
+        const float dk2 = fold(sK, -(al * bt));
+        columns(sG, u);
+        const float ddl = fold(sK, write_weight(a, sL[own], sL[CH - 1]));  // the state-write weight
         if (g == 0) {
-            sDa[t] = dal - bt * dk2;
-            sDb[t] = dba - al * dk2;
+            sDb[own] = dba - al * dk2;
+            sDdl[own] = ddl;
+            sDk[own] = bt * dk2;
         }
-    } else {
-        const int s = 16 * w + l16;  // this lane's step (key side)
-        const float dl = write_weight(a, sL[s], sL[CH - 1]);  // the state-write weight
-        float *dkr = bw.dk.re + b * bw.dk.s0 + h * bw.dk.s1 + (int64_t)(t0 + s) * bw.dk.s2;
-        float *dki = bw.dk.im + b * bw.dk.s0 + h * bw.dk.s1 + (int64_t)(t0 + s) * bw.dk.s2;
-        floatx4 urr[4], ui[4], pr[4], pi[4], hr[4], hi[4];
-        {  // U rows; dP, dGk blocks (tt >= w, w) in x_K layout
-            const float *du = rec + WS_U + s * D + 4 * g;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                urr[q] = *reinterpret_cast<const floatx4 *>(du + 16 * q);
-                ui[q] = *reinterpret_cast<const floatx4 *>(du + D * D + 16 * q);
-            }
-#pragma unroll
-            for (int tt = 0; tt < 4; ++tt) {
-                if (tt < w) continue;
-                const float *p = brec + BW_PK + blk(tt, w) * BLK + lane * 4;
-                const float *q = brec + BW_GK + blk(tt, w) * BLK + lane * 4;
-                pr[tt] = *reinterpret_cast<const floatx4 *>(p);
-                pi[tt] = *reinterpret_cast<const floatx4 *>(p + 256);
-                hr[tt] = *reinterpret_cast<const floatx4 *>(q);
-                hi[tt] = *reinterpret_cast<const floatx4 *>(q + 256);
-            }
-        }
-        float ddl = 0.f;
-#pragma unroll 1  // (unrolled, the compiler keeps every column tile's operands live and spills)
-        for (int jt = 0; jt < 4; ++jt) {
-            const int j = 16 * jt + l16;
-            // sum_t q~[t][j] conj(dP[t][s]) + K[t][j] conj(dGk[t][s])  (k = t = 16 tt + 4 g + r)
-            Gauss x;
-            gz(x);
-#pragma unroll
-            for (int tt = 0; tt < 4; ++tt) {
-                if (tt < w) continue;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int t = 16 * tt + 4 * g + r;
-                    gstep(x, sQ[t * KP + j], sQ[PL + t * KP + j], pr[tt][r], -pi[tt][r]);
-                    gstep(x, sK[t * KP + j], sK[PL + t * KP + j], hr[tt][r], -hi[tt][r]);
-                }
-            }
-            // UG^T[j][s] = sum_i conj(G[i][j]) U[s][i]
-            Gauss y;
-            gz(y);
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int i = 16 * q + 4 * g + r;
-                    gstep(y, sG[i * KP + j], -sG[PL + i * KP + j], urr[q][r], ui[q][r]);
-                }
-            const floatx4 ugr = gre(y), ugi = gim(y);
-            const floatx4 kr4 = *reinterpret_cast<const floatx4 *>(sK + s * KP + 16 * jt + 4 * g);
-            const floatx4 ki4 = *reinterpret_cast<const floatx4 *>(sK + PL + s * KP + 16 * jt + 4 * g);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) ddl += kr4[r] * ugr[r] + ki4[r] * ugi[r];
-            if (s < valid) {  // the key side's part of dk; the query side adds its part below
-                *reinterpret_cast<floatx4 *>(dkr + 16 * jt + 4 * g) = gre(x) + dl * ugr;
-                *reinterpret_cast<floatx4 *>(dki + 16 * jt + 4 * g) = gim(x) + dl * ugi;
-            }
-        }
-        ddl += __shfl_xor(ddl, 16);
-        ddl += __shfl_xor(ddl, 32);
-        if (g == 0) sDdl[s] = ddl;
+        if (own < valid) store(bw.dk, 1.f);
     }
-    __syncthreads();  // the key side's dk rows are written (and visible to the block)
-    if (qside) {
-        const int t = 16 * w + l16;
-        if (t < valid) {
-            float *dkr = bw.dk.re + b * bw.dk.s0 + h * bw.dk.s1 + (int64_t)(t0 + t) * bw.dk.s2 + 4 * g;
-            float *dki = bw.dk.im + b * bw.dk.s0 + h * bw.dk.s1 + (int64_t)(t0 + t) * bw.dk.s2 + 4 * g;
-#pragma unroll
-            for (int jt = 0; jt < 4; ++jt) {
-                *reinterpret_cast<floatx4 *>(dkr + 16 * jt) += xkr[jt];
-                *reinterpret_cast<floatx4 *>(dki + 16 * jt) += xki[jt];
-            }
-        }
-    }
-    if (wv == 4) {  // lane = step: dL, its reverse cumsum, dgamma and dbeta
+    __syncthreads();
+    if (wv == 0) {  // lane = step: dL, its reverse cumsum, dgamma and dbeta
         const int t = lane;
         const float Lt = sL[t], Llast = sL[CH - 1];
-        const float al = __expf(Lt), atot = __expf(Llast), dl = write_weight(a, Lt, Llast);
+        const float alt = __expf(Lt), atot = __expf(Llast), dl = write_weight(a, Lt, Llast);
         const bool tv = t < valid;
-        float x = tv ? sLp[t] + sDa[t] * al - sDdl[t] * dl * write_weight_dl(a, Lt) : 0.f;
+        float col = 0.f;
+        for (int tt = t >> 4; tt < 4; ++tt) col += sCol[tt * CH + t];
+        for (int tt = t >> 4; tt < 4; ++tt) col += sCol[(4 + tt) * CH + t];
+        const float lp = sRow[t] + sRow[CH + t] - col;
+        float x = tv ? lp + (sDa[t] - sDk[t]) * alt - sDdl[t] * dl * write_weight_dl(a, Lt) : 0.f;
         const float tot = wave_sum(tv ? sDdl[t] * dl : 0.f);
         float dac = 0.f;
 #pragma unroll
@@ -1381,9 +1247,6 @@ extern "C" int qpam_delta_bwd(const qpam_delta_bwd_args *g, void *stream) {
     hipLaunchKernelGGL(delta_bwd_chain_kernel, dim3((unsigned)(a.B * a.H * ROW_BLOCKS)), dim3(256), 0, s, *g, a,
                        n_chunks);
     st = launch_status("delta_bwd_chain_kernel");
-    if (st) return st;
-    hipLaunchKernelGGL(delta_bwd_score_kernel, dim3((unsigned)items), dim3(256), 0, s, *g, a, n_chunks);
-    st = launch_status("delta_bwd_score_kernel");
     if (st) return st;
     QPAM_CHECK_HIP(hipFuncSetAttribute((const void *)delta_bwd_grad_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)G2_SMEM));
