@@ -217,6 +217,8 @@ int qpam_decode_step_bwd(const qpam_decode_bwd_args *a, void *stream);
  * gamma: fp32 [M,B,H,T]; rot (r_m, optional, NULL = 1): planar fp32 [M,B,H,T].
  * s0: optional initial state, planar fp32 [M,B,H,d,d] contiguous.
  * y: planar fp32 (or bf16, y_dtype) [B,H,T,d]; s_out: final state planar fp32 [M,B,H,d,d].
+ * With fp32 inputs y may also be one split-real [B,H,T,d,2] tensor: im = re + 1, strides
+ * in floats and even, 8-byte aligned.
  * The workspace keeps the state entering every chunk, planar fp32
  * [M,B,H,n_chunks,d,d]; qpam_scan_bwd reads it.  d == 64, C in {16,32,64}.
  */
@@ -283,7 +285,10 @@ int qpam_scan_fwd_noalloc(const qpam_scan_args *a, void *stream);
  * ds0 (optional) planar fp32 [M,B,H,d,d].  bwd_workspace holds per-chunk
  * state gradients, size from qpam_scan_bwd_workspace_size.  With bf16 q/k/v
  * and C == 64, dq/dk/dv planes must be 8-byte aligned with strides that are
- * multiples of 4 elements (their rows are stored in 8-byte runs). */
+ * multiples of 4 elements (their rows are stored in 8-byte runs).  With fp32
+ * q/k/v and C == 64, each of dy, dq, dk and dv may also be one split-real
+ * [B,H,T,d,2] tensor (im = re + 1, strides in floats, multiples of 4) if every
+ * gradient row starts on 16 bytes. */
 typedef struct {
     const qpam_scan_args *fwd;
     qpam_cview dy;

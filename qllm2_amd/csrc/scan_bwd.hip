@@ -206,7 +206,16 @@ __global__ void __launch_bounds__(THREADS) grad_chunk_state_kernel(BwdParams p) 
     }
     const int64_t go = b * p.dy.s0 + h * p.dy.s1 + (int64_t)c0 * p.dy.s2;
     const int64_t qo = b * a.q.s0 + h * a.q.s1 + (int64_t)c0 * a.q.s2;
-    {
+    if (std::is_same<Tin, float>::value && pairs(p.dy)) {
+        F32Tile<C> qr, qi, yr, yi;
+        tile_load<C>(qr, (const float *)a.q.re + qo, a.q.s2, valid);
+        tile_load<C>(qi, (const float *)a.q.im + qo, a.q.s2, valid);
+        tile_load_pairs<C>(yr, yi, (const float *)p.dy.re + go, p.dy.s2, valid);
+        tile_store<C>(sQr, qr, a.q_scale);
+        tile_store<C>(sQi, qi, a.q_scale);
+        tile_store<C>(sGr, yr, 1.f);
+        tile_store<C>(sGi, yi, 1.f);
+    } else {
         float *const gd[2] = {sGr, sGi};
         const float *const gs[2] = {(const float *)p.dy.re + go, (const float *)p.dy.im + go};
         float *const id[2] = {sQr, sQi};
@@ -864,7 +873,8 @@ __global__ void __launch_bounds__(THREADS) key_side_kernel(BwdParams p) {
 // 0.92 of the two kernels', the worst output of every case no larger.  Bound by the matrix
 // cores (60 us at full rate for 768 chunks) and the causal steps' decay arithmetic between
 // them.  Against the query and key sides as kernels of four waves, each staging all four
-// tiles and using four-product MFMAs: B=4, H=12, T=1000, M=1: 115 + 129 -> 133 us.
+// tiles and using four-product MFMAs: B=4, H=12, T=1000, M=1: 115 + 129 -> 133 us
+// (139 us with split-real dy, dq, dk and dv).
 constexpr int CGF_THREADS = 512;
 template <int M>
 constexpr size_t cgf_smem() { return 4 * TILE * sizeof(float2) + (11 * M * 64 + 8 * M) * sizeof(float); }
@@ -920,7 +930,18 @@ __global__ void __launch_bounds__(CGF_THREADS, 2) chunk_grad_f32_kernel(BwdParam
         view(xq, a.q);
         view(xk, a.k);
         view(xv, a.v);
-        view(xy, p.dy);
+        if (pairs(p.dy)) {
+            const float *src = static_cast<const float *>(p.dy.re) + b * p.dy.s0 + h * p.dy.s1 + (int64_t)c0 * p.dy.s2;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const float4 *s4 = reinterpret_cast<const float4 *>(src + min(sr + 32 * i, valid - 1) * p.dy.s2 + 2 * sc);
+                const float4 u = s4[0], v = s4[1];
+                xy.re[i] = make_float4(u.x, u.z, v.x, v.z);
+                xy.im[i] = make_float4(u.y, u.w, v.y, v.w);
+            }
+        } else {
+            view(xy, p.dy);
+        }
         if (wv < M) {
             const float *gp = a.gamma + wv * a.sg_m + b * a.sg_b + h * a.sg_h + (int64_t)c0 * a.sg_t;
             gam = gp[(int64_t)min(lane, valid - 1) * a.sg_t];
@@ -1167,7 +1188,17 @@ __global__ void __launch_bounds__(CGF_THREADS, 2) chunk_grad_f32_kernel(BwdParam
         }
     }
     const auto store = [&](const qpam_mview &v, const floatx4 (&re)[4], const floatx4 (&im)[4], float f) {
-        const int64_t o = b * v.s0 + h * v.s1 + (int64_t)(c0 + own) * v.s2 + 4 * g;
+        const int64_t row = b * v.s0 + h * v.s1 + (int64_t)(c0 + own) * v.s2, o = row + 4 * g;
+        if (pairs(v)) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const floatx4 x = re[k] * f, y = im[k] * f;
+                float4 *dst = reinterpret_cast<float4 *>(v.re + row + 2 * (16 * k + 4 * g));
+                dst[0] = make_float4(x[0], y[0], x[1], y[1]);
+                dst[1] = make_float4(x[2], y[2], x[3], y[3]);
+            }
+            return;
+        }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             *reinterpret_cast<floatx4 *>(v.re + o + 16 * k) = re[k] * f;
@@ -2174,7 +2205,11 @@ int launch_chunk_grad_f32(const BwdParams &p, hipStream_t stream) {
 // chunk_grad_f32 stores gradient rows in 16-byte runs; other output layouts keep
 // the query and key sides as kernels of their own
 bool rows16(const qpam_mview &v) {
-    return (((uintptr_t)v.re | (uintptr_t)v.im) % 16) == 0 && v.s0 % 4 == 0 && v.s1 % 4 == 0 && v.s2 % 4 == 0;
+    return ((uintptr_t)v.re % 16) == 0 && (pairs(v) || ((uintptr_t)v.im % 16) == 0) && v.s0 % 4 == 0 && v.s1 % 4 == 0 &&
+           v.s2 % 4 == 0;
+}
+bool fused_f32(const qpam_scan_args &a, const qpam_mview &dq, const qpam_mview &dk, const qpam_mview &dv) {
+    return a.dtype == QPAM_F32 && a.C == 64 && rows16(dq) && rows16(dk) && rows16(dv);
 }
 
 template <typename Tin, int C>
@@ -2182,7 +2217,7 @@ int launch_bwd(const BwdParams &p, hipStream_t stream) {
     const qpam_scan_args &a = p.a;
     dim3 grid(p.n_chunks, a.H, a.B);
     if constexpr (std::is_same<Tin, float>::value && C == 64) {
-        if (rows16(p.dq) && rows16(p.dk) && rows16(p.dv)) {
+        if (fused_f32(a, p.dq, p.dk, p.dv)) {
             const size_t s1 = gcs_smem<C>();
             QPAM_CHECK_HIP(hipFuncSetAttribute((const void *)grad_chunk_state_kernel<Tin, C>,
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)s1));
@@ -2257,9 +2292,13 @@ int scan_bwd(const qpam_scan_bwd_args *bw, hipStream_t stream) {
     const qpam_scan_args *a = bw->fwd;
     int st = validate_scan(a, "qpam_scan_bwd", false);
     if (st) return st;
-    QPAM_REQUIRE(bw->dy.re && bw->dy.im && ((uintptr_t)bw->dy.re % 16) == 0 && ((uintptr_t)bw->dy.im % 16) == 0 &&
-                     bw->dy.s0 % 4 == 0 && bw->dy.s1 % 4 == 0 && bw->dy.s2 % 4 == 0,
+    const bool fused = fused_f32(*a, bw->dq, bw->dk, bw->dv);  // the kernels that read and write interleaved rows
+    QPAM_REQUIRE(bw->dy.re && bw->dy.im && ((uintptr_t)bw->dy.re % 16) == 0 &&
+                     (((uintptr_t)bw->dy.im % 16) == 0 || (fused && pairs(bw->dy))) && bw->dy.s0 % 4 == 0 &&
+                     bw->dy.s1 % 4 == 0 && bw->dy.s2 % 4 == 0,
                  "qpam_scan_bwd: dy must be 16-byte aligned fp32 planes with strides multiple of 4");
+    QPAM_REQUIRE(fused || !(pairs(bw->dq) || pairs(bw->dk) || pairs(bw->dv)),
+                 "qpam_scan_bwd: interleaved gradients need fp32 inputs, 64-step chunks and 16-byte rows");
     QPAM_REQUIRE(bw->dy_dtype == QPAM_F32 ||
                      (bw->dy_dtype == QPAM_BF16 && a->dtype == QPAM_BF16 && a->C == 64 && bw->dy.s0 % 8 == 0 &&
                       bw->dy.s1 % 8 == 0 && bw->dy.s2 % 8 == 0),

@@ -385,15 +385,21 @@ __global__ void __launch_bounds__(THREADS, 2) chunk_output_f32_kernel(FwdParams 
         }
     }
 
+    const bool ypairs = pairs(a.y);
     const int64_t yo = b * a.y.s0 + h * a.y.s1 + (int64_t)c0 * a.y.s2;
 #pragma unroll
     for (int it = 0; it < 4; ++it)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int tr = 16 * tt + 4 * g + r;
-            if (tr < valid) {
-                a.y.re[yo + (int64_t)tr * a.y.s2 + 16 * it + l16] = y1[it][r] - y2[it][r];
-                a.y.im[yo + (int64_t)tr * a.y.s2 + 16 * it + l16] = y3[it][r] - y1[it][r] - y2[it][r];
+            if (tr >= valid) continue;
+            const float re = y1[it][r] - y2[it][r], im = y3[it][r] - y1[it][r] - y2[it][r];
+            float *y = a.y.re + yo + (int64_t)tr * a.y.s2;
+            if (ypairs) {
+                reinterpret_cast<float2 *>(y)[16 * it + l16] = make_float2(re, im);
+            } else {
+                y[16 * it + l16] = re;
+                a.y.im[yo + (int64_t)tr * a.y.s2 + 16 * it + l16] = im;
             }
         }
 }
@@ -1477,6 +1483,10 @@ int validate_scan(const qpam_scan_args *a, const char *who, bool fwd_outputs) {
     QPAM_REQUIRE((a->s0_re == nullptr) == (a->s0_im == nullptr), "%s: s0 needs both planes", who);
     QPAM_REQUIRE((a->s_re == nullptr) == (a->s_im == nullptr), "%s: s_out needs both planes", who);
     QPAM_REQUIRE(!fwd_outputs || (a->y.re && a->y.im), "%s: null y", who);
+    QPAM_REQUIRE(!fwd_outputs || !pairs(a->y) ||
+                     (a->dtype == QPAM_F32 && ((uintptr_t)a->y.re % 8) == 0 && a->y.s0 % 2 == 0 && a->y.s1 % 2 == 0 &&
+                      a->y.s2 % 2 == 0),
+                 "%s: interleaved y needs fp32 inputs, 8-byte aligned rows and even strides", who);
     QPAM_REQUIRE(a->y_dtype == QPAM_F32 || (a->y_dtype == QPAM_BF16 && a->dtype == QPAM_BF16 && a->C == 64),
                  "%s: y_dtype %d (bf16 y needs bf16 inputs and chunk 64)", who, a->y_dtype);
     const uintptr_t al = (uintptr_t)a->s0_re | (uintptr_t)a->s0_im | (uintptr_t)a->s_re | (uintptr_t)a->s_im;

@@ -75,6 +75,11 @@ def _mview(re, im):
     return _lib.MView(re.data_ptr(), im.data_ptr(), *re.stride()[:3])
 
 
+def _mview_pairs(x):
+    """x [B,H,T,d,2] fp32 with complex rows of unit stride, im one float after re."""
+    return _lib.MView(x.data_ptr(), x.data_ptr() + 4, *x.stride()[:3])
+
+
 def _fill_args(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, s0_im, q_scale, chunk):
     M, B, H, T = gamma.shape
     q, qr, qi = _cview(_aligned_plane(q_re), _aligned_plane(q_im))
@@ -124,6 +129,9 @@ def _validate(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, 
             raise ValueError("s0 planes must be fp32 [M, B, H, 64, 64]")
 
 
+PAIRS = 4  # y_layout inside the split-real ops: y one [B,H,T,64,2] tensor, fp32
+
+
 @op("qpam::scan_fwd")
 def scan_fwd_op(q_re: Tensor, q_im: Tensor, k_re: Tensor, k_im: Tensor, v_re: Tensor, v_im: Tensor,
                 gamma: Tensor, rot_re: Optional[Tensor], rot_im: Optional[Tensor], s0_re: Optional[Tensor],
@@ -148,6 +156,10 @@ def _scan_fwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, 
         y_im = y_re.new_empty(0)
         a.y = _mview(y_re[:, :, 0].transpose(1, 2), y_re[:, :, 1].transpose(1, 2))
         a.y_dtype = 1 if y_layout == 3 else 0
+    elif y_layout == PAIRS:
+        y_re = torch.empty(B, H, T, d, 2, device=dev, dtype=torch.float32)
+        y_im = y_re.new_empty(0)
+        a.y = _mview_pairs(y_re)
     else:
         y_re = torch.empty((B, T, H, d) if y_layout == 1 else (B, H, T, d), device=dev, dtype=torch.float32)
         y_im = torch.empty_like(y_re)
@@ -231,18 +243,25 @@ def _scan_bwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, 
         dy = dy_re.contiguous()
         bw.dy_dtype = 1 if y_layout == 3 else 0
         dy_re, dy_im = dy[:, :, 0].transpose(1, 2), dy[:, :, 1].transpose(1, 2)
-    else:
+    elif dy_im is not None:
         dy_re, dy_im = dy_re.contiguous(), dy_im.contiguous()
         if y_layout == 1:
             dy_re, dy_im = dy_re.transpose(1, 2), dy_im.transpose(1, 2)
-    bw.dy, _, _ = _cview(dy_re, dy_im)
+    if dy_im is None:  # one [B,H,T,d,2] gradient (layout PAIRS)
+        bw.dy = _lib.CView(dy_re.data_ptr(), dy_re.data_ptr() + 4, *dy_re.stride()[:3])
+    else:
+        bw.dy, _, _ = _cview(dy_re, dy_im)
     if ds_re is not None:
         ds_re, ds_im = ds_re.contiguous(), ds_im.contiguous()
         bw.ds_re, bw.ds_im = ds_re.data_ptr(), ds_im.data_ptr()
-    outs = [torch.empty(B, H, T, d, device=dev, dtype=q_re.dtype) for _ in range(6)]
-    bw.dq = _mview(outs[0], outs[1])
-    bw.dk = _mview(outs[2], outs[3])
-    bw.dv = _mview(outs[4], outs[5])
+    if y_layout == PAIRS:
+        outs = [torch.empty(B, H, T, d, 2, device=dev, dtype=torch.float32) for _ in range(3)]
+        bw.dq, bw.dk, bw.dv = (_mview_pairs(x) for x in outs)
+    else:
+        outs = [torch.empty(B, H, T, d, device=dev, dtype=q_re.dtype) for _ in range(6)]
+        bw.dq = _mview(outs[0], outs[1])
+        bw.dk = _mview(outs[2], outs[3])
+        bw.dv = _mview(outs[4], outs[5])
     dgamma = torch.empty(M, B, H, T, device=dev, dtype=torch.float32)
     bw.dgamma = dgamma.data_ptr()
     if rot_re is not None:
@@ -457,6 +476,18 @@ def _scan_blocks(q_re, q_im, k_re, k_im, v_re, v_im, gamma, q_scale, chunk, rot,
 
 # ---------------------------------------------------------------- split-real front end
 
+def _writes_pairs(dtype, d, chunk):
+    """fp32 head dim 64 with 64-step chunks: the kernels write y and the gradients as
+    split-real rows, and read dy as such; other cases pack and unpack planes."""
+    return dtype == torch.float32 and d == planes.KD and chunk == 64
+
+
+def _reads_pairs(dy):
+    """Complex rows the kernels load in 16-byte pieces."""
+    return (dy.dtype == torch.float32 and dy.stride(-1) == 1 and dy.stride(-2) == 2 and dy.data_ptr() % 16 == 0
+            and all(s % 4 == 0 for s in dy.stride()[:3]))
+
+
 @op("qpam::scan_il_fwd")
 def scan_il_fwd_op(q: Tensor, k: Tensor, v: Tensor, gamma: Tensor, rot_re: Optional[Tensor],
                    rot_im: Optional[Tensor], q_scale: float, chunk: int) -> List[Tensor]:
@@ -465,10 +496,14 @@ def scan_il_fwd_op(q: Tensor, k: Tensor, v: Tensor, gamma: Tensor, rot_re: Optio
     [y [B,H,T,d,2], s [M,B,H,d,d,2] in q's dtype, planes [3,2,B,H,T,64],
     workspace]; the planes are what the backward reads."""
     d = q.shape[3]
+    pairs = _writes_pairs(q.dtype, d, chunk)
     pl = planes.split_rows((q, k, v), q.dtype)
     y_re, y_im, s_re, s_im, ws = _scan_fwd(pl[0, 0], pl[0, 1], pl[1, 0], pl[1, 1], pl[2, 0], pl[2, 1], gamma, rot_re,
-                                           rot_im, None, None, q_scale, chunk, 0)
-    y, s = planes.merge([(y_re, y_im)], [(s_re, s_im)], d, q.dtype)
+                                           rot_im, None, None, q_scale, chunk, PAIRS if pairs else 0)
+    if pairs:
+        y, s = y_re, planes.merge([], [(s_re, s_im)], d, q.dtype)[0]
+    else:
+        y, s = planes.merge([(y_re, y_im)], [(s_re, s_im)], d, q.dtype)
     return [y, s, pl, ws]
 
 
@@ -485,13 +520,18 @@ def _(q, k, v, gamma, rot_re, rot_im, q_scale, chunk):
 def scan_il_bwd_op(pl: Tensor, gamma: Tensor, rot_re: Optional[Tensor], rot_im: Optional[Tensor], q_scale: float,
                    chunk: int, ws: Tensor, dy: Optional[Tensor], ds: Optional[Tensor], d: int) -> List[Tensor]:
     """[dq, dk, dv [B,H,T,d,2] in the planes' dtype, dgamma, drot_re, drot_im]."""
-    if dy is not None:
-        dyp = planes.split_rows((dy,), torch.float32)[0]
-    else:
+    pairs = _writes_pairs(pl.dtype, d, chunk)
+    if dy is None:
         dyp = torch.zeros(pl.shape[1:], device=pl.device, dtype=torch.float32)
+    elif pairs and _reads_pairs(dy):
+        dyp = (dy, None)
+    else:
+        dyp = planes.split_rows((dy,), torch.float32)[0]
     dsp = planes.split_states(ds) if ds is not None else (None, None)
     g = _scan_bwd(pl[0, 0], pl[0, 1], pl[1, 0], pl[1, 1], pl[2, 0], pl[2, 1], gamma, rot_re, rot_im, None, None,
-                  q_scale, chunk, ws, dyp[0], dyp[1], dsp[0], dsp[1], 0)
+                  q_scale, chunk, ws, dyp[0], dyp[1], dsp[0], dsp[1], PAIRS if pairs else 0)
+    if pairs:
+        return g[:6]
     return planes.merge([(g[0], g[1]), (g[2], g[3]), (g[4], g[5])], [], d, pl.dtype) + [g[6], g[7], g[8]]
 
 

@@ -105,3 +105,51 @@ def test_delta_split_real_equals_planar(gpu_lib, d, T, chunk, dtype, given, how)
     want = [y, s, *_grads(y, s, leaves, dy, ds)]
     for i, (a, b) in enumerate(zip(got, want)):
         assert a.dtype == b.dtype and torch.equal(a, b), i
+
+
+@pytest.mark.parametrize("T,M,form", [
+    (1, 1, "dense"), (63, 2, "dense"), (130, 4, "dense"),
+    (70, 1, "heads_last"),   # the rows of a [B,T,H,64,2] tensor
+    (70, 2, "expanded"),     # one row for all (strides 0)
+    (70, 1, "padded"),       # rows of 65 complex elements: packed first
+    (70, 1, "offset"),       # 8-byte aligned storage: packed first
+    (70, 1, "none"),         # the state's gradient only
+])
+def test_split_real_rows_equal_planes(gpu_lib, T, M, form):
+    """fp32, head dim 64, 64-step chunks: y leaves and the gradients arrive and leave as
+    split-real rows.  The arithmetic is that of the planes, so every result is the
+    planar call's bit for bit, whatever the strides of dy."""
+    from qllm2_amd.pam_scan import pam_scan_interleaved, pam_scan_planar
+    B, H, d = 2, 3, 64
+    g = torch.Generator().manual_seed(17 * T + M)
+    qkv = [(0.3 * torch.randn(B, H, T, d, 2, generator=g)).cuda() for _ in range(3)]
+    gamma = (0.85 + 0.15 * torch.rand(M, B, H, T, generator=g)).cuda()
+    ds = torch.randn(M, B, H, d, d, 2, generator=g).cuda()
+    dy = torch.randn(B, H, T, d, 2, generator=g).cuda()
+    if form == "heads_last":
+        dy = dy.transpose(1, 2).contiguous().transpose(1, 2)
+    elif form == "expanded":
+        dy = dy[:1, :1, :1].expand(B, H, T, d, 2)
+    elif form == "padded":
+        dy = torch.nn.functional.pad(dy, (0, 0, 0, 1))[..., :d, :]
+    elif form == "offset":
+        buf = torch.empty(dy.numel() + 2, device="cuda")
+        buf[2:] = dy.reshape(-1)
+        dy = buf[2:].view(B, H, T, d, 2)
+
+    xs = [x.clone().requires_grad_(True) for x in (*qkv, gamma)]
+    y, s = pam_scan_interleaved(*xs, d, 64)
+    ps = [x[..., i].contiguous().requires_grad_(True) for x in qkv for i in (0, 1)]
+    gam = gamma.clone().requires_grad_(True)
+    y_re, y_im, s_re, s_im = pam_scan_planar(*ps, gam, q_scale=d ** -0.5, chunk=64)
+    assert torch.equal(y, torch.stack([y_re, y_im], -1)) and torch.equal(s, torch.stack([s_re, s_im], -1))
+    if form == "none":
+        got = torch.autograd.grad([s], xs, [ds])
+        ref = torch.autograd.grad([s_re, s_im], [*ps, gam], [ds[..., 0], ds[..., 1]])
+    else:
+        got = torch.autograd.grad([y, s], xs, [dy, ds])
+        ref = torch.autograd.grad([y_re, y_im, s_re, s_im], [*ps, gam],
+                                  [dy[..., 0].contiguous(), dy[..., 1].contiguous(), ds[..., 0], ds[..., 1]])
+    for i in range(3):
+        assert torch.equal(got[i], torch.stack([ref[2 * i], ref[2 * i + 1]], -1)), i
+    assert torch.equal(got[3], ref[6])
