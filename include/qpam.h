@@ -517,7 +517,8 @@ int qpam_delta_fwd(const qpam_delta_args *a, void *stream);
  * workspace still holds the per-chunk records).  dy fp32 planar [B,H,T,d]; ds
  * optional gradient of the final state.  Out: dq, dk, dv planar fp32; dgamma,
  * dbeta [B,H,T] with the strides of gamma; ds0 optional [B,H,d,d].
- * Deterministic (fixed-order reductions). */
+ * Deterministic (fixed-order reductions).  y, dy, dq, dk and dv may each be one
+ * split-real [B,H,T,d,2] tensor instead of planes: im = re + 1, strides in floats. */
 typedef struct {
     const qpam_delta_args *fwd;
     qpam_cview dy;

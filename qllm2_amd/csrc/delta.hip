@@ -59,6 +59,36 @@ constexpr int ROW_BLOCKS = 4;          // blocks per chain in the chunk pass (16
 // matrix, the state-write weight alpha_last / (alpha_s + 1e-12)) follow the
 // reference's chunk boundaries.
 __host__ __device__ __forceinline__ int chunk_len(const qpam_delta_args &a) { return a.chunk > 0 ? a.chunk : CH; }
+// Four steps t .. t + 3 of one column of y or dv (planes or interleaved rows).
+__device__ __forceinline__ void store_column(const qpam_mview &v, int b, int h, int t0, int t, int valid, int col,
+                                             const floatx4 &re, const floatx4 &im) {
+    float *base = v.re + b * v.s0 + h * v.s1 + (int64_t)(t0 + t) * v.s2;
+    const bool il = pairs(v);
+    const int64_t pl = v.im - v.re;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if (t + r >= valid) continue;
+        if (il) {
+            reinterpret_cast<float2 *>(base + r * v.s2)[col] = make_float2(re[r], im[r]);
+        } else {
+            base[r * v.s2 + col] = re[r];
+            base[r * v.s2 + col + pl] = im[r];
+        }
+    }
+}
+// Four columns from col of step t of dy.
+__device__ __forceinline__ void load_four(const qpam_cview &v, int b, int h, int t, int col, floatx4 &re, floatx4 &im) {
+    const int64_t row = b * v.s0 + h * v.s1 + (int64_t)t * v.s2;
+    const float *r = static_cast<const float *>(v.re) + row;
+    if (pairs(v)) {
+        const floatx4 x = *reinterpret_cast<const floatx4 *>(r + 2 * col), y = *reinterpret_cast<const floatx4 *>(r + 2 * col + 4);
+        re = floatx4{x[0], x[2], y[0], y[2]};
+        im = floatx4{x[1], x[3], y[1], y[3]};
+    } else {
+        re = *reinterpret_cast<const floatx4 *>(r + col);
+        im = *reinterpret_cast<const floatx4 *>(static_cast<const float *>(v.im) + row + col);
+    }
+}
 // log of a step's decay factor (gamma + gamma_eps, kept at or above the smallest
 // normal float so that gamma = 0 stays finite)
 __device__ __forceinline__ float decay_log(float gamma, float eps) { return logf(fmaxf(gamma + eps, 1.17549435e-38f)); }
@@ -562,16 +592,7 @@ __global__ void __launch_bounds__(256, 2) delta_chunk_kernel(qpam_delta_args a, 
                 gstep(x, al * sKQr[ty * KP + j], al * sKQi[ty * KP + j], sSr[cur][j * SP + l16], sSi[cur][j * SP + l16]);
             }
             const floatx4 yr = gre(x), yi = gim(x);
-            float *yre = a.y.re + b * a.y.s0 + h * a.y.s1 + i0 + l16;
-            float *yim = a.y.im + b * a.y.s0 + h * a.y.s1 + i0 + l16;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int tr = 16 * wy + 4 * g + r;
-                if (tr < valid) {
-                    yre[(int64_t)(t0 + tr) * a.y.s2] = yr[r];
-                    yim[(int64_t)(t0 + tr) * a.y.s2] = yi[r];
-                }
-            }
+            store_column(a.y, b, h, t0, 16 * wy + 4 * g, valid, i0 + l16, yr, yi);
         }
         __syncthreads();  // before the next chunk's tiles replace Q and U
         cur ^= 1;
@@ -658,10 +679,10 @@ __global__ void __launch_bounds__(256, 2) delta_bwd_chain_kernel(qpam_delta_bwd_
     floatx4 dyr, dyi;
     auto fetch_dy = [&](int c) {
         const int t0 = c * chunk_len(a), valid = min(chunk_len(a), a.T - t0);
-        const int64_t o = b * bw.dy.s0 + h * bw.dy.s1 + (int64_t)(t0 + min(yt, valid - 1)) * bw.dy.s2 + i0 + yc;
         const float f = yt < valid ? 1.f : 0.f;
-        dyr = *reinterpret_cast<const floatx4 *>(static_cast<const float *>(bw.dy.re) + o) * f;
-        dyi = *reinterpret_cast<const floatx4 *>(static_cast<const float *>(bw.dy.im) + o) * f;
+        load_four(bw.dy, b, h, t0 + min(yt, valid - 1), i0 + yc, dyr, dyi);
+        dyr *= f;
+        dyi *= f;
     };
     float lnext = 0.f, bnext = 0.f;
     auto fetch_lb = [&](int c) {  // wave 0: L and beta of chunk c (beta 0 past the end)
@@ -784,19 +805,16 @@ __global__ void __launch_bounds__(256, 2) delta_bwd_chain_kernel(qpam_delta_bwd_
         }
         {  // dW -> the record; dv = beta dW
             float *dw = brec + BW_W + i0 + l16;
-            float *dvr = bw.dv.re + b * bw.dv.s0 + h * bw.dv.s1 + i0 + l16;
-            float *dvi = bw.dv.im + b * bw.dv.s0 + h * bw.dv.s1 + i0 + l16;
+            floatx4 vr, vi;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int t = 16 * w + 4 * g + r;
                 dw[t * D] = wr[r];
                 dw[D * D + t * D] = wi[r];
-                if (t < valid) {
-                    const float bt = sBt[t];
-                    dvr[(int64_t)(t0 + t) * bw.dv.s2] = bt * wr[r];
-                    dvi[(int64_t)(t0 + t) * bw.dv.s2] = bt * wi[r];
-                }
+                vr[r] = sBt[t] * wr[r];
+                vi[r] = sBt[t] * wi[r];
             }
+            store_column(bw.dv, b, h, t0, 16 * w + 4 * g, valid, i0 + l16, vr, vi);
         }
         __syncthreads();  // dU no longer read
 #pragma unroll
@@ -914,11 +932,10 @@ __global__ void __launch_bounds__(512, 2) delta_bwd_grad_kernel(qpam_delta_bwd_a
         load(xu, rec + WS_U, rec + WS_U + D * D, D, CH);
         if (qside) {
             const float f = own < valid ? 1.f : 0.f;
-            const int64_t o = b * bw.dy.s0 + h * bw.dy.s1 + (int64_t)(t0 + min(own, valid - 1)) * bw.dy.s2 + 4 * g;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const floatx4 re = *reinterpret_cast<const floatx4 *>(static_cast<const float *>(bw.dy.re) + o + 16 * k);
-                const floatx4 im = *reinterpret_cast<const floatx4 *>(static_cast<const float *>(bw.dy.im) + o + 16 * k);
+                floatx4 re, im;
+                load_four(bw.dy, b, h, t0 + min(own, valid - 1), 16 * k + 4 * g, re, im);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) row[k].re[r] = re[r] * f, row[k].im[r] = im[r] * f;
             }
@@ -1094,11 +1111,18 @@ __global__ void __launch_bounds__(512, 2) delta_bwd_grad_kernel(qpam_delta_bwd_a
         return dot;
     };
     const auto store = [&](const qpam_mview &v, float f) {
-        const int64_t o = b * v.s0 + h * v.s1 + (int64_t)(t0 + own) * v.s2 + 4 * g;
+        const int64_t row = b * v.s0 + h * v.s1 + (int64_t)(t0 + own) * v.s2;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            *reinterpret_cast<floatx4 *>(v.re + o + 16 * k) = xr[k] * f;
-            *reinterpret_cast<floatx4 *>(v.im + o + 16 * k) = xi[k] * f;
+            const floatx4 re = xr[k] * f, im = xi[k] * f;
+            if (pairs(v)) {
+                floatx4 *dst = reinterpret_cast<floatx4 *>(v.re + row + 2 * (16 * k + 4 * g));
+                dst[0] = floatx4{re[0], im[0], re[1], im[1]};
+                dst[1] = floatx4{re[2], im[2], re[3], im[3]};
+            } else {
+                *reinterpret_cast<floatx4 *>(v.re + row + 16 * k + 4 * g) = re;
+                *reinterpret_cast<floatx4 *>(v.im + row + 16 * k + 4 * g) = im;
+            }
         }
     };
     const float al = __expf(sL[own]), bt = sBt[own];
@@ -1159,11 +1183,14 @@ __global__ void __launch_bounds__(512, 2) delta_bwd_grad_kernel(qpam_delta_bwd_a
 
 bool aligned(const void *p, int bytes) { return ((uintptr_t)p % bytes) == 0; }
 
-bool cview_ok(const qpam_cview &v) {
-    return v.re && v.im && aligned(v.re, 16) && aligned(v.im, 16) && v.s0 % 4 == 0 && v.s1 % 4 == 0 && v.s2 % 4 == 0;
+template <typename V>
+bool rows_ok(const V &v) {  // 16-byte rows
+    return v.re && v.im && aligned(v.re, 16) && v.s0 % 4 == 0 && v.s1 % 4 == 0 && v.s2 % 4 == 0;
 }
-bool mview_ok(const qpam_mview &v) {
-    return v.re && v.im && aligned(v.re, 16) && aligned(v.im, 16) && v.s0 % 4 == 0 && v.s1 % 4 == 0 && v.s2 % 4 == 0;
+bool planes_ok(const qpam_cview &v) { return rows_ok(v) && aligned(v.im, 16); }
+template <typename V>
+bool view_ok(const V &v) {  // planes or interleaved rows
+    return rows_ok(v) && (pairs(v) || aligned(v.im, 16));
 }
 
 size_t n_chunks_of(const qpam_delta_args &a) { return (size_t)((a.T + chunk_len(a) - 1) / chunk_len(a)); }
@@ -1177,7 +1204,7 @@ int validate(const qpam_delta_args *a) {
     QPAM_REQUIRE(a->d == D, "qpam_delta: head_dim %d unsupported (64 only)", a->d);
     QPAM_REQUIRE(a->chunk >= 0 && a->chunk <= CH, "qpam_delta: chunk %d outside 1..%d (0 = %d)", a->chunk, CH, CH);
     QPAM_REQUIRE(a->exact_write == 0 || a->exact_write == 1, "qpam_delta: exact_write must be 0 or 1");
-    QPAM_REQUIRE(cview_ok(a->q) && cview_ok(a->k) && cview_ok(a->v),
+    QPAM_REQUIRE(planes_ok(a->q) && planes_ok(a->k) && planes_ok(a->v),
                  "qpam_delta: q, k, v must be 16-byte aligned fp32 planes with strides multiple of 4");
     QPAM_REQUIRE(a->gamma && a->beta, "qpam_delta: gamma and beta required");
     QPAM_REQUIRE((a->s0_re == nullptr) == (a->s0_im == nullptr), "qpam_delta: s0 needs both planes");
@@ -1198,7 +1225,7 @@ extern "C" size_t qpam_delta_scratch_size(const qpam_delta_args *a) { return a ?
 extern "C" int qpam_delta_fwd(const qpam_delta_args *a, void *stream) {
     int st = validate(a);
     if (st) return st;
-    QPAM_REQUIRE(mview_ok(a->y) && a->s_re && a->s_im && aligned(a->s_re, 16) && aligned(a->s_im, 16),
+    QPAM_REQUIRE(view_ok(a->y) && a->s_re && a->s_im && aligned(a->s_re, 16) && aligned(a->s_im, 16),
                  "qpam_delta_fwd: y (16-byte aligned planes) and the final state are required");
     QPAM_REQUIRE(a->workspace == nullptr || (aligned(a->workspace, 16) && a->workspace_bytes >= fwd_ws(*a)),
                  "qpam_delta_fwd: workspace of %zu bytes needed (or NULL without a backward)", fwd_ws(*a));
@@ -1234,7 +1261,7 @@ extern "C" int qpam_delta_bwd(const qpam_delta_bwd_args *g, void *stream) {
                  "qpam_delta_bwd: the forward's workspace (its per-chunk records) is required");
     QPAM_REQUIRE(g->workspace && aligned(g->workspace, 16) && g->workspace_bytes >= bwd_ws(a),
                  "qpam_delta_bwd: workspace of %zu bytes needed", bwd_ws(a));
-    QPAM_REQUIRE(cview_ok(g->dy) && mview_ok(g->dq) && mview_ok(g->dk) && mview_ok(g->dv),
+    QPAM_REQUIRE(view_ok(g->dy) && view_ok(g->dq) && view_ok(g->dk) && view_ok(g->dv),
                  "qpam_delta_bwd: dy, dq, dk, dv must be 16-byte aligned fp32 planes with strides multiple of 4");
     QPAM_REQUIRE(g->dgamma && g->dbeta, "qpam_delta_bwd: dgamma and dbeta required");
     QPAM_REQUIRE((g->ds_re == nullptr) == (g->ds_im == nullptr) && (g->ds0_re == nullptr) == (g->ds0_im == nullptr),

@@ -90,17 +90,7 @@ __device__ __forceinline__ void tile_load_u(F32Tile<ROWS> &t, const float *base,
     }
 }
 
-// A view of interleaved complex rows: im is the element after re, strides in floats.
-// y, dy and the gradients of the fp32 kernels take it beside separate planes, so a
-// split-real [..., d, 2] tensor needs no pass of its own to be packed or unpacked:
-// B=4, H=12, T=1000, M=1 training call 346 -> 309 us (y, dy, dq, dk, dv; the two kernels
-// that read or write them take 13 us more, the copies they replace took 50).
-inline __host__ __device__ bool pairs(const qpam_cview &v) {
-    return v.re && static_cast<const float *>(v.im) == static_cast<const float *>(v.re) + 1;
-}
-inline __host__ __device__ bool pairs(const qpam_mview &v) { return v.re && v.im == v.re + 1; }
-
-// tile_load of both planes from such rows.
+// tile_load of both planes from interleaved rows (pairs).
 template <int ROWS>
 __device__ __forceinline__ void tile_load_pairs(F32Tile<ROWS> &re, F32Tile<ROWS> &im, const float *base, int64_t st,
                                                 int valid) {

@@ -24,7 +24,7 @@ from torch import Tensor
 
 from . import _lib, planes
 from ._ops import op
-from .pam_scan import _cview, _mview
+from .pam_scan import _cview, _cview_pairs, _mview, _mview_pairs, _reads_pairs
 
 CHUNK_EPS = 1e-6
 
@@ -81,16 +81,17 @@ def delta_fwd_op(q_re: Tensor, q_im: Tensor, k_re: Tensor, k_im: Tensor, v_re: T
 
 
 def _delta_fwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, beta, s0_re, s0_im, q_scale, gamma_eps, chunk, exact_write,
-               keep_workspace):
+               keep_workspace, pairs=False):
+    """pairs: y is one [B,H,T,d,2] tensor in the y_re slot (y_im empty)."""
     a, keep = _fill(q_re, q_im, k_re, k_im, v_re, v_im, gamma, beta, s0_re, s0_im, q_scale, gamma_eps, chunk,
                     exact_write)
     B, H, T, d = q_re.shape
     dev = q_re.device
-    y_re = torch.empty(B, H, T, d, device=dev, dtype=torch.float32)
-    y_im = torch.empty_like(y_re)
+    y_re = torch.empty((B, H, T, d, 2) if pairs else (B, H, T, d), device=dev, dtype=torch.float32)
+    y_im = y_re.new_empty(0) if pairs else torch.empty_like(y_re)
     s_re = torch.empty(B, H, d, d, device=dev, dtype=torch.float32)
     s_im = torch.empty_like(s_re)
-    a.y = _mview(y_re, y_im)
+    a.y = _mview_pairs(y_re) if pairs else _mview(y_re, y_im)
     a.s_re, a.s_im = s_re.data_ptr(), s_im.data_ptr()
     L = _lib.lib()
     if keep_workspace:
@@ -148,7 +149,8 @@ def delta_bwd_op(q_re: Tensor, q_im: Tensor, k_re: Tensor, k_im: Tensor, v_re: T
 
 
 def _delta_bwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, beta, s0_re, s0_im, q_scale, gamma_eps, chunk, exact_write,
-               ws, dy_re, dy_im, ds_re, ds_im):
+               ws, dy_re, dy_im, ds_re, ds_im, pairs=False):
+    # pairs: the first three results are [B,H,T,d,2] tensors; dy is one when dy_im is None
     # the kernels write dgamma and dbeta with gamma's strides: contiguous planes,
     # matching the gradients allocated below
     gamma, beta = gamma.contiguous(), beta.contiguous()
@@ -159,13 +161,20 @@ def _delta_bwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, beta, s0_re, s0_im, q_
     a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel() * 4
     g = _lib.DeltaBwdArgs()
     g.fwd = _lib.ctypes.pointer(a)
-    dy_re, dy_im = dy_re.float().contiguous(), dy_im.float().contiguous()
-    g.dy, _, _ = _cview(dy_re, dy_im)
+    if dy_im is None:
+        g.dy = _cview_pairs(dy_re)
+    else:
+        dy_re, dy_im = dy_re.float().contiguous(), dy_im.float().contiguous()
+        g.dy, _, _ = _cview(dy_re, dy_im)
     if ds_re is not None:
         ds_re, ds_im = ds_re.float().contiguous(), ds_im.float().contiguous()
         g.ds_re, g.ds_im = ds_re.data_ptr(), ds_im.data_ptr()
-    outs = [torch.empty(B, H, T, d, device=dev, dtype=torch.float32) for _ in range(6)]
-    g.dq, g.dk, g.dv = _mview(outs[0], outs[1]), _mview(outs[2], outs[3]), _mview(outs[4], outs[5])
+    if pairs:
+        outs = [torch.empty(B, H, T, d, 2, device=dev, dtype=torch.float32) for _ in range(3)]
+        g.dq, g.dk, g.dv = (_mview_pairs(x) for x in outs)
+    else:
+        outs = [torch.empty(B, H, T, d, device=dev, dtype=torch.float32) for _ in range(6)]
+        g.dq, g.dk, g.dv = _mview(outs[0], outs[1]), _mview(outs[2], outs[3]), _mview(outs[4], outs[5])
     dgamma = torch.empty(B, H, T, device=dev, dtype=torch.float32)
     dbeta = torch.empty_like(dgamma)
     g.dgamma, g.dbeta = dgamma.data_ptr(), dbeta.data_ptr()
@@ -269,9 +278,13 @@ def delta_il_fwd_op(q: Tensor, k: Tensor, v: Tensor, gamma: Tensor, beta: Tensor
     unpacked into padded fp32 planes by one launch, y and the state packed by
     another.  Returns [y, s in q's dtype, planes [3,2,B,H,T,64], workspace]."""
     pl = planes.split_rows((q, k, v), torch.float32)
+    pairs = q.dtype == torch.float32 and q.shape[3] == planes.KD  # the kernels write split-real rows themselves
     y_re, y_im, s_re, s_im, ws = _delta_fwd(pl[0, 0], pl[0, 1], pl[1, 0], pl[1, 1], pl[2, 0], pl[2, 1], gamma, beta,
-                                            None, None, q_scale, CHUNK_EPS, chunk, False, keep_workspace)
-    y, s = planes.merge([(y_re, y_im)], [(s_re, s_im)], q.shape[3], q.dtype)
+                                            None, None, q_scale, CHUNK_EPS, chunk, False, keep_workspace, pairs)
+    if pairs:
+        y, s = y_re, planes.merge([], [(s_re, s_im)], q.shape[3], q.dtype)[0]
+    else:
+        y, s = planes.merge([(y_re, y_im)], [(s_re, s_im)], q.shape[3], q.dtype)
     return [y, s, pl, ws]
 
 
@@ -287,13 +300,18 @@ def _(q, k, v, gamma, beta, q_scale, chunk, keep_workspace):
 def delta_il_bwd_op(pl: Tensor, gamma: Tensor, beta: Tensor, q_scale: float, chunk: int, ws: Tensor,
                     dy: Optional[Tensor], ds: Optional[Tensor], d: int, bf16: bool) -> List[Tensor]:
     """[dq, dk, dv [B,H,T,d,2] (bf16 or fp32), dgamma, dbeta]."""
-    if dy is not None:
-        dyp = planes.split_rows((dy,), torch.float32)[0]
-    else:
+    pairs = not bf16 and d == planes.KD
+    if dy is None:
         dyp = torch.zeros(pl.shape[1:], device=pl.device, dtype=torch.float32)
+    elif pairs and _reads_pairs(dy):
+        dyp = (dy, None)
+    else:
+        dyp = planes.split_rows((dy,), torch.float32)[0]
     dsp = planes.split_states(ds) if ds is not None else (None, None)
     g = _delta_bwd(pl[0, 0], pl[0, 1], pl[1, 0], pl[1, 1], pl[2, 0], pl[2, 1], gamma, beta, None, None, q_scale,
-                   CHUNK_EPS, chunk, False, ws, dyp[0], dyp[1], dsp[0], dsp[1])
+                   CHUNK_EPS, chunk, False, ws, dyp[0], dyp[1], dsp[0], dsp[1], pairs)
+    if pairs:
+        return g[:5]
     return planes.merge([(g[0], g[1]), (g[2], g[3]), (g[4], g[5])], [], d,
                         torch.bfloat16 if bf16 else torch.float32) + [g[6], g[7]]
 

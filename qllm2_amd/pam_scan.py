@@ -80,6 +80,10 @@ def _mview_pairs(x):
     return _lib.MView(x.data_ptr(), x.data_ptr() + 4, *x.stride()[:3])
 
 
+def _cview_pairs(x):
+    return _lib.CView(x.data_ptr(), x.data_ptr() + 4, *x.stride()[:3])
+
+
 def _fill_args(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, s0_im, q_scale, chunk):
     M, B, H, T = gamma.shape
     q, qr, qi = _cview(_aligned_plane(q_re), _aligned_plane(q_im))
@@ -248,7 +252,7 @@ def _scan_bwd(q_re, q_im, k_re, k_im, v_re, v_im, gamma, rot_re, rot_im, s0_re, 
         if y_layout == 1:
             dy_re, dy_im = dy_re.transpose(1, 2), dy_im.transpose(1, 2)
     if dy_im is None:  # one [B,H,T,d,2] gradient (layout PAIRS)
-        bw.dy = _lib.CView(dy_re.data_ptr(), dy_re.data_ptr() + 4, *dy_re.stride()[:3])
+        bw.dy = _cview_pairs(dy_re)
     else:
         bw.dy, _, _ = _cview(dy_re, dy_im)
     if ds_re is not None:

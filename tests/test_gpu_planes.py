@@ -107,6 +107,7 @@ def test_delta_split_real_equals_planar(gpu_lib, d, T, chunk, dtype, given, how)
         assert a.dtype == b.dtype and torch.equal(a, b), i
 
 
+@pytest.mark.parametrize("kind", ["scan", "delta"])
 @pytest.mark.parametrize("T,M,form", [
     (1, 1, "dense"), (63, 2, "dense"), (130, 4, "dense"),
     (70, 1, "heads_last"),   # the rows of a [B,T,H,64,2] tensor
@@ -115,16 +116,20 @@ def test_delta_split_real_equals_planar(gpu_lib, d, T, chunk, dtype, given, how)
     (70, 1, "offset"),       # 8-byte aligned storage: packed first
     (70, 1, "none"),         # the state's gradient only
 ])
-def test_split_real_rows_equal_planes(gpu_lib, T, M, form):
-    """fp32, head dim 64, 64-step chunks: y leaves and the gradients arrive and leave as
+def test_split_real_rows_equal_planes(gpu_lib, T, M, form, kind):
+    """fp32, head dim 64 (64-step chunks for the scan): y leaves and the gradients arrive and leave as
     split-real rows.  The arithmetic is that of the planes, so every result is the
     planar call's bit for bit, whatever the strides of dy."""
+    from qllm2_amd.pam_delta import delta_planar, forward_delta
     from qllm2_amd.pam_scan import pam_scan_interleaved, pam_scan_planar
     B, H, d = 2, 3, 64
     g = torch.Generator().manual_seed(17 * T + M)
     qkv = [(0.3 * torch.randn(B, H, T, d, 2, generator=g)).cuda() for _ in range(3)]
-    gamma = (0.85 + 0.15 * torch.rand(M, B, H, T, generator=g)).cuda()
-    ds = torch.randn(M, B, H, d, d, 2, generator=g).cuda()
+    lead = (M, B, H) if kind == "scan" else (B, H)
+    gates = [(0.85 + 0.15 * torch.rand(*lead, T, generator=g)).cuda()]
+    if kind == "delta":
+        gates.append(torch.rand(*lead, T, generator=g).cuda())
+    ds = torch.randn(*lead, d, d, 2, generator=g).cuda()
     dy = torch.randn(B, H, T, d, 2, generator=g).cuda()
     if form == "heads_last":
         dy = dy.transpose(1, 2).contiguous().transpose(1, 2)
@@ -137,19 +142,21 @@ def test_split_real_rows_equal_planes(gpu_lib, T, M, form):
         buf[2:] = dy.reshape(-1)
         dy = buf[2:].view(B, H, T, d, 2)
 
-    xs = [x.clone().requires_grad_(True) for x in (*qkv, gamma)]
-    y, s = pam_scan_interleaved(*xs, d, 64)
+    xs = [x.clone().requires_grad_(True) for x in (*qkv, *gates)]
+    y, s = pam_scan_interleaved(*xs, d, 64) if kind == "scan" else forward_delta(*xs, d)
     ps = [x[..., i].contiguous().requires_grad_(True) for x in qkv for i in (0, 1)]
-    gam = gamma.clone().requires_grad_(True)
-    y_re, y_im, s_re, s_im = pam_scan_planar(*ps, gam, q_scale=d ** -0.5, chunk=64)
+    gs = [x.clone().requires_grad_(True) for x in gates]
+    y_re, y_im, s_re, s_im = (pam_scan_planar(*ps, *gs, q_scale=d ** -0.5, chunk=64) if kind == "scan"
+                              else delta_planar(*ps, *gs, q_scale=d ** -0.5))
     assert torch.equal(y, torch.stack([y_re, y_im], -1)) and torch.equal(s, torch.stack([s_re, s_im], -1))
     if form == "none":
         got = torch.autograd.grad([s], xs, [ds])
-        ref = torch.autograd.grad([s_re, s_im], [*ps, gam], [ds[..., 0], ds[..., 1]])
+        ref = torch.autograd.grad([s_re, s_im], [*ps, *gs], [ds[..., 0], ds[..., 1]])
     else:
         got = torch.autograd.grad([y, s], xs, [dy, ds])
-        ref = torch.autograd.grad([y_re, y_im, s_re, s_im], [*ps, gam],
+        ref = torch.autograd.grad([y_re, y_im, s_re, s_im], [*ps, *gs],
                                   [dy[..., 0].contiguous(), dy[..., 1].contiguous(), ds[..., 0], ds[..., 1]])
     for i in range(3):
         assert torch.equal(got[i], torch.stack([ref[2 * i], ref[2 * i + 1]], -1)), i
-    assert torch.equal(got[3], ref[6])
+    for a, b in zip(got[3:], ref[6:]):
+        assert torch.equal(a, b)
