@@ -7,8 +7,8 @@
 // cache lines.  fp32 calls of head dim 64 pass here with q, k, v and the state only (their
 // y and gradients leave the kernels as split-real rows); the others also with y, dy and
 // the gradients.  At B=8, H=12, T=2048, d=64 fp32 (100 MB a tensor) splitting q, k, v moves
-// 604 MB in 91 us = 6.6 TB/s; a step that copies all eight tensors moves 1.6 GB in 265 us, where slices, zero fills, adds and stacks
-// took 870 us.
+// 604 MB in 91 us = 6.6 TB/s; a step that copies all eight tensors moves 1.6 GB in
+// 265 us, where the slices, zero fills, adds and stacks of the library took 870 us.
 #include "common.h"
 
 namespace qpam {

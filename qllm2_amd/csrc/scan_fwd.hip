@@ -211,7 +211,8 @@ __device__ __forceinline__ void by_tile(int tt, F &&f) {
     }
 }
 
-template <int C>
+// PAIRS: y as split-real rows (a branch in the store loop cost the planar form 1%).
+template <int C, bool PAIRS>
 __global__ void __launch_bounds__(THREADS, 2) chunk_output_f32_kernel(FwdParams p) {
     extern __shared__ float smem[];
     float *sKr = smem, *sKi = sKr + C * P, *sVr = sKi + C * P, *sVi = sVr + C * P;
@@ -385,7 +386,6 @@ __global__ void __launch_bounds__(THREADS, 2) chunk_output_f32_kernel(FwdParams 
         }
     }
 
-    const bool ypairs = pairs(a.y);
     const int64_t yo = b * a.y.s0 + h * a.y.s1 + (int64_t)c0 * a.y.s2;
 #pragma unroll
     for (int it = 0; it < 4; ++it)
@@ -395,7 +395,7 @@ __global__ void __launch_bounds__(THREADS, 2) chunk_output_f32_kernel(FwdParams 
             if (tr >= valid) continue;
             const float re = y1[it][r] - y2[it][r], im = y3[it][r] - y1[it][r] - y2[it][r];
             float *y = a.y.re + yo + (int64_t)tr * a.y.s2;
-            if (ypairs) {
+            if constexpr (PAIRS) {
                 reinterpret_cast<float2 *>(y)[16 * it + l16] = make_float2(re, im);
             } else {
                 y[16 * it + l16] = re;
@@ -1375,7 +1375,10 @@ int launch_fwd(const FwdParams &p, hipStream_t stream) {
     const qpam_scan_args &a = p.a;
     dim3 grid(p.n_chunks, a.H, a.B);
     constexpr bool f32 = std::is_same<Tin, float>::value;
-    const void *out_kernel = f32 ? (const void *)chunk_output_f32_kernel<C> : (const void *)chunk_output_kernel<Tin, C>;
+    const bool pr = pairs(p.a.y);
+    const void *out_kernel = !f32 ? (const void *)chunk_output_kernel<Tin, C>
+                             : pr ? (const void *)chunk_output_f32_kernel<C, true>
+                                  : (const void *)chunk_output_f32_kernel<C, false>;
     const size_t s1 = state_smem<C>(), s3 = f32 ? output_f32_smem<C>() : output_smem<C>();
     QPAM_CHECK_HIP(hipFuncSetAttribute(out_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)s3));
     int st;
@@ -1400,8 +1403,10 @@ int launch_fwd(const FwdParams &p, hipStream_t stream) {
         if (st) return st;
     }
     if (a.prof_ev[0]) QPAM_CHECK_HIP(hipEventRecord((hipEvent_t)a.prof_ev[0], stream));
-    if constexpr (f32) hipLaunchKernelGGL((chunk_output_f32_kernel<C>), grid, dim3(THREADS), s3, stream, p);
-    else hipLaunchKernelGGL((chunk_output_kernel<Tin, C>), grid, dim3(THREADS), s3, stream, p);
+    if constexpr (f32) {
+        if (pr) hipLaunchKernelGGL((chunk_output_f32_kernel<C, true>), grid, dim3(THREADS), s3, stream, p);
+        else hipLaunchKernelGGL((chunk_output_f32_kernel<C, false>), grid, dim3(THREADS), s3, stream, p);
+    } else hipLaunchKernelGGL((chunk_output_kernel<Tin, C>), grid, dim3(THREADS), s3, stream, p);
     st = launch_status("chunk_output_kernel");
     if (st) return st;
     if (a.prof_ev[1]) QPAM_CHECK_HIP(hipEventRecord((hipEvent_t)a.prof_ev[1], stream));
