@@ -9,9 +9,9 @@ Reference methods replaced (v11/model.py):
   _recur_step_additive      927-965  (one decode step)
   _recurrent                845-925  (decode token loop; all K states of a
                                       token in one kernel launch)
-  _forward_chunked_perchannel 421-489 (E1 per-channel decay: the fold and the
-                                      state scan as HIP kernels, the chunk
-                                      products as batched complex GEMMs)
+  _forward_chunked_perchannel 421-489 (E1 per-channel decay: HIP chunk kernels
+                                      up to head dim 64; above, HIP fold and
+                                      state scan around batched complex GEMMs)
   _forward_delta            491-576  (E2 delta write; HIP token recurrence
                                       instead of the per-chunk solve)
   _recur_step_delta         967-1002 (one E2 decode token)
