@@ -21,10 +21,11 @@ HBM.  Larger head dims (two or more 64-wide tiles per operand) run as
 
 Both have gradients for q, k, v and gamma.  The whole computation is fp32 (the
 reference computes in the input dtype); outputs are cast back to the input
-dtype.
+dtype.  A second derivative raises, as it does for the registered operators.
 """
 
 import ctypes
+import functools
 
 import torch
 
@@ -59,17 +60,48 @@ def _ptr(t):
     return t.data_ptr() if t is not None else None
 
 
+class _FirstOrder(torch.autograd.Function):
+    """The first n arguments (a backward's results, formed outside autograd), tied
+    to the others, the tensors they were formed from."""
+
+    @staticmethod
+    def forward(ctx, n, *tensors):
+        return tuple(t.view_as(t) if t is not None else None for t in tensors[:n])
+
+    @staticmethod
+    def backward(ctx, *grads):
+        raise RuntimeError("qpam per-channel scan: the gradients come from the HIP library and have no second "
+                           "derivative")
+
+
+def _first_order(backward):
+    """A backward whose results a second derivative must not take for constants:
+    under create_graph they raise when they are differentiated.  (torch's
+    once_differentiable ties them to the incoming gradients only: with a constant
+    one, their dependence on the saved tensors would be lost without an error.)
+    The saved tensors are inputs or outputs of the function, not copies of them."""
+
+    @functools.wraps(backward)
+    def wrapped(ctx, *grads):
+        with torch.no_grad():
+            out = backward(ctx, *grads)
+        if not torch.is_grad_enabled():
+            return out
+        return _FirstOrder.apply(len(out), *out, *ctx.saved_tensors, *grads)
+
+    return wrapped
+
+
 class _Fold(torch.autograd.Function):
-    """(q, k [B,H,T,d,2], gamma [B,H,T,d]) -> qf, kf, wf [B*H, n, C, d, 2] fp32
-    and atot [B*H, n, d]: the folded operands of every chunk."""
+    """(q, k [B,H,T,d,2] of one dtype, complex rows contiguous, gamma [B,H,T,d],
+    channels contiguous) -> qf, kf, wf [B*H, n, C, d, 2] fp32 and atot [B*H, n, d]:
+    the folded operands of every chunk."""
 
     @staticmethod
     def forward(ctx, q, k, gamma, chunk, q_scale):
         if q.dim() != 5 or q.shape[-1] != 2 or k.shape != q.shape or gamma.shape != q.shape[:4]:
             raise ValueError(f"qpam per-channel fold: q, k [B,H,T,d,2] and gamma [B,H,T,d] expected, got "
                              f"{tuple(q.shape)}, {tuple(k.shape)}, {tuple(gamma.shape)}")
-        q, k = _pairs(q), _pairs(k.to(q.dtype))
-        gamma = gamma if gamma.stride(-1) == 1 else gamma.contiguous()
         B, H, T, d = q.shape[:4]
         n = -(-T // chunk)
         dev = q.device
@@ -97,6 +129,7 @@ class _Fold(torch.autograd.Function):
         return a
 
     @staticmethod
+    @_first_order
     def backward(ctx, dqf, dkf, dwf, datot):
         q, k, gamma = ctx.saved_tensors
         dq, dk = torch.empty(q.shape, device=q.device, dtype=q.dtype), torch.empty(k.shape, device=k.device,
@@ -122,15 +155,14 @@ def _scan(x, a, out, init, fin, reverse):
 
 
 class _Scan(torch.autograd.Function):
-    """(x [N,n,d,d,2] chunk increments, a [N,n,d] column decays) -> (state
-    entering each chunk [N,n,d,d,2], final state [N,d,d,2])."""
+    """(x [N,n,d,d,2] chunk increments, a [N,n,d] column decays, contiguous) ->
+    (state entering each chunk [N,n,d,d,2], final state [N,d,d,2])."""
 
     @staticmethod
     def forward(ctx, x, a):
         if a.dim() != 3 or x.shape != (*a.shape, a.shape[2], 2):
             raise ValueError(f"qpam per-channel scan: x [N,n,d,d,2] and a [N,n,d] expected, got "
                              f"{tuple(x.shape)}, {tuple(a.shape)}")
-        x, a = x.contiguous(), a.contiguous()
         N, n, d = a.shape
         out = torch.empty_like(x)
         fin = torch.empty(N, d, d, 2, device=x.device, dtype=torch.float32)
@@ -139,6 +171,7 @@ class _Scan(torch.autograd.Function):
         return out, fin
 
     @staticmethod
+    @_first_order
     def backward(ctx, dout, dfin):
         a, out = ctx.saved_tensors
         dout = dout.contiguous() if dout is not None else torch.zeros_like(out)
@@ -161,13 +194,11 @@ def _aligned(x):
 
 
 class _Chunked(torch.autograd.Function):
-    """(q, k, v [B,H,T,d,2], gamma [B,H,T,d], d <= 64) -> y [B,H,T,d,2] in q's
-    dtype and the final state [B,H,d,d,2] fp32."""
+    """(q, k, v [B,H,T,d,2], _aligned, gamma [B,H,T,d], channels contiguous,
+    d <= 64) -> y [B,H,T,d,2] in q's dtype and the final state [B,H,d,d,2] fp32."""
 
     @staticmethod
     def forward(ctx, q, k, v, gamma, chunk, q_scale):
-        q, k, v = _aligned(q), _aligned(k), _aligned(v)
-        gamma = gamma if gamma.stride(-1) == 1 else gamma.contiguous()
         B, H, T, d = q.shape[:4]
         n = -(-T // chunk)
         f32 = dict(device=q.device, dtype=torch.float32)
@@ -198,6 +229,7 @@ class _Chunked(torch.autograd.Function):
         return a
 
     @staticmethod
+    @_first_order
     def backward(ctx, dy, dfin):
         q, k, v, gamma, s_in, atot = ctx.saved_tensors
         dy = dy.contiguous() if dy is not None else torch.zeros(q.shape, device=q.device, dtype=q.dtype)
@@ -223,6 +255,7 @@ def perchannel_chunked(queries, keys, protected_values, decay_gamma, head_dim, c
     C = int(chunk_size)
     if not 1 <= C <= 64:
         raise ValueError(f"qpam per-channel scan: chunk_size {C} outside 1..64")
+    gamma = decay_gamma if decay_gamma.stride(-1) == 1 else decay_gamma.contiguous()
     if d <= KERNEL_D:
         if queries.dim() != 5 or keys.shape != queries.shape or protected_values.shape != queries.shape \
                 or queries.shape[-1] != 2 or decay_gamma.shape != queries.shape[:4]:
@@ -230,12 +263,12 @@ def perchannel_chunked(queries, keys, protected_values, decay_gamma, head_dim, c
                              f"{tuple(queries.shape)}, {tuple(keys.shape)}, {tuple(protected_values.shape)}, "
                              f"{tuple(decay_gamma.shape)}")
         v = protected_values
-        y, s_fin = _Chunked.apply(queries, keys.to(queries.dtype),
-                                  v if v.dtype in (torch.float32, torch.bfloat16) else v.float(), decay_gamma, C,
+        y, s_fin = _Chunked.apply(_aligned(queries), _aligned(keys.to(queries.dtype)),
+                                  _aligned(v if v.dtype in (torch.float32, torch.bfloat16) else v.float()), gamma, C,
                                   head_dim ** -0.5)
         return y, s_fin.to(queries.dtype)
     n = -(-T // C)
-    qf, kf, wf, atot = _Fold.apply(queries, keys, decay_gamma, C, head_dim ** -0.5)
+    qf, kf, wf, atot = _Fold.apply(_pairs(queries), _pairs(keys.to(queries.dtype)), gamma, C, head_dim ** -0.5)
     Q, K, W = (torch.view_as_complex(t) for t in (qf, kf, wf))   # [N, n, C, d]
     v = protected_values.float()
     if n * C != T:
@@ -245,7 +278,7 @@ def perchannel_chunked(queries, keys, protected_values, decay_gamma, head_dim, c
     P = (Q @ K.conj().transpose(-1, -2).contiguous()) * _mask(C, queries.device)   # masked score [N,n,C,C]
     Y = P @ V
     dS = V.transpose(-1, -2).contiguous() @ W.conj().resolve_conj()                # sum_s v_s[i] conj(w_s[j])
-    s_in, s_fin = _Scan.apply(torch.view_as_real(dS), atot)
+    s_in, s_fin = _Scan.apply(torch.view_as_real(dS).contiguous(), atot)
     Y = Y + Q @ torch.view_as_complex(s_in).transpose(-1, -2).contiguous()      # carried read q' S^T
     y = torch.view_as_real(Y).reshape(B, H, n * C, d, 2)[:, :, :T]
     return y.to(queries.dtype), s_fin.reshape(B, H, d, d, 2).to(queries.dtype)
