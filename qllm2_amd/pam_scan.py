@@ -542,8 +542,10 @@ def scan_il_bwd_op(pl: Tensor, gamma: Tensor, rot_re: Optional[Tensor], rot_im: 
 @scan_il_bwd_op.register_fake
 def _(pl, gamma, rot_re, rot_im, q_scale, chunk, ws, dy, ds, d):
     _, _, B, H, T, _ = pl.shape
-    dr = [torch.empty_like(gamma) if rot_re is not None else gamma.new_empty(0) for _ in range(2)]
-    return [pl.new_empty(B, H, T, d, 2) for _ in range(3)] + [torch.empty_like(gamma)] + dr
+    # contiguous whatever gamma's strides (empty_like would keep a transposed gate's)
+    dg = gamma.new_empty(gamma.shape)
+    dr = [gamma.new_empty(gamma.shape) if rot_re is not None else gamma.new_empty(0) for _ in range(2)]
+    return [pl.new_empty(B, H, T, d, 2) for _ in range(3)] + [dg] + dr
 
 
 def _il_setup(ctx, inputs, output):

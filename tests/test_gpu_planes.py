@@ -160,3 +160,28 @@ def test_split_real_rows_equal_planes(gpu_lib, T, M, form, kind):
         assert torch.equal(got[i], torch.stack([ref[2 * i], ref[2 * i + 1]], -1)), i
     for a, b in zip(got[3:], ref[6:]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("d,M,T,dtype", [(64, 1, 70, torch.float32), (48, 2, 33, torch.float32), (64, 2, 65, torch.bfloat16)])
+def test_fake_kernels_match_the_real_ones(gpu_lib, d, M, T, dtype):
+    """Shape, strides and dtype of every output, with a gate (and rotations) transposed from [B,T,H]."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from qllm2_amd import pam_delta, pam_scan
+    print(f"case d={d} M={M} T={T} {dtype}", flush=True)
+    B, H = 2, 4
+
+    def calls(make):
+        q = make(B, H, T, d, 2).to(dtype)
+        gate = make(B, T, H).transpose(1, 2)
+        gamma = make(M, B, T, H).transpose(2, 3)
+        rot = (gamma, gamma) if M > 1 else (None, None)
+        y, s, pl, ws = out = pam_scan.scan_il_fwd_op(q, q, q, gamma, *rot, 0.125, 64)
+        outs = out + pam_scan.scan_il_bwd_op(pl, gamma, *rot, 0.125, 64, ws, y, s, d)
+        y, s, pl, ws = out = pam_delta.delta_il_fwd_op(q, q, q, gate, gate, 0.125, 64, True)
+        return outs + out + pam_delta.delta_il_bwd_op(pl, gate, gate, 0.125, 64, ws, y, s, d, dtype == torch.bfloat16)
+
+    real = calls(lambda *s: torch.full(s, 0.5, device="cuda"))
+    with FakeTensorMode():
+        fake = calls(lambda *s: torch.empty(s, device="cuda"))
+    for i, (r, f) in enumerate(zip(real, fake)):
+        assert r.shape == f.shape and r.stride() == f.stride() and r.dtype == f.dtype, i
