@@ -27,6 +27,33 @@ __device__ __forceinline__ void gstep(Gauss &x, float ar, float ai, float br, fl
 __device__ __forceinline__ floatx4 gre(const Gauss &x) { return x.t1 - x.t2; }
 __device__ __forceinline__ floatx4 gim(const Gauss &x) { return x.t3 - x.t1 - x.t2; }
 
+// The same product with every real part summed on its own, re in one sum and im in
+// another: four MFMAs, but no im = t3 - t1 - t2 from sums that each carry their own
+// rounding (and an infinite part of an operand stays out of the other part).  conj:
+// of neither operand, of a, or of b.
+struct Plain {
+    floatx4 re, im;
+};
+__device__ __forceinline__ void pz(Plain &x) { x.re = x.im = floatx4{0.f, 0.f, 0.f, 0.f}; }
+__device__ __forceinline__ void pstep(Plain &x, float ar, float ai, float br, float bi) {
+    x.re = mfma4(ar, br, x.re);
+    x.im = mfma4(ar, bi, x.im);
+    x.re = mfma4(ai, -bi, x.re);
+    x.im = mfma4(ai, br, x.im);
+}
+__device__ __forceinline__ void pstep_ca(Plain &x, float ar, float ai, float br, float bi) {
+    x.re = mfma4(ar, br, x.re);
+    x.im = mfma4(ar, bi, x.im);
+    x.re = mfma4(ai, bi, x.re);
+    x.im = mfma4(ai, -br, x.im);
+}
+__device__ __forceinline__ void pstep_cb(Plain &x, float ar, float ai, float br, float bi) {
+    x.re = mfma4(ar, br, x.re);
+    x.im = mfma4(ar, -bi, x.im);
+    x.re = mfma4(ai, bi, x.re);
+    x.im = mfma4(ai, br, x.im);
+}
+
 // Interleaved complex LDS tiles: 64 rows of pitch CP.  One 8-byte read gives both
 // parts of an operand down a column, two 16-byte reads four consecutive ones along
 // a row; CP = 68 puts the four lane groups' rows 4 g + r of a column read on

@@ -867,14 +867,17 @@ __global__ void __launch_bounds__(THREADS) key_side_kernel(BwdParams p) {
 // columns.  Per state m, S_m and G'_m then take V's and dY's tiles (the lanes keep
 // their own rows of both).  The decay gradient's row sums over s stay in the lane,
 // its column sums over t are DPP row sums into one LDS slice per wave, added in
-// wave order, so the result is reproducible.  Three real MFMAs per complex product
-// (gauss.h), but four separate real sums for the two products the decay gradient is made
-// of (+2 us): over lengths 50-930 and 1-4 states the gradients' error against 64 bits is
-// 0.92 of the two kernels', the worst output of every case no larger.  Bound by the matrix
-// cores (60 us at full rate for 768 chunks) and the causal steps' decay arithmetic between
-// them.  Against the query and key sides as kernels of four waves, each staging all four
-// tiles and using four-product MFMAs: B=4, H=12, T=1000, M=1: 115 + 129 -> 133 us
-// (139 us with split-real dy, dq, dk and dv).
+// wave order, so the result is reproducible.  Every real part of a product is summed on
+// its own (gauss.h, Plain; the two products the decay gradient is made of in four sums
+// each): with three MFMAs per product dv's imaginary plane was 1.04-1.11 times as far from
+// 64 bits as with the query and key sides as kernels of their own.  Now, pooled over lengths
+// 50-930 and 1-4 states, every plane of dq is at 0.86-0.98 of their distance, dk 0.59-0.84, dv
+// 1.00 and dgamma 0.90-1.04.  Bound by the matrix cores (77 us at full rate for 768 chunks) and the
+// causal steps' decay arithmetic between them; no spills for 1 to 4 states (204-235
+// registers; the three-MFMA sums held 236 and spilled 19-30 from two states on).  B=4, H=12,
+// T=1000, split-real rows, 1 / 2 / 3 / 4 states: 152 / 195 / 235 / 284 us (145 / 192 / 238 /
+// 287 with three MFMAs; 248 / 335 / 437 / 530 as query and key sides, four waves each, each
+// staging all four tiles).
 constexpr int CGF_THREADS = 512;
 template <int M>
 constexpr size_t cgf_smem() { return 4 * TILE * sizeof(float2) + (11 * M * 64 + 8 * M) * sizeof(float); }
@@ -965,9 +968,9 @@ __global__ void __launch_bounds__(CGF_THREADS, 2) chunk_grad_f32_kernel(BwdParam
 
     Four row[4];                                   // query: the dY row of step `own`; key: its V row
     floatx4 xr[4], xi[4], yr[4], yi[4];            // query: dQ (x); key: dV (x) and dK (y)
-    Gauss acc[4];
+    Plain acc[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) gz(acc[k]), xr[k] = xi[k] = yr[k] = yi[k] = zero4();
+    for (int k = 0; k < 4; ++k) pz(acc[k]), xr[k] = xi[k] = yr[k] = yi[k] = zero4();
     if (active) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) row[k] = row4(qside ? sY : sV, own, 16 * k + 4 * g);
@@ -1036,7 +1039,7 @@ __global__ void __launch_bounds__(CGF_THREADS, 2) chunk_grad_f32_kernel(BwdParam
 #pragma unroll
                     for (int jt = 0; jt < 4; ++jt) {
                         const float2 e = sK[(16 * st + 4 * g + r) * CP + 16 * jt + l16];
-                        gstep(acc[jt], e.x, e.y, gwr[r], gwi[r]);
+                        pstep(acc[jt], e.x, e.y, gwr[r], gwi[r]);
                     }
             }
 #pragma unroll
@@ -1047,22 +1050,22 @@ __global__ void __launch_bounds__(CGF_THREADS, 2) chunk_grad_f32_kernel(BwdParam
                 if (g == 0) sRow[m * 64 + t] = u, sDRr[m * 64 + t] = v, sDRi[m * 64 + t] = z;
             }
 #pragma unroll
-            for (int k = 0; k < 4; ++k) xr[k] = gre(acc[k]), xi[k] = gim(acc[k]);
+            for (int k = 0; k < 4; ++k) xr[k] = acc[k].re, xi[k] = acc[k].im;
         } else {
             // X[t][s] = A[t] . conj(B[s]) times D~ (or its conjugate), t = 16 tt + 4 g + r, lane s = own,
             // then acc^T[.][s] += C[t][.] conj(X[t][s])
             const auto side = [&](const float2 *A, const float2 *B, const float2 *Cx, float conj) {
 #pragma unroll 1
                 for (int tt = w; tt <= last; ++tt) {
-                    Gauss x;
-                    gz(x);
+                    Plain x;
+                    pz(x);
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
                         const Four u = row4(A, 16 * tt + l16, 16 * k + 4 * g), v = row4(B, own, 16 * k + 4 * g);
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) gstep(x, u.re[r], u.im[r], v.re[r], -v.im[r]);
+                        for (int r = 0; r < 4; ++r) pstep_cb(x, u.re[r], u.im[r], v.re[r], v.im[r]);
                     }
-                    const floatx4 ur = gre(x), ui = gim(x);
+                    const floatx4 ur = x.re, ui = x.im;
                     floatx4 pr, pi;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
@@ -1083,16 +1086,16 @@ __global__ void __launch_bounds__(CGF_THREADS, 2) chunk_grad_f32_kernel(BwdParam
 #pragma unroll
                         for (int it = 0; it < 4; ++it) {
                             const float2 e = Cx[(16 * tt + 4 * g + r) * CP + 16 * it + l16];
-                            gstep(acc[it], e.x, e.y, pr[r], -pi[r]);
+                            pstep_cb(acc[it], e.x, e.y, pr[r], pi[r]);
                         }
                 }
             };
             side(sQ, sK, sY, 1.f);  // A = W D~, dV = A^H dY
 #pragma unroll
-            for (int k = 0; k < 4; ++k) xr[k] = gre(acc[k]), xi[k] = gim(acc[k]), gz(acc[k]);
+            for (int k = 0; k < 4; ++k) xr[k] = acc[k].re, xi[k] = acc[k].im, pz(acc[k]);
             side(sY, sV, sQ, -1.f);  // gW = dA conj(D~), dK = gW^H Q~
 #pragma unroll
-            for (int k = 0; k < 4; ++k) yr[k] = gre(acc[k]), yi[k] = gim(acc[k]);
+            for (int k = 0; k < 4; ++k) yr[k] = acc[k].re, yi[k] = acc[k].im;
         }
     }
 
@@ -1119,7 +1122,7 @@ __global__ void __launch_bounds__(CGF_THREADS, 2) chunk_grad_f32_kernel(BwdParam
         __syncthreads();
         if (!active) continue;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) gz(acc[k]);
+        for (int k = 0; k < 4; ++k) pz(acc[k]);
         // acc^T[j][own] = sum_i conj(A[i][j]) row[i]
         const auto columns = [&](const float2 *A) {
 #pragma unroll
@@ -1129,7 +1132,7 @@ __global__ void __launch_bounds__(CGF_THREADS, 2) chunk_grad_f32_kernel(BwdParam
 #pragma unroll
                     for (int jt = 0; jt < 4; ++jt) {
                         const float2 e = A[(16 * k + 4 * g + r) * CP + 16 * jt + l16];
-                        gstep(acc[jt], e.x, -e.y, row[k].re[r], row[k].im[r]);
+                        pstep_ca(acc[jt], e.x, e.y, row[k].re[r], row[k].im[r]);
                     }
         };
         if (qside) {
@@ -1140,7 +1143,7 @@ __global__ void __launch_bounds__(CGF_THREADS, 2) chunk_grad_f32_kernel(BwdParam
             float pr = 0.f, pi = 0.f;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const floatx4 ur = gre(acc[k]), ui = gim(acc[k]);
+                const floatx4 ur = acc[k].re, ui = acc[k].im;
                 const Four q = row4(sQ, own, 16 * k + 4 * g);
                 xr[k] += rhr * ur + rhi * ui;
                 xi[k] += rhr * ui - rhi * ur;
@@ -1162,7 +1165,7 @@ __global__ void __launch_bounds__(CGF_THREADS, 2) chunk_grad_f32_kernel(BwdParam
             const float dl = own < valid ? __expf(fminf(lx, 0.f)) : 0.f;
             columns(sY);  // dK += dl V conj(G')
 #pragma unroll
-            for (int k = 0; k < 4; ++k) yr[k] += dl * gre(acc[k]), yi[k] += dl * gim(acc[k]), gz(acc[k]);
+            for (int k = 0; k < 4; ++k) yr[k] += dl * acc[k].re, yi[k] += dl * acc[k].im, pz(acc[k]);
 #pragma unroll
             for (int k = 0; k < 4; ++k) {  // Z = K G'^T; dV += dl Z; gdl = Re<V, Z>
                 const Four kk = row4(sK, own, 16 * k + 4 * g);
@@ -1170,13 +1173,13 @@ __global__ void __launch_bounds__(CGF_THREADS, 2) chunk_grad_f32_kernel(BwdParam
                 for (int it = 0; it < 4; ++it) {
                     const Four gg = row4(sY, 16 * it + l16, 16 * k + 4 * g);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) gstep(acc[it], gg.re[r], gg.im[r], kk.re[r], kk.im[r]);
+                    for (int r = 0; r < 4; ++r) pstep(acc[it], gg.re[r], gg.im[r], kk.re[r], kk.im[r]);
                 }
             }
             float gdl = 0.f;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const floatx4 zr = gre(acc[k]), zi = gim(acc[k]);
+                const floatx4 zr = acc[k].re, zi = acc[k].im;
                 xr[k] += dl * zr;
                 xi[k] += dl * zi;
 #pragma unroll

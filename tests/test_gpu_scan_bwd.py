@@ -371,22 +371,11 @@ def test_scan_backward_deterministic(gpu_lib, dtype, M, T, C):
             assert torch.equal(a, b), f"{name}: differs between two runs"
 
 
-@pytest.mark.parametrize("M,T,with_rot,with_s0", [
-    (1, 1, False, False), (1, 1, False, True),      # one step, without and with a state to carry
-    (2, 15, True, False), (3, 17, True, True),      # around a tile of 16 steps
-    (4, 63, True, True), (1, 64, False, False), (4, 65, True, False),  # around a chunk
-    (2, 16 * 7, True, True), (1, 64 * 3 + 33, False, True),
-])
-def test_fused_chunk_grad_equals_query_and_key_kernels(gpu_lib, monkeypatch, M, T, with_rot, with_s0):
-    """fp32 with 64-step chunks: gradient planes with 16-byte rows take one fused
-    kernel, others the query-side and key-side kernels.  The same pass over planes
-    with rows of 65 elements gives the same gradients within rounding: a gradient
-    chains three sums of at most 128 terms, each kernel within 3 * 128 * 2^-24 of
-    the exact value in norm."""
+def _query_and_key_grads(monkeypatch, case, d, with_rot):
+    """fp32, 64-step chunks: the gradients written into planes with rows of 65
+    elements, which the query-side and key-side kernels take (planes with 16-byte
+    rows take one fused kernel)."""
     from qllm2_amd import pam_scan
-    B, H, d = 2, 3, 64
-    case = _case(M, B, H, T, d, 7000 + 10 * M + T, with_rot, with_s0, torch.float32)
-    fused = _gpu_grads(*case, d, 64, torch.float32, with_rot)
     mview, run = pam_scan._mview, pam_scan._scan_bwd
     pads = []
 
@@ -403,8 +392,52 @@ def test_fused_chunk_grad_equals_query_and_key_kernels(gpu_lib, monkeypatch, M, 
         return out
 
     monkeypatch.setattr(pam_scan, "_scan_bwd", padded_bwd)
-    general = _gpu_grads(*case, d, 64, torch.float32, with_rot)
+    grads = _gpu_grads(*case, d, 64, torch.float32, with_rot)
     assert pads
+    return grads
+
+
+@pytest.mark.parametrize("M,T,with_rot,with_s0", [
+    (1, 1, False, False), (1, 1, False, True),      # one step, without and with a state to carry
+    (2, 15, True, False), (3, 17, True, True),      # around a tile of 16 steps
+    (4, 63, True, True), (1, 64, False, False), (4, 65, True, False),  # around a chunk
+    (2, 16 * 7, True, True), (1, 64 * 3 + 33, False, True),
+])
+def test_fused_chunk_grad_equals_query_and_key_kernels(gpu_lib, monkeypatch, M, T, with_rot, with_s0):
+    """fp32 with 64-step chunks: gradient planes with 16-byte rows take one fused
+    kernel, others the query-side and key-side kernels.  The same pass over planes
+    with rows of 65 elements gives the same gradients within rounding: a gradient
+    chains three sums of at most 128 terms, each kernel within 3 * 128 * 2^-24 of
+    the exact value in norm."""
+    B, H, d = 2, 3, 64
+    case = _case(M, B, H, T, d, 7000 + 10 * M + T, with_rot, with_s0, torch.float32)
+    fused = _gpu_grads(*case, d, 64, torch.float32, with_rot)
+    general = _query_and_key_grads(monkeypatch, case, d, with_rot)
     for name, a, b in zip(NAMES, fused, general):
         if a is not None:
             assert float((a - b).norm()) <= 2 * 3 * 128 * 2.0 ** -24 * float(b.norm()), name
+
+
+@pytest.mark.parametrize("M,T,with_rot,with_s0", [(1, 640, False, False), (1, 200, False, True), (2, 300, True, True),
+                                                  (4, 200, True, False)])
+def test_fused_chunk_grad_is_as_exact_as_the_query_and_key_kernels(gpu_lib, monkeypatch, M, T, with_rot, with_s0):
+    """Each plane's distance from 64 bits, the fused kernel's against the query-side
+    and key-side kernels', which sum every real product of a complex one on its own:
+    no larger, but for the chance by which two norms of n independent errors of one
+    size differ, three deviations of 1 / sqrt(n).  n is the plane's 2 * 3 * T * 64
+    elements for dq, dk and dv, and one per state, head and chunk for dgamma (a sum
+    from the chunk's end: the errors of its steps are not independent)."""
+    B, H, d = 2, 3, 64
+    case = _case(M, B, H, T, d, 7500 + 10 * M + T, with_rot, with_s0, torch.float32)
+    ref = _oracle_grads(*case, d, 64)
+    fused = _gpu_grads(*case, d, 64, torch.float32, with_rot)
+    general = _query_and_key_grads(monkeypatch, case, d, with_rot)
+    worse = []
+    for name, a, b, r in list(zip(NAMES, fused, general, ref))[:4]:
+        n = 6 * T * 64 if name != "dgamma" else M * 6 * -(-T // 64)
+        for i in (0, 1) if name != "dgamma" else (Ellipsis,):
+            new, old = (float((x[..., i].double() - r[..., i]).norm() / r[..., i].norm()) for x in (a, b))
+            print(f"M={M} T={T} {name}[{i}]: fused {new:.3e} separate {old:.3e} ratio {new / old:.3f}", flush=True)
+            if new > (1 + 3 * n ** -0.5) * old:
+                worse.append((name, i, new / old))
+    assert not worse, worse
