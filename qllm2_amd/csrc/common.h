@@ -102,6 +102,15 @@ __device__ __forceinline__ unsigned pack_bf16x2(float lo, float hi) {
     return __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{lo, hi}, bf16x2));
 }
 
+// Orders a wave's earlier LDS accesses before its later ones for data passed between its
+// lanes.  The hardware runs one wave's LDS accesses in order; the fences tell the compiler
+// (a wave barrier alone only stops it from moving instructions across).
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // DPP lane permutations (quad_perm [1,0,3,2], [2,3,0,1], row_half_mirror,
 // row_mirror) and reductions over the 16 lanes of a DPP row: every lane of the
 // row ends with the result.  Four steps: pairs, quads, halves, rows.

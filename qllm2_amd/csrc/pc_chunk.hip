@@ -244,12 +244,13 @@ __global__ void __launch_bounds__(OUT_THREADS, 2) pc_output_kernel(qpam_pc_args 
 #pragma unroll
         for (int r = 0; r < OUT_ROWS; ++r)
             sX[p.row(r) * CP + p.j] = keep(p.ok(r), widen(xq[r], a.dtype), __expf(fmaxf(cs[r], CUM_FLOOR)) * a.q_scale);
-        // a wave stages exactly the rows it reads: no barrier before, one before K takes the tile
+        // a wave stages exactly the rows it reads: its own LDS order before and after the reads,
+        // and the block's barrier once K has taken the tile
         static_assert(OUT_ROWS == 16, "a wave's staged rows are its query tile");
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_order();
 #pragma unroll
         for (int k = 0; k < DT; ++k) q[k] = row4(sX, t, 16 * k + 4 * g);
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_order();
 #pragma unroll
         for (int r = 0; r < OUT_ROWS; ++r)
             sX[p.row(r) * CP + p.j] = keep(p.ok(r), widen(xk[r], a.dtype), __expf(-fmaxf(cs[r], CUM_FLOOR)));
