@@ -8,12 +8,17 @@
 // passes through HBM between the launches:
 //   forward:  pc_state (increments V^T conj(W)) -> qpam_pc_scan -> pc_output
 //   backward: pc_state (increments dY^T conj(Qf)) -> qpam_pc_scan in reverse -> pc_grad
-// At B=8, H=12, T=2048, d=64, chunk 64 (fp32) a training step takes 1.02 ms (was
+// At B=8, H=12, T=2048, d=64, chunk 64 (fp32) a training step takes 1.04 ms (was
 // 2.64 ms: twelve batched library products whose operands and results each crossed
 // HBM, 1.36 ms, the fold kernels, 0.41 ms, and conjugations, transposes, masks and
-// sums).  Four-product complex MFMAs in place of Gauss's three cost 4 %: the
-// kernels are bound by each block's load, product and store phases following one
-// another at one to three blocks per CU, not by the matrix cores.
+// sums).  The kernels are bound by each block's load, product and store phases
+// following one another at one to three blocks per CU, more than by the matrix cores.
+// Precision: every real part of a product is summed on its own (gauss.h, Plain).  With
+// three MFMAs per product, e^{L} and e^{-L} by __expf, and W formed as Kf E, the step
+// took 1.01 ms, but the imaginary planes of y, s, dk and dv were 1.03-1.31 times as far
+// from 64 bits as the library products' (now 0.80-1.02, within chance), and prefixes
+// near -30 cost dk and dv 1.12-1.14 in both planes: expf where both e^{L} and e^{-L}
+// enter a result, W by its own exponential.
 //
 // Tiles are staged by lane = column, so a wave's access to a row is one 512-byte run.
 #include "gauss.h"
@@ -143,8 +148,8 @@ __device__ __forceinline__ float prefix(const Pos<ROWS> &p, const float (&gam)[R
 // chunk's column decays E) in the forward, A = dY, B = Qf in the backward.  A block
 // of 4 waves per (chain, chunk), wave w rows 16 w.. of X.  HBM-bound: reads two
 // tensors and gamma, writes the increments.  The rows pass through LDS in two
-// halves (36 KB): three blocks per CU, whose loads and products overlap (88 us =
-// 4.0 TB/s at the shape above; 98 us with whole tiles, two blocks per CU).
+// halves (36 KB): three blocks per CU, whose loads and products overlap (104 us =
+// 3.4 TB/s at the shape above; 92 us with three MFMAs per product).
 constexpr int ST_THREADS = 256, ST_ROWS = CH * 64 / ST_THREADS, ST_HALF = CH / 2;
 constexpr size_t ST_SMEM = 2 * ST_HALF * CP * sizeof(float2) + (4 + 1) * CH * sizeof(float);
 
@@ -168,9 +173,9 @@ __global__ void __launch_bounds__(ST_THREADS, 3) pc_state_kernel(qpam_pc_args a,
     const float Llast = prefix<ST_ROWS>(p, gam, a.g_dtype, cs, sTot, sLast);
     if (!BWD && p.grp == 0 && p.jv) a.atot[p.cc * a.d + p.j] = __expf(Llast);
     const int w = p.grp, lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
-    Gauss x[DT];
+    Plain x[DT];
 #pragma unroll
-    for (int jt = 0; jt < DT; ++jt) gz(x[jt]);
+    for (int jt = 0; jt < DT; ++jt) pz(x[jt]);
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
         if (ST_HALF * half >= p.valid) break;  // rows past the chunk are zero
@@ -194,7 +199,7 @@ __global__ void __launch_bounds__(ST_THREADS, 3) pc_state_kernel(qpam_pc_args a,
 #pragma unroll
                 for (int jt = 0; jt < DT; ++jt) {
                     const float2 v = sB[t * CP + 16 * jt + l16];
-                    gstep(x[jt], u.x, u.y, v.x, -v.y);
+                    pstep_cb(x[jt], u.x, u.y, v.x, v.y);
                 }
             }
         }
@@ -203,7 +208,7 @@ __global__ void __launch_bounds__(ST_THREADS, 3) pc_state_kernel(qpam_pc_args a,
     float *dst = a.x + p.cc * a.d * a.d * 2;
 #pragma unroll
     for (int jt = 0; jt < DT; ++jt) {
-        const floatx4 re = gre(x[jt]), im = gim(x[jt]);
+        const floatx4 re = x[jt].re, im = x[jt].im;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int i = 16 * w + 4 * g + r, j = 16 * jt + l16;
@@ -218,8 +223,8 @@ __global__ void __launch_bounds__(ST_THREADS, 3) pc_state_kernel(qpam_pc_args a,
 // and one LDS tile holds Qf, then Kf, V and S, which wait in registers (36 KB: the
 // registers set the blocks per CU).  The carried read is summed apart from the
 // chunk's own and added once: one 128-term chain of fp32 sums is 1.4 x less exact
-// (relative error of y against float64 3.9e-7, apart 2.9e-7).  190 us for 550 MB and
-// 11 GFLOP issued.
+// (relative error of y against float64 3.9e-7, apart 2.6e-7).  215 us for 550 MB and
+// 15 GFLOP issued (202 us with three MFMAs per product and __expf).
 constexpr int OUT_THREADS = 256, OUT_ROWS = CH * 64 / OUT_THREADS;
 constexpr size_t OUT_SMEM = TILE * sizeof(float2) + (4 + 1) * CH * sizeof(float);
 
@@ -243,7 +248,7 @@ __global__ void __launch_bounds__(OUT_THREADS, 2) pc_output_kernel(qpam_pc_args 
         prefix<OUT_ROWS>(p, gam, a.g_dtype, cs, sTot, sLast);
 #pragma unroll
         for (int r = 0; r < OUT_ROWS; ++r)
-            sX[p.row(r) * CP + p.j] = keep(p.ok(r), widen(xq[r], a.dtype), __expf(fmaxf(cs[r], CUM_FLOOR)) * a.q_scale);
+            sX[p.row(r) * CP + p.j] = keep(p.ok(r), widen(xq[r], a.dtype), expf(fmaxf(cs[r], CUM_FLOOR)) * a.q_scale);
         // a wave stages exactly the rows it reads: its own LDS order before and after the reads,
         // and the block's barrier once K has taken the tile
         static_assert(OUT_ROWS == 16, "a wave's staged rows are its query tile");
@@ -253,7 +258,7 @@ __global__ void __launch_bounds__(OUT_THREADS, 2) pc_output_kernel(qpam_pc_args 
         wave_lds_order();
 #pragma unroll
         for (int r = 0; r < OUT_ROWS; ++r)
-            sX[p.row(r) * CP + p.j] = keep(p.ok(r), widen(xk[r], a.dtype), __expf(-fmaxf(cs[r], CUM_FLOOR)));
+            sX[p.row(r) * CP + p.j] = keep(p.ok(r), widen(xk[r], a.dtype), expf(-fmaxf(cs[r], CUM_FLOOR)));
     }
     __syncthreads();
 
@@ -262,16 +267,16 @@ __global__ void __launch_bounds__(OUT_THREADS, 2) pc_output_kernel(qpam_pc_args 
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
             if (st > w) continue;
-            Gauss x;  // sum_j conj(K[s][j]) Q[t][j]
-            gz(x);
+            Plain x;  // sum_j conj(K[s][j]) Q[t][j]
+            pz(x);
 #pragma unroll
             for (int k = 0; k < DT; ++k) {
                 const Four kk = row4(sX, 16 * st + l16, 16 * k + 4 * g);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) gstep(x, kk.re[r], -kk.im[r], q[k].re[r], q[k].im[r]);
+                for (int r = 0; r < 4; ++r) pstep_ca(x, kk.re[r], kk.im[r], q[k].re[r], q[k].im[r]);
             }
-            pr[st] = gre(x);
-            pi[st] = gim(x);
+            pr[st] = x.re;
+            pi[st] = x.im;
             if (st == w) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
@@ -288,9 +293,9 @@ __global__ void __launch_bounds__(OUT_THREADS, 2) pc_output_kernel(qpam_pc_args 
     for (int r = 0; r < OUT_ROWS; ++r) sX[p.row(r) * CP + p.j] = keep(p.ok(r), widen(xv[r], a.v_dtype));
     __syncthreads();
 
-    Gauss y[DT];
+    Plain y[DT];
 #pragma unroll
-    for (int it = 0; it < DT; ++it) gz(y[it]);
+    for (int it = 0; it < DT; ++it) pz(y[it]);
     if (active) {
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
@@ -300,13 +305,13 @@ __global__ void __launch_bounds__(OUT_THREADS, 2) pc_output_kernel(qpam_pc_args 
 #pragma unroll
                 for (int it = 0; it < DT; ++it) {
                     const float2 v = sX[(16 * st + 4 * g + r) * CP + 16 * it + l16];
-                    gstep(y[it], pr[st][r], pi[st][r], v.x, v.y);
+                    pstep(y[it], pr[st][r], pi[st][r], v.x, v.y);
                 }
         }
     }
     floatx4 yr[DT], yi[DT];
 #pragma unroll
-    for (int it = 0; it < DT; ++it) yr[it] = gre(y[it]), yi[it] = gim(y[it]);
+    for (int it = 0; it < DT; ++it) yr[it] = y[it].re, yi[it] = y[it].im;
     if (carry) {
         __syncthreads();
 #pragma unroll
@@ -314,17 +319,17 @@ __global__ void __launch_bounds__(OUT_THREADS, 2) pc_output_kernel(qpam_pc_args 
         __syncthreads();
         if (active) {
 #pragma unroll
-            for (int it = 0; it < DT; ++it) gz(y[it]);
+            for (int it = 0; it < DT; ++it) pz(y[it]);
 #pragma unroll
             for (int k = 0; k < DT; ++k)
 #pragma unroll
                 for (int it = 0; it < DT; ++it) {
                     const Four s = row4(sX, 16 * it + l16, 16 * k + 4 * g);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) gstep(y[it], q[k].re[r], q[k].im[r], s.re[r], s.im[r]);
+                    for (int r = 0; r < 4; ++r) pstep(y[it], q[k].re[r], q[k].im[r], s.re[r], s.im[r]);
                 }
 #pragma unroll
-            for (int it = 0; it < DT; ++it) yr[it] += gre(y[it]), yi[it] += gim(y[it]);
+            for (int it = 0; it < DT; ++it) yr[it] += y[it].re, yi[it] += y[it].im;
         }
     }
     if (!active) return;
@@ -345,18 +350,17 @@ __global__ void __launch_bounds__(OUT_THREADS, 2) pc_output_kernel(qpam_pc_args 
 // LDS (148 KB, one block per CU).  Waves 0-3 take query tile w, waves 4-7 key tile
 // w; a SIMD holds one of each, so its causal work does not depend on w:
 //   query: dP = tril(dY V^H), dQ = dP Kf + dY conj(S), and of key tile w
-//          dK2 = V conj(G'),
-//   key:   P, dP, dV = P^H dY + Kf G'^T, dK1 = dP^H Qf,
-// with S the entering state, G the gradient of the state after the chunk and
-// G' = G E (column j scaled by E_j, which turns W = Kf E into Kf).  S and G' wait
-// in registers and take V's and dY's tiles after the score products.  The four
-// results replace the tiles, and each lane finishes its own channel and
-// steps as the fold's backward: dq = dQ e^{L} q_scale, dk = (dK1 + dK2) e^{-L},
-//   dL_t = Re(conj(Qf) dQ) - Re(conj(Kf) (dK1 + dK2)),
-//   dL_last += sum_t Re(conj(Kf) dK2) + sum_i Re(conj(S) G'),
+//          dK2 = V conj(G),
+//   key:   P, dP, dV = P^H dY + W G^T, dK1 = dP^H Qf,
+// with S the entering state and G the gradient of the state after the chunk, which
+// wait in registers and take V's and dY's tiles after the score products, W then Kf's.
+// The four results replace the tiles, and each lane finishes its own channel and
+// steps as the fold's backward: dq = dQ e^{L} q_scale, dk = dK1 e^{-L} + dK2 e^{L_last - L},
+//   dL_t = Re(conj(Qf) dQ) - Re(conj(Kf) dK1) - Re(conj(W) dK2),
+//   dL_last += sum_t Re(conj(W) dK2) + E sum_i Re(conj(S) G),
 // masked where the prefix sat below -30, summed from the chunk's end and divided
-// by gamma where gamma >= 1e-6.  All sums run in a fixed order.  582 us for 1.0 GB
-// and 30 GFLOP issued.
+// by gamma where gamma >= 1e-6.  All sums run in a fixed order.  647 us for 1.0 GB
+// and 40 GFLOP issued (604 us with three MFMAs per product, G scaled by E and Kf in W's place).
 constexpr int GR_THREADS = 512, GR_ROWS = CH * 64 / GR_THREADS, GR_GROUPS = GR_THREADS / 64;
 constexpr size_t GR_SMEM = 4 * TILE * sizeof(float2) + (3 * GR_GROUPS + 1) * CH * sizeof(float);
 
@@ -380,7 +384,7 @@ __global__ void __launch_bounds__(GR_THREADS, 2) pc_grad_kernel(qpam_pc_args a, 
         Llast = prefix<GR_ROWS>(p, gam, a.g_dtype, cs, sTot, sLast);
 #pragma unroll
         for (int r = 0; r < GR_ROWS; ++r) {
-            const float L = fmaxf(cs[r], CUM_FLOOR), al = __expf(L) * a.q_scale, be = __expf(-L);
+            const float L = fmaxf(cs[r], CUM_FLOOR), al = expf(L) * a.q_scale, be = expf(-L);
             const int o = p.row(r) * CP + p.j;
             sQ[o] = keep(p.ok(r), widen(xq[r], a.dtype), al);
             sK[o] = keep(p.ok(r), widen(xk[r], a.dtype), be);
@@ -396,11 +400,11 @@ __global__ void __launch_bounds__(GR_THREADS, 2) pc_grad_kernel(qpam_pc_args a, 
     const int w = p.grp & 3, lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4, own = 16 * w + l16;
     const bool qside = p.grp < 4, active = 16 * w < p.valid;
     const int last = (p.valid - 1) >> 4;  // last row tile with steps
-    Four own_a[DT], own_v[DT];  // query: the dY and V rows of step `own`; key: its Kf row (own_a)
+    Four own_a[DT], own_v[DT];  // query: the dY and V rows of step `own`; key (own_a): its rows of K and V, then of W
     floatx4 vr[DT], vi[DT];  // key: dV; query (later): dK2
-    Gauss acc[DT];           // the chunk's own dQ (query) or dK1 (key)
+    Plain acc[DT];           // the chunk's own dQ (query) or dK1 (key)
 #pragma unroll
-    for (int k = 0; k < DT; ++k) gz(acc[k]), vr[k] = vi[k] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < DT; ++k) pz(acc[k]), vr[k] = vi[k] = floatx4{0.f, 0.f, 0.f, 0.f};
     if (active) {
         if (qside) {
 #pragma unroll
@@ -408,15 +412,15 @@ __global__ void __launch_bounds__(GR_THREADS, 2) pc_grad_kernel(qpam_pc_args a, 
 #pragma unroll
             for (int st = 0; st < 4; ++st) {
                 if (st > w) continue;
-                Gauss x;  // dP[t][s], lane t = own, s = 16 st + 4 g + r
-                gz(x);
+                Plain x;  // dP[t][s], lane t = own, s = 16 st + 4 g + r
+                pz(x);
 #pragma unroll
                 for (int k = 0; k < DT; ++k) {
                     const Four v = row4(sV, 16 * st + l16, 16 * k + 4 * g);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) gstep(x, v.re[r], -v.im[r], own_a[k].re[r], own_a[k].im[r]);
+                    for (int r = 0; r < 4; ++r) pstep_ca(x, v.re[r], v.im[r], own_a[k].re[r], own_a[k].im[r]);
                 }
-                floatx4 re = gre(x), im = gim(x);
+                floatx4 re = x.re, im = x.im;
                 if (st == w) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
@@ -427,7 +431,7 @@ __global__ void __launch_bounds__(GR_THREADS, 2) pc_grad_kernel(qpam_pc_args a, 
 #pragma unroll
                     for (int jt = 0; jt < DT; ++jt) {
                         const float2 k = sK[(16 * st + 4 * g + r) * CP + 16 * jt + l16];
-                        gstep(acc[jt], k.x, k.y, re[r], im[r]);
+                        pstep(acc[jt], k.x, k.y, re[r], im[r]);
                     }
             }
 #pragma unroll
@@ -441,15 +445,15 @@ __global__ void __launch_bounds__(GR_THREADS, 2) pc_grad_kernel(qpam_pc_args a, 
 #pragma unroll
                 for (int tt = 0; tt < 4; ++tt) {
                     if (tt < w || tt > last) continue;
-                    Gauss x;
-                    gz(x);
+                    Plain x;
+                    pz(x);
 #pragma unroll
                     for (int k = 0; k < DT; ++k) {
                         const Four q = row4(A, 16 * tt + l16, 16 * k + 4 * g);
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) gstep(x, q.re[r], q.im[r], own_a[k].re[r], -own_a[k].im[r]);
+                        for (int r = 0; r < 4; ++r) pstep_cb(x, q.re[r], q.im[r], own_a[k].re[r], own_a[k].im[r]);
                     }
-                    floatx4 re = gre(x), im = gim(x);
+                    floatx4 re = x.re, im = x.im;
                     if (tt == w) {
 #pragma unroll
                         for (int r = 0; r < 4; ++r)
@@ -460,42 +464,51 @@ __global__ void __launch_bounds__(GR_THREADS, 2) pc_grad_kernel(qpam_pc_args a, 
 #pragma unroll
                         for (int it = 0; it < DT; ++it) {
                             const float2 d = C[(16 * tt + 4 * g + r) * CP + 16 * it + l16];
-                            gstep(acc[it], d.x, d.y, re[r], -im[r]);
+                            pstep_cb(acc[it], d.x, d.y, re[r], im[r]);
                         }
                 }
             };
             side(sQ, sK, sY);  // P, dV = P^H dY
 #pragma unroll
-            for (int k = 0; k < DT; ++k) vr[k] = gre(acc[k]), vi[k] = gim(acc[k]), gz(acc[k]);
+            for (int k = 0; k < DT; ++k) vr[k] = acc[k].re, vi[k] = acc[k].im, pz(acc[k]);
             side(sY, sV, sQ);  // dP, dK1 = dP^H Q
-#pragma unroll
-            for (int k = 0; k < DT; ++k) own_a[k] = row4(sK, own, 16 * k + 4 * g);
         }
     }
+    float2 kf[GR_ROWS];  // k of the lane's steps again (from the caches)
+    load_rows<GR_ROWS>(kf, p, a.k, p.at(a.k_sb, a.k_sh, a.k_st), a.k_st, a.dtype);
     __syncthreads();
-    // every tile is consumed: S and G' take V's and dY's, the chunk's own dQ and dK1
-    // Q's and K's; the carried products are summed apart and added (as in pc_output)
-    const float E = __expf(Llast);
-    float wpart = 0.f;  // sum_i Re(conj(S) G') of the lane's rows
+    // every tile is consumed: S, G and W take V's, dY's and K's, the chunk's own dQ and
+    // dK1 then Q's and W's; the carried products are summed apart and added (as in pc_output)
+    float wpart = 0.f;  // sum_i Re(conj(S) G) of the lane's rows
 #pragma unroll
     for (int r = 0; r < GR_ROWS; ++r) {
         const int o = p.row(r) * CP + p.j;
         const bool ok = p.jv && p.row(r) < a.d;
         xs[r] = keep(ok, xs[r]);
-        xg[r] = keep(ok, xg[r], E);
+        xg[r] = keep(ok, xg[r]);
         wpart += xs[r].x * xg[r].x + xs[r].y * xg[r].y;
         sV[o] = xs[r];
         sY[o] = xg[r];
+        sK[o] = keep(p.ok(r), widen(kf[r], a.dtype), __expf(Llast - fmaxf(cs[r], CUM_FLOOR)));
     }
+    wpart *= __expf(Llast);
+    if (qside) {
 #pragma unroll
-    for (int k = 0; k < DT; ++k) {
-        put4(qside ? sQ : sK, own, 16 * k + 4 * g, gre(acc[k]), gim(acc[k]));
-        gz(acc[k]);
+        for (int k = 0; k < DT; ++k) put4(sQ, own, 16 * k + 4 * g, acc[k].re, acc[k].im);
     }
     __syncthreads();
+    if (!qside) {  // a lane replaces only what it has read itself
+#pragma unroll
+        for (int k = 0; k < DT; ++k) {
+            own_a[k] = row4(sK, own, 16 * k + 4 * g);
+            put4(sK, own, 16 * k + 4 * g, acc[k].re, acc[k].im);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < DT; ++k) pz(acc[k]);
     if (active) {
         if (qside) {
-            // dQ^T[j][t] += conj(S[i][j]) dY[t][i], then dK2^T[j][s] = conj(G'[i][j]) V[s][i]
+            // dQ^T[j][t] += conj(S[i][j]) dY[t][i], then dK2^T[j][s] = conj(G[i][j]) V[s][i]
             const auto carried = [&](const float2 *m, const Four (&own_x)[DT]) {
 #pragma unroll
                 for (int k = 0; k < DT; ++k)
@@ -504,7 +517,7 @@ __global__ void __launch_bounds__(GR_THREADS, 2) pc_grad_kernel(qpam_pc_args a, 
 #pragma unroll
                         for (int jt = 0; jt < DT; ++jt) {
                             const float2 e = m[(16 * k + 4 * g + r) * CP + 16 * jt + l16];
-                            gstep(acc[jt], e.x, -e.y, own_x[k].re[r], own_x[k].im[r]);
+                            pstep_ca(acc[jt], e.x, e.y, own_x[k].re[r], own_x[k].im[r]);
                         }
             };
             carried(sV, own_a);
@@ -512,12 +525,12 @@ __global__ void __launch_bounds__(GR_THREADS, 2) pc_grad_kernel(qpam_pc_args a, 
             for (int k = 0; k < DT; ++k) {
                 const Four x = row4(sQ, own, 16 * k + 4 * g);
                 const floatx4 xr = {x.re[0], x.re[1], x.re[2], x.re[3]}, xi = {x.im[0], x.im[1], x.im[2], x.im[3]};
-                put4(sQ, own, 16 * k + 4 * g, xr + gre(acc[k]), xi + gim(acc[k]));
-                gz(acc[k]);
+                put4(sQ, own, 16 * k + 4 * g, xr + acc[k].re, xi + acc[k].im);
+                pz(acc[k]);
             }
             carried(sY, own_v);
 #pragma unroll
-            for (int k = 0; k < DT; ++k) vr[k] = gre(acc[k]), vi[k] = gim(acc[k]);
+            for (int k = 0; k < DT; ++k) vr[k] = acc[k].re, vi[k] = acc[k].im;
         } else {
 #pragma unroll
             for (int k = 0; k < DT; ++k)
@@ -525,19 +538,18 @@ __global__ void __launch_bounds__(GR_THREADS, 2) pc_grad_kernel(qpam_pc_args a, 
                 for (int it = 0; it < DT; ++it) {
                     const Four gg = row4(sY, 16 * it + l16, 16 * k + 4 * g);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r)  // dV^T[i][s] += G'[i][j] Kf[s][j]
-                        gstep(acc[it], gg.re[r], gg.im[r], own_a[k].re[r], own_a[k].im[r]);
+                    for (int r = 0; r < 4; ++r)  // dV^T[i][s] += G[i][j] W[s][j]
+                        pstep(acc[it], gg.re[r], gg.im[r], own_a[k].re[r], own_a[k].im[r]);
                 }
 #pragma unroll
-            for (int k = 0; k < DT; ++k) vr[k] += gre(acc[k]), vi[k] += gim(acc[k]);
+            for (int k = 0; k < DT; ++k) vr[k] += acc[k].re, vi[k] += acc[k].im;
         }
     }
-    // q, k and gamma of the lane's steps again (from the caches)
+    // and q and gamma
     float gam[GR_ROWS];
-    float2 qf[GR_ROWS], kf[GR_ROWS];
+    float2 qf[GR_ROWS];
     load_gamma<GR_ROWS>(gam, p, a);
     load_rows<GR_ROWS>(qf, p, a.q, p.at(a.q_sb, a.q_sh, a.q_st), a.q_st, a.dtype);
-    load_rows<GR_ROWS>(kf, p, a.k, p.at(a.k_sb, a.k_sh, a.k_st), a.k_st, a.dtype);
     __syncthreads();
     // dK2 -> sY (query waves), dV -> sV (key waves); inactive row tiles are never read
 #pragma unroll
@@ -552,13 +564,13 @@ __global__ void __launch_bounds__(GR_THREADS, 2) pc_grad_kernel(qpam_pc_args a, 
         if (!p.ok(r)) continue;
         const float2 dq = sQ[o], dk1 = sK[o], dk2 = sY[o], dv = sV[o];
         const float2 xq = widen(qf[r], a.dtype), xk = widen(kf[r], a.dtype);
-        const float2 dk = make_float2(dk1.x + dk2.x, dk1.y + dk2.y);
-        const float L = fmaxf(cs[r], CUM_FLOOR), al = __expf(L) * a.q_scale, be = __expf(-L);
-        dL[r] = al * (xq.x * dq.x + xq.y * dq.y) - be * (xk.x * dk.x + xk.y * dk.y);
-        wpart += be * (xk.x * dk2.x + xk.y * dk2.y);
+        const float L = fmaxf(cs[r], CUM_FLOOR), al = expf(L) * a.q_scale, be = expf(-L), ta = __expf(Llast - L);
+        const float wdk = ta * (xk.x * dk2.x + xk.y * dk2.y);
+        dL[r] = al * (xq.x * dq.x + xq.y * dq.y) - be * (xk.x * dk1.x + xk.y * dk1.y) - wdk;
+        wpart += wdk;
         const int64_t e = 2 * (oo + p.row(r) * a.d);
         st_c(a.dq, e, 2u * p.j, make_float2(dq.x * al, dq.y * al), a.dtype);
-        st_c(a.dk, e, 2u * p.j, make_float2(dk.x * be, dk.y * be), a.dtype);
+        st_c(a.dk, e, 2u * p.j, make_float2(dk1.x * be + dk2.x * ta, dk1.y * be + dk2.y * ta), a.dtype);
         st_c(a.dv, e, 2u * p.j, dv, a.v_dtype);
     }
     sW[p.grp * CH + p.j] = wpart;

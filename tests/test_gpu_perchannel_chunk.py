@@ -64,3 +64,46 @@ def test_chunk_kernels_equal_general_path(gpu_lib, monkeypatch, d, C, T, dtypes,
             terms = (q.float() * res[1][2].float()).abs().max() + (k.float() * res[1][3].float()).abs().max()
             top = max(top, (terms / gamma.float().min()).item())
         assert err <= tol * max(top, 1e-30), f"{name}: {err:.2e} of {top:.2e}"
+
+
+@pytest.mark.parametrize("d,C,T,shift", [(64, 64, 300, 3.0), (64, 64, 300, 0.0), (64, 16, 200, 3.0), (33, 33, 100, 5.0),
+                                         (16, 64, 200, 3.0)])
+def test_chunk_kernels_are_as_exact_as_the_general_path(gpu_lib, monkeypatch, d, C, T, shift):
+    """Each plane's distance from 64 bits, the chunk kernels' against the general
+    path's: no larger, but for chance.  With E the squared errors of the groups that
+    are independent of one another (an element, whose two parts share its factors;
+    for dgamma a channel's chunk, which is one running sum), a squared norm sum(E)
+    has a variance of at most sum(E^2), so two norms differ by a deviation of
+    (sum(E^2) / 2)^(1/2) / sum(E); three of them.  shift 0: prefixes past -30, where
+    the factors e^{L}, e^{-L} and e^{L_last - L} are far apart."""
+    from oracle import pam as O
+    from qllm2_amd import pam_perchannel as P
+    B, H = 2, 4
+    g = torch.Generator().manual_seed(10 * T + d)
+    q, k, v = (torch.randn(B, H, T, d, 2, generator=g) * (2 * d) ** -0.5 for _ in range(3))
+    gamma = torch.sigmoid(torch.randn(B, H, T, d, generator=g) + shift)
+    dy, ds = torch.randn(B, H, T, d, 2, generator=g), torch.randn(B, H, d, d, 2, generator=g)
+    ref = [x.double().requires_grad_(True) for x in (q, k, v, gamma)]
+    y, s = O.chunked_perchannel(*ref, d, C)
+    want = [y, s, *torch.autograd.grad((y, s), ref, (dy.double(), ds.double()))]
+    res = []
+    for limit in (64, 0):
+        monkeypatch.setattr(P, "KERNEL_D", limit)
+        leaves = [x.cuda().requires_grad_(True) for x in (q, k, v, gamma)]
+        y, s = P.perchannel_chunked(*leaves, d, C)
+        res.append([y, s, *torch.autograd.grad((y, s), leaves, (dy.cuda(), ds.cuda()))])
+    worse = []
+    for name, r, a, b in zip(("y", "s", "dq", "dk", "dv", "dgamma"), want, *res):
+        ea, eb = ((x.detach().double().cpu() - r.detach()) ** 2 for x in (a, b))
+        if name == "dgamma":
+            eb = torch.nn.functional.pad(eb, (0, 0, 0, -T % C)).unflatten(2, (-1, C))
+            E, parts = eb.sum(3), [(ea.sum(), eb.sum())]
+        else:
+            E, parts = eb.sum(-1), [(ea[..., i].sum(), eb[..., i].sum()) for i in (0, 1)]
+        slack = 3 * (((E ** 2).sum() / 2) ** 0.5 / E.sum()).item()
+        for i, (x, z) in enumerate(parts):
+            ratio = (x / z).sqrt().item()
+            print(f"d={d} C={C} T={T} {name}[{i}]: chunk kernels / general path {ratio:.3f}, slack {slack:.3f}", flush=True)
+            if ratio > 1 + slack:
+                worse.append((name, i, ratio, slack))
+    assert not worse, worse
