@@ -595,7 +595,8 @@ int qpam_pc_scan(const qpam_pc_scan_args *a, void *stream);
  * entering each chunk), fp32.  qpam_pc_bwd takes that x as s_in and atot, dy
  * (y's layout) and dfin (s_fin's, optional), uses x as its workspace (the state
  * gradients, same size) and writes dq, dk (dtype), dv (v_dtype) [B,H,T,d,2] and
- * dgamma (g_dtype) [B,H,T,d], contiguous. */
+ * dgamma (g_dtype) [B,H,T,d], contiguous.  Complex elements of all of these start
+ * on their own size too. */
 typedef struct {
     int32_t dtype, v_dtype, g_dtype, chunk;
     int64_t B, H, T, d;

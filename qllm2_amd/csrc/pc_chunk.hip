@@ -598,6 +598,9 @@ __global__ void __launch_bounds__(GR_THREADS, 2) pc_grad_kernel(qpam_pc_args a, 
     }
 }
 
+// complex elements are read and written whole: 8-byte (fp32) or 4-byte (bf16) accesses
+bool whole(const void *p, int dt) { return (uintptr_t)p % (dt == QPAM_BF16 ? 4 : 8) == 0; }
+
 int validate(const qpam_pc_args *a, const char *who) {
     QPAM_REQUIRE(a != nullptr, "%s: null args", who);
     QPAM_REQUIRE(a->B > 0 && a->H > 0 && a->T > 0, "%s: B, H, T must be positive", who);
@@ -609,13 +612,12 @@ int validate(const qpam_pc_args *a, const char *who) {
     QPAM_REQUIRE(a->B * a->H < (1ll << 31) && a->T < (1ll << 31) &&
                      a->B * a->H * ((a->T + a->chunk - 1) / a->chunk) < (1ll << 31),
                  "%s: grid too large", who);
-    // elements are read as pairs: 8-byte (fp32) or 4-byte (bf16) accesses
     const auto pairs = [](const void *p, int dt, int64_t s0, int64_t s1, int64_t s2) {
-        return ((s0 | s1 | s2) & 1) == 0 && (uintptr_t)p % (dt == QPAM_BF16 ? 4 : 8) == 0;
+        return ((s0 | s1 | s2) & 1) == 0 && whole(p, dt);
     };
     QPAM_REQUIRE(pairs(a->q, a->dtype, a->q_sb, a->q_sh, a->q_st) && pairs(a->k, a->dtype, a->k_sb, a->k_sh, a->k_st) &&
-                     pairs(a->v, a->v_dtype, a->v_sb, a->v_sh, a->v_st),
-                 "%s: complex elements of q, k and v must be aligned", who);
+                     pairs(a->v, a->v_dtype, a->v_sb, a->v_sh, a->v_st) && whole(a->x, QPAM_F32),
+                 "%s: complex elements of q, k, v and x must be aligned", who);
     return QPAM_OK;
 }
 
@@ -649,6 +651,8 @@ extern "C" int qpam_pc_fwd(const qpam_pc_args *a, void *stream) {
     int st = validate(a, "qpam_pc_fwd");
     if (st) return st;
     QPAM_REQUIRE(a->y && a->s_fin, "qpam_pc_fwd: y and s_fin are required");
+    QPAM_REQUIRE(whole(a->y, a->dtype) && whole(a->s_fin, QPAM_F32),
+                 "qpam_pc_fwd: complex elements of y and s_fin must be aligned");
     const int n = (int)((a->T + a->chunk - 1) / a->chunk);
     hipStream_t s = (hipStream_t)stream;
     st = a->d > 32 ? launch(pc_state_kernel<4, false>, ST_SMEM, ST_THREADS, *a, n, s, "pc_state_kernel")
@@ -665,6 +669,9 @@ extern "C" int qpam_pc_bwd(const qpam_pc_args *a, void *stream) {
     if (st) return st;
     QPAM_REQUIRE(a->s_in && a->dy && a->dq && a->dk && a->dv && a->dgamma,
                  "qpam_pc_bwd: s_in, dy, dq, dk, dv and dgamma are required");
+    QPAM_REQUIRE(whole(a->s_in, QPAM_F32) && whole(a->dy, a->dtype) && whole(a->dfin, QPAM_F32) && whole(a->dq, a->dtype) &&
+                     whole(a->dk, a->dtype) && whole(a->dv, a->v_dtype),
+                 "qpam_pc_bwd: complex elements of s_in, dy, dfin, dq, dk and dv must be aligned");
     const int n = (int)((a->T + a->chunk - 1) / a->chunk);
     hipStream_t s = (hipStream_t)stream;
     st = a->d > 32 ? launch(pc_state_kernel<4, true>, ST_SMEM, ST_THREADS, *a, n, s, "pc_state_kernel")

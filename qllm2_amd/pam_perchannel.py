@@ -56,6 +56,13 @@ def _pairs(x):
     return x if (x.stride(-1) == 1 and x.stride(-2) == 2) else x.contiguous()
 
 
+def _whole(x):
+    """x contiguous, its complex elements on their own alignment (a gradient may
+    be a contiguous view at an odd offset)."""
+    x = x.contiguous()
+    return x if x.data_ptr() % (2 * x.element_size()) == 0 else x.clone()
+
+
 def _ptr(t):
     return t.data_ptr() if t is not None else None
 
@@ -135,7 +142,7 @@ class _Fold(torch.autograd.Function):
         dq, dk = torch.empty(q.shape, device=q.device, dtype=q.dtype), torch.empty(k.shape, device=k.device,
                                                                                      dtype=q.dtype)
         dgamma = torch.empty(gamma.shape, device=gamma.device, dtype=gamma.dtype)
-        grads = [g.contiguous() if g is not None else None for g in (dqf, dkf, dwf, datot)]
+        grads = [_whole(g) if g is not None else None for g in (dqf, dkf, dwf, datot)]
         a = _Fold._args(q, k, gamma, ctx.chunk, ctx.q_scale)
         a.dqf, a.dkf, a.dwf, a.datot = (_ptr(g) for g in grads)
         a.dq, a.dk, a.dgamma = dq.data_ptr(), dk.data_ptr(), dgamma.data_ptr()
@@ -174,8 +181,8 @@ class _Scan(torch.autograd.Function):
     @_first_order
     def backward(ctx, dout, dfin):
         a, out = ctx.saved_tensors
-        dout = dout.contiguous() if dout is not None else torch.zeros_like(out)
-        dfin = dfin.contiguous() if dfin is not None else None
+        dout = _whole(dout) if dout is not None else torch.zeros_like(out)
+        dfin = _whole(dfin) if dfin is not None else None
         dx = torch.empty_like(out)
         _scan(dout, a, dx, dfin, None, True)
         # d a[c][j] = sum_i Re(conj(S_in[c][i][j]) dx[c][i][j])
@@ -232,8 +239,8 @@ class _Chunked(torch.autograd.Function):
     @_first_order
     def backward(ctx, dy, dfin):
         q, k, v, gamma, s_in, atot = ctx.saved_tensors
-        dy = dy.contiguous() if dy is not None else torch.zeros(q.shape, device=q.device, dtype=q.dtype)
-        dfin = dfin.contiguous() if dfin is not None else None
+        dy = _whole(dy) if dy is not None else torch.zeros(q.shape, device=q.device, dtype=q.dtype)
+        dfin = _whole(dfin) if dfin is not None else None
         dq, dk, dv, dgamma = (torch.empty(t.shape, device=t.device, dtype=t.dtype) for t in (q, k, v, gamma))
         ws = torch.empty_like(s_in)
         a = _Chunked._args(q, k, v, gamma, ctx.chunk, ctx.q_scale, ws, atot)

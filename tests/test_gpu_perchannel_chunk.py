@@ -107,3 +107,23 @@ def test_chunk_kernels_are_as_exact_as_the_general_path(gpu_lib, monkeypatch, d,
             if ratio > 1 + slack:
                 worse.append((name, i, ratio, slack))
     assert not worse, worse
+
+
+@pytest.mark.parametrize("d,dtype", [(64, torch.float32), (33, torch.bfloat16), (80, torch.float32)])
+def test_incoming_gradients_at_any_offset(gpu_lib, d, dtype):
+    """Contiguous gradients whose complex elements start between their alignments
+    give what aligned ones give, on the chunk kernels and on the general path."""
+    from qllm2_amd import pam_perchannel as P
+    print(f"case d={d} {dtype}", flush=True)
+    B, H, T, C = 1, 2, 70, 64
+    g = torch.Generator().manual_seed(d)
+    rn = lambda *s: torch.randn(*s, generator=g).cuda()  # noqa: E731
+    q, k, v = ((rn(B, H, T, d, 2) * (2 * d) ** -0.5).to(dtype).requires_grad_(True) for _ in range(3))
+    gamma = torch.sigmoid(rn(B, H, T, d) + 3).to(dtype).requires_grad_(True)
+    dy, ds = rn(B, H, T, d, 2).to(dtype), rn(B, H, d, d, 2).to(dtype)
+    got = []
+    for how in ("contiguous", "offset"):
+        y, s = P.perchannel_chunked(q, k, v, gamma, d, C)
+        got.append(torch.autograd.grad((y, s), (q, k, v, gamma), (_layout(dy, how), _layout(ds, how))))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)

@@ -60,3 +60,59 @@ def test_second_derivative_raises(stubbed, make, misaligned):
                 torch.autograd.grad((x * x).sum() + (g * g).sum(), x, retain_graph=True)
     plain = torch.autograd.grad(outs, leaves, gouts)
     assert all(g.grad_fn is None and g.shape == x.shape for g, x in zip(plain, leaves))
+
+
+def _offset(x):
+    """x's values in a contiguous view one element past an aligned start."""
+    buf = x.new_zeros(x.numel() + 1)
+    buf[1:] = x.reshape(-1)
+    return buf[1:].view(x.shape)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_incoming_gradients_reach_the_library_aligned(stubbed, monkeypatch, dtype):
+    """The kernels read dy and the state's gradient as whole complex elements."""
+    from qllm2_amd import _lib
+    seen = {}
+
+    class Lib:
+        def qpam_pc_fwd(self, a, s):
+            return 0
+
+        def qpam_pc_bwd(self, a, s):
+            seen.update(dy=a._obj.dy % (2 * dtype.itemsize), dfin=a._obj.dfin % 8)
+            return 0
+
+        def qpam_pc_scan(self, a, s):
+            seen.update(init=(a._obj.init or 0) % 8, x=a._obj.x % 8)
+            return 0
+
+    monkeypatch.setattr(_lib, "lib", lambda: Lib())
+    P = stubbed
+    q, k, v, g = (x.to(dtype).detach().requires_grad_(True) for x in _leaves(*[(1, 2, 5, 3, 2)] * 3, (1, 2, 5, 3)))
+    y, s = P._Chunked.apply(q, k, v, g, 4, 0.5)
+    torch.autograd.grad((y, s), (q, k, v, g), (_offset(torch.ones_like(y)), _offset(torch.ones_like(s))))
+    x, a = _leaves((2, 3, 4, 4, 2), (2, 3, 4))
+    out, fin = P._Scan.apply(x, a)
+    torch.autograd.grad((out, fin), (x, a), (_offset(torch.ones_like(out)), _offset(torch.ones_like(fin))))
+    assert seen == {"dy": 0, "dfin": 0, "init": 0, "x": 0}
+
+
+@pytest.mark.parametrize("entry,field", [("qpam_pc_fwd", f) for f in ("q", "k", "v", "x", "y", "s_fin")] +
+                         [("qpam_pc_bwd", f) for f in ("x", "s_in", "dy", "dfin", "dq", "dk", "dv")])
+@pytest.mark.parametrize("dtype", [0, 1])
+def test_library_refuses_split_complex_elements(entry, field, dtype):
+    """Refused on the host, before any launch (the addresses are never touched)."""
+    from qllm2_amd import _lib
+    a = _lib.PcArgs()
+    a.dtype = a.v_dtype = a.g_dtype = dtype
+    a.B, a.H, a.T, a.d, a.chunk, a.q_scale = 1, 2, 5, 3, 4, 0.5
+    for name in ("q", "k", "v"):
+        for ax, st in (("sb", 60), ("sh", 30), ("st", 6)):
+            setattr(a, f"{name}_{ax}", st)
+    a.g_sb, a.g_sh, a.g_st = 30, 15, 3
+    names = ("q", "k", "v", "gamma", "y", "x", "atot", "s_fin", "s_in", "dy", "dfin", "dq", "dk", "dv", "dgamma")
+    for i, name in enumerate(names):
+        setattr(a, name, 4096 * (i + 1) + ((2 if dtype and field not in ("x", "s_fin", "s_in", "dfin") else 4) if name == field else 0))
+    with pytest.raises(_lib.QpamError, match="aligned"):
+        _lib.check(getattr(_lib.lib(), entry)(a, None), entry)
