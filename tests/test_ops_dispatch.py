@@ -171,3 +171,75 @@ def test_refusals_match(what):
     assert raised[0] == raised[1], out
     if not raised[0] and out[0] is not None:
         assert torch.equal(out[0], out[1])
+
+
+def _scaled(a: Tensor, s: float = 2.0, k: int = 1) -> Tensor:
+    return a * (s * k)
+
+
+def _make(prefix, fn, name):
+    if prefix == "qpam":
+        return _ops.op(f"qpam::{name}")(fn)
+    return torch.library.custom_op(f"{prefix}::{name}", mutates_args=())(fn)
+
+
+@pytest.mark.parametrize("prefix", ["qpam", "qpam_ref"])
+def test_defaults_reach_the_formula(prefix):
+    """Arguments left (or equal) to their defaults, which the dispatcher drops."""
+    f = _make(prefix, _scaled, "t_scaled")
+    seen = []
+
+    def setup(ctx, inputs, output):
+        a, s, k = inputs
+        ctx.f = s * k
+        seen.append((s, k))
+
+    def back(ctx, g):
+        assert ctx.needs_input_grad[0] and not any(ctx.needs_input_grad[1:]) and len(ctx.needs_input_grad) <= 3
+        return g * ctx.f, None, None
+
+    f.register_autograd(back, setup_context=setup)
+    for args, kw, want in (((), {}, 2.0), ((3.0,), {}, 3.0), ((), {"k": 5}, 10.0), ((2.0, 1), {}, 2.0)):
+        a = torch.ones(2, requires_grad=True)
+        y = f(a, *args, **kw)
+        for _ in range(2):   # the second over the same context
+            assert torch.equal(torch.autograd.grad(y.sum(), a, retain_graph=True)[0], torch.full((2,), want))
+    assert seen == [(2.0, 1), (3.0, 1), (2.0, 5), (2.0, 1)]
+
+
+def _same(a: Tensor) -> Tensor:
+    return a
+
+
+def _beside(a: Tensor) -> List[Tensor]:
+    return [a * 1, a]
+
+
+@pytest.mark.parametrize("prefix", ["qpam", "qpam_ref"])
+@pytest.mark.parametrize("fn", [_same, _beside])
+@pytest.mark.parametrize("grad", [False, True])
+def test_outputs_that_are_inputs_are_refused(prefix, fn, grad):
+    f = _make(prefix, fn, f"t{fn.__name__}_{grad}")
+    with pytest.raises(RuntimeError):
+        f(torch.ones(3, requires_grad=grad))
+
+
+def _keyword(a: Tensor, *, s: float) -> Tensor:
+    return a * s
+
+
+def test_keyword_only_arguments_are_refused():
+    with pytest.raises(ValueError, match="keyword-only"):
+        _ops.op("qpam::t_keyword")(_keyword)
+
+
+def test_custom_op_where_a_private_name_is_missing(monkeypatch):
+    monkeypatch.setattr(_ops, "_NAMES", _ops._NAMES + ("no_such_name",))
+    f, bw, one = _wire(lambda n, fn: _ops.op(f"qpam::other_{n}")(fn))
+    assert not any(isinstance(x, _ops.Op) for x in (f, bw, one))
+    a, b = _leaves()
+    y = f(a, b, 1.5)
+    want = OURS[0](a, b, 1.5)
+    assert all(torch.equal(x, z) for x, z in zip(y, want))
+    got = torch.autograd.grad(y, (a, b), [torch.ones_like(x) for x in y])
+    assert all(torch.equal(x, z) for x, z in zip(got, torch.autograd.grad(want, (a, b), [torch.ones_like(x) for x in want])))
