@@ -27,6 +27,9 @@ namespace qpam {
 namespace {
 
 constexpr int CH = 64;                   // rows of a kernel chunk (steps past the chunk's are zero)
+// A grid holds at most 2^32 - 1 threads along an axis (one past it wraps without an
+// error): chunks beyond 2^20 go on along y, up to 65535 rows of them.
+constexpr int64_t GRID_X = 1 << 20;
 constexpr float GAMMA_FLOOR = 1e-6f;     // gamma.clamp_min(1e-6), v11/model.py:436
 constexpr float CUM_FLOOR = -30.f;       // cumsum.clamp(min=-30), v11/model.py:438
 
@@ -53,8 +56,12 @@ struct Pos {
     int64_t cc;  // chain * n + c
     int j, jc, grp, b, h, t0, valid;  // jc: j clamped into the channels
     bool jv;
+    // blocks past the last chunk (in the grid's last row of several) have nothing to do
+    __device__ __forceinline__ static bool past(const qpam_pc_args &a, int n) {
+        return (int64_t)blockIdx.y * GRID_X + blockIdx.x >= a.B * a.H * n;
+    }
     __device__ __forceinline__ Pos(const qpam_pc_args &a, int n) {
-        cc = blockIdx.x;
+        cc = (int64_t)blockIdx.y * GRID_X + blockIdx.x;
         j = threadIdx.x & 63;
         grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: scalar branches and row offsets
         const int c = (int)(cc % n);
@@ -158,6 +165,7 @@ __global__ void __launch_bounds__(ST_THREADS, 3) pc_state_kernel(qpam_pc_args a,
     extern __shared__ __align__(16) float2 smem[];
     float2 *sA = smem, *sB = sA + ST_HALF * CP;
     float *sTot = reinterpret_cast<float *>(sB + ST_HALF * CP), *sLast = sTot + 4 * CH;
+    if (Pos<ST_ROWS>::past(a, n)) return;
     const Pos<ST_ROWS> p(a, n);
     float2 xa[ST_ROWS], xb[ST_ROWS];
     float gam[ST_ROWS], cs[ST_ROWS];
@@ -233,6 +241,7 @@ __global__ void __launch_bounds__(OUT_THREADS, 2) pc_output_kernel(qpam_pc_args 
     extern __shared__ __align__(16) float2 smem[];
     float2 *sX = smem;
     float *sTot = reinterpret_cast<float *>(sX + TILE), *sLast = sTot + 4 * CH;
+    if (Pos<OUT_ROWS>::past(a, n)) return;
     const Pos<OUT_ROWS> p(a, n);
     const int w = p.grp, lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4, t = 16 * w + l16;
     const bool active = 16 * w < p.valid;
@@ -370,6 +379,7 @@ __global__ void __launch_bounds__(GR_THREADS, 2) pc_grad_kernel(qpam_pc_args a, 
     float2 *sQ = smem, *sK = sQ + TILE, *sV = sK + TILE, *sY = sV + TILE;
     float *sTot = reinterpret_cast<float *>(sY + TILE), *sW = sTot + GR_GROUPS * CH, *sD = sW + GR_GROUPS * CH,
           *sLast = sD + GR_GROUPS * CH;
+    if (Pos<GR_ROWS>::past(a, n)) return;
     const Pos<GR_ROWS> p(a, n);
     const int64_t so = (int64_t)a.T * a.d * 2;
     float cs[GR_ROWS], Llast;
@@ -624,7 +634,9 @@ int validate(const qpam_pc_args *a, const char *who) {
 template <typename K>
 int launch(K kernel, size_t smem, int threads, const qpam_pc_args &a, int n, hipStream_t s, const char *what) {
     QPAM_CHECK_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(a.B * a.H * n)), dim3(threads), smem, s, a, n);
+    const int64_t items = a.B * a.H * n;
+    const dim3 grid((unsigned)(items < GRID_X ? items : GRID_X), (unsigned)((items + GRID_X - 1) / GRID_X));
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), smem, s, a, n);
     return launch_status(what);
 }
 

@@ -150,3 +150,23 @@ def test_incoming_gradients_at_any_offset(gpu_lib, d, dtype):
         got.append(torch.autograd.grad((y, s), (q, k, v, gamma), (_layout(dy, how), _layout(ds, how))))
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+def test_more_chunks_than_one_grid_row_of_threads(gpu_lib):
+    """8.64 million chunks of one step: 2^32 threads and more in one row of 512-thread
+    blocks.  The result does not depend on the chunk length (prefixes stay far above
+    -30), so chunks of 64 steps are the reference; both sum at most 100 decayed terms
+    of weight (a sum of gamma^n below 1 / (1 - 0.9)) in fp32: 2e-5 of the largest."""
+    from qllm2_amd import pam_perchannel as P
+    B, H, T, d = 1, 96, 90000, 1
+    g = torch.Generator(device="cuda").manual_seed(0)
+    q, k, v = (torch.randn(B, H, T, d, 2, device="cuda", generator=g).requires_grad_(True) for _ in range(3))
+    gamma = (0.7 + 0.2 * torch.rand(B, H, T, d, device="cuda", generator=g)).requires_grad_(True)
+    dy = torch.randn(B, H, T, d, 2, device="cuda", generator=g)
+    res = []
+    for C in (1, 64):
+        print(f"chunk {C}: {B * H * -(-T // C)} chunks", flush=True)
+        y, s = P.perchannel_chunked(q, k, v, gamma, d, C)
+        res.append([y, s, *torch.autograd.grad(y, (q, k, v, gamma), dy)])
+    for name, a, b in zip(("y", "s", "dq", "dk", "dv", "dgamma"), *res):
+        assert (a - b).abs().max().item() <= 2e-5 * b.abs().max().item(), name
