@@ -368,17 +368,19 @@ __global__ void __launch_bounds__(OUT_THREADS, 2) pc_output_kernel(qpam_pc_args 
 //   dL_t = Re(conj(Qf) dQ) - Re(conj(Kf) dK1) - Re(conj(W) dK2),
 //   dL_last += sum_t Re(conj(W) dK2) + E sum_i Re(conj(S) G),
 // masked where the prefix sat below -30, summed from the chunk's end and divided
-// by gamma where gamma >= 1e-6.  All sums run in a fixed order.  647 us for 1.0 GB
+// by gamma where gamma >= 1e-6.  All sums run in a fixed order; those of dL, whose
+// terms cancel, in 64 bits (dgamma's distance from float64 0.96, in fp32 1.02 of that
+// with three-MFMA products; the step's time is the same).  647 us for 1.0 GB
 // and 40 GFLOP issued (604 us with three MFMAs per product, G scaled by E and Kf in W's place).
 constexpr int GR_THREADS = 512, GR_ROWS = CH * 64 / GR_THREADS, GR_GROUPS = GR_THREADS / 64;
-constexpr size_t GR_SMEM = 4 * TILE * sizeof(float2) + (3 * GR_GROUPS + 1) * CH * sizeof(float);
+constexpr size_t GR_SMEM = 4 * TILE * sizeof(float2) + (5 * GR_GROUPS + 1) * CH * sizeof(float);
 
 template <int DT>
 __global__ void __launch_bounds__(GR_THREADS, 2) pc_grad_kernel(qpam_pc_args a, int n) {
     extern __shared__ __align__(16) float2 smem[];
     float2 *sQ = smem, *sK = sQ + TILE, *sV = sK + TILE, *sY = sV + TILE;
-    float *sTot = reinterpret_cast<float *>(sY + TILE), *sW = sTot + GR_GROUPS * CH, *sD = sW + GR_GROUPS * CH,
-          *sLast = sD + GR_GROUPS * CH;
+    float *sTot = reinterpret_cast<float *>(sY + TILE), *sLast = sTot + GR_GROUPS * CH;
+    double *sW = reinterpret_cast<double *>(sLast + CH), *sD = sW + GR_GROUPS * CH;
     if (Pos<GR_ROWS>::past(a, n)) return;
     const Pos<GR_ROWS> p(a, n);
     const int64_t so = (int64_t)a.T * a.d * 2;
@@ -489,7 +491,7 @@ __global__ void __launch_bounds__(GR_THREADS, 2) pc_grad_kernel(qpam_pc_args a, 
     __syncthreads();
     // every tile is consumed: S, G and W take V's, dY's and K's, the chunk's own dQ and
     // dK1 then Q's and W's; the carried products are summed apart and added (as in pc_output)
-    float wpart = 0.f;  // sum_i Re(conj(S) G) of the lane's rows
+    double wpart = 0.;  // sum_i Re(conj(S) G) of the lane's rows
 #pragma unroll
     for (int r = 0; r < GR_ROWS; ++r) {
         const int o = p.row(r) * CP + p.j;
@@ -585,23 +587,23 @@ __global__ void __launch_bounds__(GR_THREADS, 2) pc_grad_kernel(qpam_pc_args a, 
     }
     sW[p.grp * CH + p.j] = wpart;
     __syncthreads();
-    float dlast = 0.f;
+    double dlast = 0.;
     for (int q = 0; q < GR_GROUPS; ++q) dlast += sW[q * CH + p.j];
-    float run = 0.f, suf[GR_ROWS];
+    double run = 0., suf[GR_ROWS];
 #pragma unroll
     for (int r = GR_ROWS - 1; r >= 0; --r) {
-        const float d = dL[r] + (p.row(r) == p.valid - 1 ? dlast : 0.f);
-        run += (p.ok(r) && cs[r] >= CUM_FLOOR) ? d : 0.f;
+        const double d = dL[r] + (p.row(r) == p.valid - 1 ? dlast : 0.);
+        run += (p.ok(r) && cs[r] >= CUM_FLOOR) ? d : 0.;
         suf[r] = run;
     }
     sD[p.grp * CH + p.j] = run;
     __syncthreads();
-    float later = 0.f;
+    double later = 0.;
     for (int q = GR_GROUPS - 1; q > p.grp; --q) later += sD[q * CH + p.j];
 #pragma unroll
     for (int r = 0; r < GR_ROWS; ++r) {
         if (!p.ok(r)) continue;
-        const float gv = widen(gam[r], a.g_dtype), v = gv >= GAMMA_FLOOR ? (suf[r] + later) / gv : 0.f;
+        const float gv = widen(gam[r], a.g_dtype), v = gv >= GAMMA_FLOOR ? (float)(suf[r] + later) / gv : 0.f;
         const int64_t e = oo + p.row(r) * a.d;
         if (a.g_dtype == QPAM_BF16) (static_cast<unsigned short *>(a.dgamma) + e)[(unsigned)p.j] = (unsigned short)pack_bf16x2(v, v);
         else (static_cast<float *>(a.dgamma) + e)[(unsigned)p.j] = v;
