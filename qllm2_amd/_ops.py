@@ -23,29 +23,20 @@ _LIB = torch.library.Library("qpam", "FRAGMENT")
 _CALL = threading.local()  # the dispatch keys of the call that is entering its autograd function
 
 
-def _fresh(name, fn):
-    """fn with a check that no output is one of its inputs: autograd and
-    functionalization take an operator's outputs for tensors of their own.
-    (custom_op looks for shared storage, views included, which costs a small call
-    3 us of its 75; that no operator here returns a view of an input is tested.)"""
-
-    def checked(*args):
-        out = fn(*args)
-        if not set(map(id, args)).isdisjoint(map(id, out if isinstance(out, list) else (out,))):
-            raise RuntimeError(f"{name}: an output is one of the inputs")
-        return out
-
-    return checked
-
-
-def _untraced(fn):
-    """fn kept out of torch.compile's tracing where it is called from a compiled
-    program; as it is while nothing has loaded the compiler (which the wrapper
-    would import on its first call)."""
+def _kernel(name, fn):
+    """fn as the operator's kernel.  It is kept out of torch.compile's tracing where it
+    is called from a compiled program, and is as it is while nothing has loaded the
+    compiler (which the wrapper would import on its first call).  No output may be one
+    of the inputs: autograd and functionalization take an operator's outputs for tensors
+    of their own.  (custom_op looks for shared storage, views included, which costs a
+    small call 3 us of its 75; that no operator here returns a view of an input is tested.)"""
     traced_off = torch._disable_dynamo(fn)
 
     def kernel(*args):
-        return fn(*args) if "torch._dynamo" not in sys.modules else traced_off(*args)
+        out = fn(*args) if "torch._dynamo" not in sys.modules else traced_off(*args)
+        if not {*map(id, args)}.isdisjoint(map(id, out if isinstance(out, list) else (out,))):
+            raise RuntimeError(f"{name}: an output is one of the inputs")
+        return out
 
     return kernel
 
@@ -64,7 +55,7 @@ class Op:
         if any(a.kwarg_only for a in arguments):
             raise ValueError(f"operator {name}: keyword-only arguments are not supported")
         self._defaults = [a.default_value for a in arguments]  # read past the arguments a call passes
-        _LIB.impl(self._name, _untraced(_fresh(name, fn)), "CompositeExplicitAutograd")
+        _LIB.impl(self._name, _kernel(name, fn), "CompositeExplicitAutograd")
         self._list = schema.rstrip().endswith("[]")
         self.__doc__, self.__name__ = fn.__doc__, fn.__name__
         self._autograd(None, None)
