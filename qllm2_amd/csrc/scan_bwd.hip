@@ -2205,8 +2205,9 @@ int launch_chunk_grad_f32(const BwdParams &p, hipStream_t stream) {
     return launch_status("chunk_grad_f32_kernel");
 }
 
-// chunk_grad_f32 stores gradient rows in 16-byte runs; other output layouts keep
-// the query and key sides as kernels of their own
+// chunk_grad_f32 stores gradient rows in 16-byte runs; other output layouts, which only
+// callers of the C interface have (pam_scan.py allocates its own planes), keep the query
+// and key sides as kernels of their own
 bool rows16(const qpam_mview &v) {
     return ((uintptr_t)v.re % 16) == 0 && (pairs(v) || ((uintptr_t)v.im % 16) == 0) && v.s0 % 4 == 0 && v.s1 % 4 == 0 &&
            v.s2 % 4 == 0;

@@ -12,8 +12,8 @@ Reference methods replaced (v11/model.py):
   _forward_chunked_perchannel 421-489 (E1 per-channel decay: HIP chunk kernels
                                       up to head dim 64; above, HIP fold and
                                       state scan around batched complex GEMMs)
-  _forward_delta            491-576  (E2 delta write; HIP token recurrence
-                                      instead of the per-chunk solve)
+  _forward_delta            491-576  (E2 delta write: the per-chunk solve on HIP
+                                      chunk kernels, both directions)
   _recur_step_delta         967-1002 (one E2 decode token)
 
   forward                   785-843  prefill of the production modes (head
