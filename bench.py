@@ -790,9 +790,8 @@ def _perchannel_reference_steps(q, k, v, gamma, d, chunk):
 
 def bench_perchannel(steps, warmup, reference=True):
     """E1 per-channel decay prefill forward + backward at the config-3 shape
-    (one state: B=8, T=2048, H=12, d=64, chunk 64, fp32): the HIP fold and
-    state-scan kernels around batched complex GEMMs against the reference's
-    per-chunk steps run in torch on the same GPU."""
+    (one state: B=8, T=2048, H=12, d=64, chunk 64, fp32): the HIP chunk kernels
+    against the reference's per-chunk steps run in torch on the same GPU."""
     import torch
     from qllm2_amd.pam_perchannel import perchannel_chunked
     B, H, T, d = 8, 12, 2048, 64
