@@ -170,3 +170,25 @@ def test_more_chunks_than_one_grid_row_of_threads(gpu_lib):
         res.append([y, s, *torch.autograd.grad(y, (q, k, v, gamma), dy)])
     for name, a, b in zip(("y", "s", "dq", "dk", "dv", "dgamma"), *res):
         assert (a - b).abs().max().item() <= 2e-5 * b.abs().max().item(), name
+
+
+@pytest.mark.parametrize("where", ["q", "k", "v", "dy", "ds"])
+def test_an_infinity_stays_in_its_part(gpu_lib, monkeypatch, where):
+    """No NaN where the general path has a number or an infinity."""
+    from qllm2_amd import pam_perchannel as P
+    print(f"case {where}", flush=True)
+    B, H, T, d, C = 1, 2, 150, 64, 64
+    g = torch.Generator().manual_seed(5)
+    x = {n: torch.randn(B, H, T, d, 2, generator=g) * (2 * d) ** -0.5 for n in ("q", "k", "v", "dy")}
+    x["ds"] = torch.randn(B, H, d, d, 2, generator=g)
+    x[where][(0, 1, 3, 4, 0) if where == "ds" else (0, 1, 70, 5, 0)] = float("inf")
+    gamma = torch.sigmoid(torch.randn(B, H, T, d, generator=g) + 2)
+    res = []
+    for limit in (64, 0):
+        monkeypatch.setattr(P, "KERNEL_D", limit)
+        leaves = [t.cuda().requires_grad_(True) for t in (x["q"], x["k"], x["v"], gamma)]
+        y, s = P.perchannel_chunked(*leaves, d, C)
+        res.append([y, s, *torch.autograd.grad((y, s), leaves, (x["dy"].cuda(), x["ds"].cuda()))])
+    assert any(not b.isfinite().all() for b in res[1])
+    for name, a, b in zip(("y", "s", "dq", "dk", "dv", "dgamma"), *res):
+        assert not (a.isnan() & ~b.isnan()).any(), name

@@ -441,3 +441,20 @@ def test_fused_chunk_grad_is_as_exact_as_the_query_and_key_kernels(gpu_lib, monk
             if new > (1 + 3 * n ** -0.5) * old:
                 worse.append((name, i, new / old))
     assert not worse, worse
+
+
+@pytest.mark.parametrize("where", ["q", "k", "v", "dy", "ds"])
+def test_fused_chunk_grad_keeps_an_infinity_in_its_part(gpu_lib, monkeypatch, where):
+    """No NaN where the query-side and key-side kernels have a number or an infinity
+    (a product formed as t3 - t1 - t2 would take an infinite part into the other)."""
+    B, H, d, T = 1, 2, 64, 150
+    case = list(_case(1, B, H, T, d, 7900, False, False, torch.float32))
+    i = {"q": 0, "k": 1, "v": 2, "dy": 4, "ds": 5}[where]
+    case[i] = case[i].clone()
+    case[i][(0, 0, 1, 3, 4, 0) if where == "ds" else (0, 1, 70, 5, 0)] = math.inf
+    fused = _gpu_grads(*case, d, 64, torch.float32, False)
+    general = _query_and_key_grads(monkeypatch, case, d, False)
+    assert any(not b.isfinite().all() for b in general if b is not None)
+    for name, a, b in zip(NAMES, fused, general):
+        if a is not None:
+            assert not (a.isnan() & ~b.isnan()).any(), name
